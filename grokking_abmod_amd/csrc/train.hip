@@ -49,7 +49,6 @@ struct QkSet {
 constexpr float kRmsEps = 1e-5f;                                         // src/gpt/mod.rs:38
 constexpr float kXsaFloor = float(double(1e-12f) * double(1e-12f));      // XSA_EPSILON^2
 constexpr int kThreads = 256;
-constexpr int kRowThreads = 64;  // per-(row, head) kernels: one wave per workgroup spreads few rows widely
 
 __device__ __forceinline__ float elu(float z) { return z >= 0.0f ? z : expm1f(z); }
 
@@ -578,138 +577,6 @@ __global__ void __launch_bounds__(kThreads) rmsnorm_backward_kernel(const float 
     }
 }
 
-// ---- attention (one thread per (row, head); the head row in registers)
-
-template <int HD>
-__global__ void __launch_bounds__(kRowThreads) attention_forward_kernel(const float *__restrict__ q,
-                                                                     const float *__restrict__ k,
-                                                                     const float *__restrict__ v,
-                                                                     float *__restrict__ y,
-                                                                     float *__restrict__ lse, int rows,
-                                                                     int sequence, int W, int H, float scale) {
-    const int t = blockIdx.x * kRowThreads + threadIdx.x;
-    if (t >= rows * H) return;
-    const int r = t / H, h = t % H, hd = W / H, pos = r % sequence, first = r - pos;
-    float qr[HD], acc[HD];
-#pragma unroll
-    for (int d = 0; d < HD; ++d) {
-        qr[d] = d < hd ? q[size_t(r) * W + h * hd + d] : 0.0f;
-        acc[d] = 0.0f;
-    }
-    float m = -INFINITY, l = 0.0f;
-    for (int j = 0; j <= pos; ++j) {
-        const float *kr = k + size_t(first + j) * W + h * hd, *vr = v + size_t(first + j) * W + h * hd;
-        float s = 0.0f;
-#pragma unroll
-        for (int d = 0; d < HD; ++d)
-            if (d < hd) s = fmaf(qr[d], kr[d], s);
-        s *= scale;
-        const float mn = fmaxf(m, s), alpha = expf(m - mn), p = expf(s - mn);
-        l = l * alpha + p;
-#pragma unroll
-        for (int d = 0; d < HD; ++d)
-            if (d < hd) acc[d] = fmaf(p, vr[d], acc[d] * alpha);
-        m = mn;
-    }
-    const float il = 1.0f / l;
-#pragma unroll
-    for (int d = 0; d < HD; ++d)
-        if (d < hd) y[size_t(r) * W + h * hd + d] = acc[d] * il;
-    lse[t] = m + logf(l);
-}
-
-// dq_i = scale sum_j P_ij (dy_i . v_j - D_i) k_j with D_i = dy_i . y_i.
-template <int HD>
-__global__ void __launch_bounds__(kRowThreads) attention_dq_kernel(const float *__restrict__ q,
-                                                                const float *__restrict__ k,
-                                                                const float *__restrict__ v,
-                                                                const float *__restrict__ y,
-                                                                const float *__restrict__ lse,
-                                                                const float *__restrict__ dy, float *__restrict__ dq,
-                                                                float *__restrict__ dsum, int rows, int sequence,
-                                                                int W, int H, float scale) {
-    const int t = blockIdx.x * kRowThreads + threadIdx.x;
-    if (t >= rows * H) return;
-    const int r = t / H, h = t % H, hd = W / H, pos = r % sequence, first = r - pos;
-    const size_t o = size_t(r) * W + h * hd;
-    float qr[HD], g[HD], acc[HD];
-    float D = 0.0f;
-#pragma unroll
-    for (int d = 0; d < HD; ++d) {
-        qr[d] = d < hd ? q[o + d] : 0.0f;
-        g[d] = d < hd ? dy[o + d] : 0.0f;
-        if (d < hd) D = fmaf(g[d], y[o + d], D);
-        acc[d] = 0.0f;
-    }
-    const float L = lse[t];
-    for (int j = 0; j <= pos; ++j) {
-        const float *kr = k + size_t(first + j) * W + h * hd, *vr = v + size_t(first + j) * W + h * hd;
-        float s = 0.0f, gv = 0.0f;
-#pragma unroll
-        for (int d = 0; d < HD; ++d)
-            if (d < hd) {
-                s = fmaf(qr[d], kr[d], s);
-                gv = fmaf(g[d], vr[d], gv);
-            }
-        const float ds = expf(s * scale - L) * (gv - D);
-#pragma unroll
-        for (int d = 0; d < HD; ++d)
-            if (d < hd) acc[d] = fmaf(ds, kr[d], acc[d]);
-    }
-#pragma unroll
-    for (int d = 0; d < HD; ++d)
-        if (d < hd) dq[o + d] = acc[d] * scale;
-    dsum[t] = D;
-}
-
-// For key row j: dv_j += sum_i P_ij dy_i, dk_j = scale sum_i P_ij (dy_i . v_j - D_i) q_i over the
-// queries i >= j of its sequence.
-template <int HD>
-__global__ void __launch_bounds__(kRowThreads) attention_dkv_kernel(const float *__restrict__ q,
-                                                                 const float *__restrict__ k,
-                                                                 const float *__restrict__ v,
-                                                                 const float *__restrict__ lse,
-                                                                 const float *__restrict__ dy,
-                                                                 const float *__restrict__ dsum,
-                                                                 float *__restrict__ dk, float *dv, int rows,
-                                                                 int sequence, int W, int H, float scale) {
-    const int t = blockIdx.x * kRowThreads + threadIdx.x;
-    if (t >= rows * H) return;
-    const int j = t / H, h = t % H, hd = W / H, pos = j % sequence, last = j - pos + sequence;
-    const size_t o = size_t(j) * W + h * hd;
-    float kr[HD], vr[HD], ak[HD], av[HD];
-#pragma unroll
-    for (int d = 0; d < HD; ++d) {
-        kr[d] = d < hd ? k[o + d] : 0.0f;
-        vr[d] = d < hd ? v[o + d] : 0.0f;
-        ak[d] = av[d] = 0.0f;
-    }
-    for (int i = j; i < last; ++i) {
-        const float *qi = q + size_t(i) * W + h * hd, *gi = dy + size_t(i) * W + h * hd;
-        float s = 0.0f, gv = 0.0f;
-#pragma unroll
-        for (int d = 0; d < HD; ++d)
-            if (d < hd) {
-                s = fmaf(qi[d], kr[d], s);
-                gv = fmaf(gi[d], vr[d], gv);
-            }
-        const float p = expf(s * scale - lse[size_t(i) * H + h]);
-        const float ds = p * (gv - dsum[size_t(i) * H + h]);
-#pragma unroll
-        for (int d = 0; d < HD; ++d)
-            if (d < hd) {
-                av[d] = fmaf(p, gi[d], av[d]);
-                ak[d] = fmaf(ds, qi[d], ak[d]);
-            }
-    }
-#pragma unroll
-    for (int d = 0; d < HD; ++d)
-        if (d < hd) {
-            dk[o + d] = ak[d] * scale;
-            dv[o + d] += av[d];
-        }
-}
-
 // ---- one wave per (row, head), lanes over the head's dims (dim lane + 64 e)
 
 template <int EPL>
@@ -1068,35 +935,31 @@ __global__ void __launch_bounds__(kThreads) attention_backward_wave(const float 
     lanes_store(dv + o, hd, lane, own);
 }
 
-template <int EPL>
-__global__ void __launch_bounds__(kThreads) xsa_forward_wave(const float *__restrict__ y, const float *__restrict__ v,
-                                                             float *__restrict__ z, int rows, int W, int H) {
+// What the matrix-core backward needs of one (row, head): dy (XSA's backward
+// of dz), the XSA's part of dv (zero without XSA) and D = dy . y.
+template <int EPL, bool XSA>
+__global__ void __launch_bounds__(kThreads) attention_output_grad_wave(const float *__restrict__ y,
+                                                                       const float *__restrict__ v,
+                                                                       const float *__restrict__ dz,
+                                                                       float *__restrict__ dy, float *__restrict__ dv,
+                                                                       float *__restrict__ dsum, int rows, int W,
+                                                                       int H) {
     const int t = row_wave(), lane = threadIdx.x & 63;
     if (t >= rows * H) return;
     const int hd = W / H;
     const size_t o = size_t(t / H) * W + (t % H) * hd;
-    float yv[EPL], vs[EPL];
+    float yv[EPL], g[EPL], d[EPL] = {};
     lanes_load(y + o, hd, lane, yv);
-    lanes_load(v + o, hd, lane, vs);
-    lanes_xsa(yv, vs);
-    lanes_store(z + o, hd, lane, yv);
-}
-
-template <int EPL>
-__global__ void __launch_bounds__(kThreads) xsa_backward_wave(const float *__restrict__ y, const float *__restrict__ v,
-                                                              const float *__restrict__ dz, float *__restrict__ dy,
-                                                              float *__restrict__ dv, int rows, int W, int H) {
-    const int t = row_wave(), lane = threadIdx.x & 63;
-    if (t >= rows * H) return;
-    const int hd = W / H;
-    const size_t o = size_t(t / H) * W + (t % H) * hd;
-    float yv[EPL], vs[EPL], g[EPL], d[EPL];
-    lanes_load(y + o, hd, lane, yv);
-    lanes_load(v + o, hd, lane, vs);
     lanes_load(dz + o, hd, lane, g);
-    lanes_xsa_backward(yv, vs, g, d);
-    lanes_store(dy + o, hd, lane, g);
+    if (XSA) {
+        float vs[EPL];
+        lanes_load(v + o, hd, lane, vs);
+        lanes_xsa_backward(yv, vs, g, d);
+        lanes_store(dy + o, hd, lane, g);
+    }
     lanes_store(dv + o, hd, lane, d);
+    const float D = lanes_dot(g, yv);
+    if (lane == 0) dsum[t] = D;
 }
 
 template <class F>
@@ -1113,10 +976,18 @@ void by_lanes(int hd, F &&f) {
         f(std::integral_constant<int, 16>{});
 }
 
-// Sequences up to this length take the wave-per-row attention kernels; longer
-// ones the thread-per-row kernels, whose key loops do 64 rows' work per wave
-// (head widths up to 128; wider heads always take the wave kernels).
-constexpr int kWaveAttentionMax = 64;
+// Whether a shape takes the matrix-core attention kernels, which work on 16 x 16
+// blocks of (query, key) and 64 rows a workgroup, or the wave-per-row kernels,
+// whose time grows with the keys a row attends over.  One gradient of 2048
+// rows, two blocks, wave against matrix kernels: head width 32 at 12 rows a
+// sequence 300 and 300 us, at 16 326 and 288, at 64 531 and 272; head width 64
+// at 12 728 and 828, at 16 786 and 782, at 32 878 and 734; head width 128 at
+// 16 1250 and 1337, at 32 1346 and 1242.  The line lies above the reference's
+// default context of 32 and not at 16: a thousand AdamW steps there carry every
+// rounding difference on, and that run keeps its published trajectory bit for
+// bit on the wave kernels.  Wider heads always take the wave kernels.
+bool matrix_attention(int sequence, int hd) { return hd <= 128 && sequence > 32; }
+
 // Sequences up to this length run the attention backward as one launch, whose
 // key waves redo the later queries' XSA backward (a few rows each).
 constexpr int kMergedBackwardMax = 8;
@@ -1304,20 +1175,6 @@ __global__ void __launch_bounds__(kThreads) adam_kernel(float *__restrict__ para
     const float mh = mi / sc->correction1, vh = vi / sc->correction2;
     const float step = __fadd_rn(mh / __fadd_rn(sqrtf(vh), o.epsilon), __fmul_rn(o.weight_decay, params[i]));
     params[i] = __fsub_rn(params[i], __fmul_rn(o.learning_rate, step));
-}
-
-template <class F>
-void by_head_width(int hd, F &&f) {
-    if (hd <= 8)
-        f(std::integral_constant<int, 8>{});
-    else if (hd <= 16)
-        f(std::integral_constant<int, 16>{});
-    else if (hd <= 32)
-        f(std::integral_constant<int, 32>{});
-    else if (hd <= 64)
-        f(std::integral_constant<int, 64>{});
-    else
-        f(std::integral_constant<int, 128>{});
 }
 
 // ---- the forward of short sequences: a workgroup holds R sequences, one wave
@@ -1965,31 +1822,20 @@ void rmsnorm_backward_sum3(const float *x, const float *inv, const float *dy0, c
 void attention_forward(const float *q, const float *k, const float *v, float *y, float *z, float *lse, int rows,
                        int sequence, int W, int H, bool xsa, hipStream_t stream) {
     const float scale = float(1.0 / std::sqrt(double(W / H)));
-    if (sequence <= kWaveAttentionMax || W / H > 128) {
-        by_lanes(W / H, [&](auto e) {
-            constexpr int EPL = decltype(e)::value;
-            const dim3 grid(blocks_for(size_t(rows) * H * 64));
-            if (xsa)
-                hipLaunchKernelGGL((attention_forward_wave<EPL, true>), grid, dim3(kThreads), 0, stream, q, k, v, y,
-                                   z, lse, rows, sequence, W, H, scale);
-            else
-                hipLaunchKernelGGL((attention_forward_wave<EPL, false>), grid, dim3(kThreads), 0, stream, q, k, v, y,
-                                   z, lse, rows, sequence, W, H, scale);
-        });
+    if (matrix_attention(sequence, W / H)) {
+        matrix_attention_forward(q, k, v, y, z, lse, rows, sequence, W, H, xsa, stream);
         return;
     }
-    by_head_width(W / H, [&](auto hd) {
-        hipLaunchKernelGGL(attention_forward_kernel<decltype(hd)::value>, dim3(blocks_for(size_t(rows) * H, kRowThreads)),
-                           dim3(kRowThreads), 0, stream, q, k, v, y, lse, rows, sequence, W, H, scale);
+    by_lanes(W / H, [&](auto e) {
+        constexpr int EPL = decltype(e)::value;
+        const dim3 grid(blocks_for(size_t(rows) * H * 64));
+        if (xsa)
+            hipLaunchKernelGGL((attention_forward_wave<EPL, true>), grid, dim3(kThreads), 0, stream, q, k, v, y, z,
+                               lse, rows, sequence, W, H, scale);
+        else
+            hipLaunchKernelGGL((attention_forward_wave<EPL, false>), grid, dim3(kThreads), 0, stream, q, k, v, y, z,
+                               lse, rows, sequence, W, H, scale);
     });
-    if (xsa) {
-        by_lanes(W / H, [&](auto e) {
-            hipLaunchKernelGGL(xsa_forward_wave<decltype(e)::value>, dim3(blocks_for(size_t(rows) * H * 64)),
-                               dim3(kThreads), 0, stream, y, v, z, rows, W, H);
-        });
-    } else {
-        copy(y, z, size_t(rows) * W, stream);
-    }
 }
 
 void attention_backward(const float *q, const float *k, const float *v, const float *y, const float *lse,
@@ -2011,35 +1857,31 @@ void attention_backward(const float *q, const float *k, const float *v, const fl
         });
         return;
     }
-    if (sequence <= kWaveAttentionMax || W / H > 128) {
+    if (matrix_attention(sequence, W / H)) {
         by_lanes(W / H, [&](auto e) {
             constexpr int EPL = decltype(e)::value;
             const dim3 grid(blocks_for(size_t(rows) * H * 64));
             if (xsa)
-                hipLaunchKernelGGL((attention_dq_wave<EPL, true>), grid, dim3(kThreads), 0, stream, q, k, v, y, lse,
-                                   dz, dy, dv, dq, dsum, rows, sequence, W, H, scale);
+                hipLaunchKernelGGL((attention_output_grad_wave<EPL, true>), grid, dim3(kThreads), 0, stream, y, v, dz,
+                                   dy, dv, dsum, rows, W, H);
             else
-                hipLaunchKernelGGL((attention_dq_wave<EPL, false>), grid, dim3(kThreads), 0, stream, q, k, v, y, lse,
-                                   dz, dy, dv, dq, dsum, rows, sequence, W, H, scale);
-            hipLaunchKernelGGL(attention_dkv_wave<EPL>, grid, dim3(kThreads), 0, stream, q, k, v, lse, g, dsum, dk, dv,
-                               rows, sequence, W, H, scale);
+                hipLaunchKernelGGL((attention_output_grad_wave<EPL, false>), grid, dim3(kThreads), 0, stream, y, v,
+                                   dz, dy, dv, dsum, rows, W, H);
         });
+        matrix_attention_backward(q, k, v, lse, g, dsum, dq, dk, dv, rows, sequence, W, H, stream);
         return;
     }
-    if (xsa) {
-        by_lanes(W / H, [&](auto e) {
-            hipLaunchKernelGGL(xsa_backward_wave<decltype(e)::value>, dim3(blocks_for(size_t(rows) * H * 64)),
-                               dim3(kThreads), 0, stream, y, v, dz, dy, dv, rows, W, H);
-        });
-    } else {
-        fill(dv, 0.0f, size_t(rows) * W, stream);
-    }
-    by_head_width(W / H, [&](auto hd) {
-        constexpr int HD = decltype(hd)::value;
-        hipLaunchKernelGGL(attention_dq_kernel<HD>, dim3(blocks_for(size_t(rows) * H, kRowThreads)), dim3(kRowThreads), 0, stream, q,
-                           k, v, y, lse, g, dq, dsum, rows, sequence, W, H, scale);
-        hipLaunchKernelGGL(attention_dkv_kernel<HD>, dim3(blocks_for(size_t(rows) * H, kRowThreads)), dim3(kRowThreads), 0, stream,
-                           q, k, v, lse, g, dsum, dk, dv, rows, sequence, W, H, scale);
+    by_lanes(W / H, [&](auto e) {
+        constexpr int EPL = decltype(e)::value;
+        const dim3 grid(blocks_for(size_t(rows) * H * 64));
+        if (xsa)
+            hipLaunchKernelGGL((attention_dq_wave<EPL, true>), grid, dim3(kThreads), 0, stream, q, k, v, y, lse, dz,
+                               dy, dv, dq, dsum, rows, sequence, W, H, scale);
+        else
+            hipLaunchKernelGGL((attention_dq_wave<EPL, false>), grid, dim3(kThreads), 0, stream, q, k, v, y, lse, dz,
+                               dy, dv, dq, dsum, rows, sequence, W, H, scale);
+        hipLaunchKernelGGL(attention_dkv_wave<EPL>, grid, dim3(kThreads), 0, stream, q, k, v, lse, g, dsum, dk, dv,
+                           rows, sequence, W, H, scale);
     });
 }
 

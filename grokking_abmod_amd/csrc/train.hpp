@@ -118,8 +118,9 @@ void qk_backward(int count, float *const *g, const float *const *pre, const floa
 
 // Causal softmax attention per (sequence, head) (reference.rs:510-554) into y,
 // then z = XSA(y) (reference.rs:577-603: y - (y.u) u, u = v / max(|v|, 1e-12)
-// per head) when xsa, else z = y; lse[r * H + h] = max + ln(sum) of the row's
-// scaled scores.
+// per head) when xsa, else z = y; lse[r * H + h] is the row's log-sum-exp as
+// attention_backward of the same shape reads it (base e from the wave kernels,
+// base 2 from the matrix-core ones).
 void attention_forward(const float *q, const float *k, const float *v, float *y, float *z, float *lse, int rows,
                        int sequence, int W, int H, bool xsa, hipStream_t stream);
 // Its backward from dz = d loss / d z: dq and dk written, dv written (XSA's
@@ -128,6 +129,14 @@ void attention_forward(const float *q, const float *k, const float *v, float *y,
 void attention_backward(const float *q, const float *k, const float *v, const float *y, const float *lse,
                         const float *dz, float *dy, float *dq, float *dk, float *dv, float *dsum, int rows,
                         int sequence, int W, int H, bool xsa, hipStream_t stream);
+// The matrix-core kernels of the two (train_attn.hip), for head widths up to
+// 128: the backward from dy = d loss / d y and dsum = dy . y, with dv holding
+// XSA's part.
+void matrix_attention_forward(const float *q, const float *k, const float *v, float *y, float *z, float *lse, int rows,
+                              int sequence, int W, int H, bool xsa, hipStream_t stream);
+void matrix_attention_backward(const float *q, const float *k, const float *v, const float *lse, const float *dy,
+                               const float *dsum, float *dq, float *dk, float *dv, int rows, int sequence, int W,
+                               int H, hipStream_t stream);
 
 // The embedding geometry (reference.rs:130-149) on V raw token rows: scaled to
 // `radius` when normalize (rinv[t] keeps 1 / max(|row|, 1e-12)), then the first

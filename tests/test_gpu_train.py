@@ -111,6 +111,64 @@ def test_loss_and_gradients_match_the_oracle(cfg, cases):
                 assert abs(model.cross_entropy(x, targets, s) - loss) <= 1e-6 * (1 + abs(loss))
 
 
+# Sequences past the wave attention kernels' 32 rows, on the matrix-core
+# attention: the first length there, one row into a second workgroup of 64,
+# ragged and whole tiles, every padded head width (8 and 12 dims padded to 16,
+# 24 to 32, 40 to 64, 72 to 128) and head widths that are no multiple of four;
+# the wave kernels at their last length.
+LONG = [(dict(width=32, heads=4), 65), (dict(width=24, heads=2), 100), (dict(width=48, heads=2), 127),
+        (dict(width=128, heads=2), 64), (dict(width=128, heads=2), 129), (dict(width=32, heads=1), 192),
+        (dict(width=40, heads=1, xsa=0), 97), (dict(width=72, heads=1), 70), (dict(width=128, heads=1), 130),
+        (dict(width=30, heads=3, rope=0, qk_norm=0), 66), (dict(width=12, heads=2), 161),
+        (dict(width=128, heads=2), 32), (dict(width=32, heads=4), 33), (dict(width=256, heads=2), 33)]
+
+
+@pytest.mark.parametrize("cfg,s", LONG, ids=[f"W{c['width']}-H{c['heads']}-S{s}" for c, s in LONG])
+def test_long_sequence_gradients_match_the_oracle(cfg, s):
+    """The gradient's error against the f64 tape in the 2-norm: about forty f32
+    roundings of 2^-24 chain from a weight to the loss, 2.4e-6 if all add up;
+    four times that is allowed."""
+    g, o = configs_for(vocab_size=11, context=s, layers=1, attention_mesh_depth=2, ffn_mesh_depth=2, **cfg)
+    params = np.random.default_rng(s).uniform(-1.0, 1.0, O.parameter_count(o)).astype(np.float32)
+    rng = np.random.default_rng(5)
+    x = rng.integers(0, 11, 2 * s).astype(np.uint32)
+    y = rng.integers(0, 11, 2 * s).astype(np.uint32)
+    ref_loss, ref_grad = O.loss_and_gradient(o, params, x, y, s)
+    with G.MeshGpt(0, g, 7) as model:
+        model.set_parameters(params)
+        loss, grad = model.loss_and_gradient(x, y, s)
+        again = model.loss_and_gradient(x, y, s)
+    assert abs(loss - ref_loss) <= 1e-5 * abs(ref_loss)
+    assert np.linalg.norm(grad - ref_grad) <= 1e-5 * np.linalg.norm(ref_grad)
+    assert again[0] == loss and np.array_equal(again[1], grad)
+
+
+def test_a_later_row_that_overflows_leaves_earlier_losses():
+    """A row whose value overflows to infinity (block 0's V mesh as in
+    test_nonfinite_step_changes_nothing) is behind the causal mask of earlier
+    rows: their losses are those without it, in the tile they share too."""
+    s = 96
+    cfg = dict(vocab_size=7, context=s, width=8, heads=2, layers=1, attention_mesh_depth=3, ffn_mesh_depth=2)
+    g, _ = configs_for(**cfg)
+    with G.MeshGpt(0, g, 7) as model:
+        params = model.parameters()
+        for layer in (0, 1):
+            params[2 * 8 * 3 * 3 + layer * 2 * 8] = 3e38
+            params[2 * 8 * 3 * 3 + layer * 2 * 8 + 1] = 0.0
+        model.set_parameters(params)
+        E = model.token_embeddings()
+        up = [t for t in range(7) if E[t, 0] > 1e-3]
+        down = np.array([t for t in range(7) if E[t, 0] < -1e-3])
+        x = down[np.arange(s) % len(down)].astype(np.uint32)
+        y = np.where(np.arange(s) < 70, np.arange(s) % 7, IGN).astype(np.uint32)
+        clean = model.cross_entropy(x, y, s)
+        x[80] = up[0]
+        assert model.cross_entropy(x, y, s) == pytest.approx(clean, rel=1e-6)
+        y[80] = 1
+        with pytest.raises(G.MeshGptError):
+            model.cross_entropy(x, y, s)
+
+
 # Stacks deeper than the 16 layers of one kernel launch, in the wave (width
 # <= 128) and the LDS (wider) mesh kernels, both connectivities, the mesh
 # embedding included.
