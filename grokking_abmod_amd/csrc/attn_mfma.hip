@@ -2,11 +2,12 @@
 // the XSA epilogue (reference.rs:510-554 attention, 577-603 exclusive self
 // attention; the reference's GPU kernel is gpt_flash_forward, gpu.rs:381-498).
 //
-// One workgroup of eight waves (four at head width 32) takes 256 (128)
-// queries of one (sequence, head); each wave owns 32 of them (two 16-query
-// blocks).  Eight waves share each K/V tile among twice the queries and put
-// four waves on every SIMD (two workgroups per CU, by LDS): config 4's
-// prefill took 23.69 ms against 23.95 with four waves (and 24.8 with 32-key
+// One workgroup takes 64 to 256 queries of one (sequence, head)
+// (attn_prefill_mfma chooses); each wave owns 16 or 32 of them (one or two
+// 16-query blocks).  Sequences of 288 rows or more run here only where
+// attn_split.hip cannot take them.  At 8192 rows eight waves share each K/V tile
+// among 256 queries and put four waves on every SIMD (two workgroups per CU, by
+// LDS): 23.69 ms a prefill against 23.95 with four waves (and 24.8 with 32-key
 // tiles, which let four workgroups share a CU).  Keys stream through LDS in
 // tiles of 64 rows of K and V, double-buffered and loaded with direct-to-LDS
 // loads (global_load_lds_dwordx4), so a tile lands while the previous one is
@@ -26,6 +27,7 @@
 // whole rows.  Scores are in the log2 domain (q pre-scaled by log2(e)/sqrt(hd)).
 #include <hip/hip_runtime.h>
 
+#include "attn_range.hpp"
 #include "kernels.hpp"
 
 namespace meshgpt::kern {
@@ -74,12 +76,12 @@ __device__ __forceinline__ float xor_lanes(float v, int mask) {
     return __shfl_xor(v, mask, 64);
 }
 
-template <int HD>
+template <int HD, int WV, int QB>
 struct MfmaCfg {
     static constexpr int BK = 64;                 // keys per tile
     static constexpr int KB = BK / 16;            // 16-key blocks per tile
-    static constexpr int NQB = 2;                 // 16-query blocks per wave
-    static constexpr int WAVES = HD == 64 ? 8 : 4;
+    static constexpr int NQB = QB;                // 16-query blocks per wave
+    static constexpr int WAVES = WV;
     static constexpr int QT = 16 * NQB * WAVES;   // queries per workgroup
     static constexpr int KS = HD / 4;             // k-steps of Q.K: dim = KS * (lane / 16) + step
     static constexpr int DB = HD / 16;            // 16-dim blocks of the output
@@ -100,15 +102,15 @@ __device__ __forceinline__ int swz(int row, int dim) {
 // of one cache slab into a swizzled LDS tile: wave w's instruction u fills
 // floats [256 i, 256 i + 256) of the tile, i = w * DMA_W + u, lane l the 16
 // bytes at 256 i + 4 l, which belong to row (256 i + 4 l) / HD.
-template <int HD>
+template <int HD, int DMA_W>
 __device__ __forceinline__ void issue_tile(const float *slab, int t0, int n, float *tile, int wave, int lane) {
-    using C = MfmaCfg<HD>;
+    constexpr int C4 = HD / 4;
 #pragma unroll
-    for (int u = 0; u < C::DMA_W; ++u) {
-        const int i = wave * C::DMA_W + u;
+    for (int u = 0; u < DMA_W; ++u) {
+        const int i = wave * DMA_W + u;
         const int f = 256 * i + 4 * lane;
         const int row = f / HD, slot = (f % HD) / 4;
-        const int c4 = slot ^ (row & (C::C4 - 1));
+        const int c4 = slot ^ (row & (C4 - 1));
         const int key = min(t0 + row, n - 1);
         dma16(slab + size_t(key) * HD + 4 * c4, tile + 256 * i);
     }
@@ -118,11 +120,11 @@ __device__ __forceinline__ void issue_tile(const float *slab, int t0, int n, flo
 // head) pairs and query tiles keeps every query tile of a pair on one XCD,
 // consecutive on it and longest first, so the tiles that stream the same keys
 // share that XCD's L2.
-template <int HD>
-__global__ void __launch_bounds__(64 * MfmaCfg<HD>::WAVES)
+template <int HD, int WV, int QB>
+__global__ void __launch_bounds__(64 * WV)
 attn_prefill_mfma_kernel(Shape s, const float *__restrict__ q, KvView kv, int nseq, int n, float *__restrict__ y,
-                         float scale_log2, int xsa) {
-    using C = MfmaCfg<HD>;
+                         float scale_log2, int xsa, const int2 *__restrict__ range) {
+    using C = MfmaCfg<HD, WV, QB>;
     constexpr int BK = C::BK, KB = C::KB, NQB = C::NQB, KS = C::KS, DB = C::DB, C4 = C::C4, TILE = C::TILE;
     __shared__ __align__(16) float lds[4 * TILE];  // [stage][K, V]
     const int ntiles = (n + C::QT - 1) / C::QT;
@@ -133,6 +135,11 @@ attn_prefill_mfma_kernel(Shape s, const float *__restrict__ q, KvView kv, int ns
     const int seq = pair / s.H, h = pair - seq * s.H;
     const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
     const int jq = lane & 15, g = lane >> 4;
+    if (range) {  // attn_split has run the pairs it can
+        const int tiles = (n + kSplitKeys - 1) / kSplitKeys;
+        int E;
+        if (pair_splits(range + size_t(pair) * tiles, tiles, lane, E)) return;
+    }
     const int qwave = qt * C::QT + wave * 16 * NQB;  // first query of this wave
     const int qlast_wg = min(qt * C::QT + C::QT, n) - 1;
     const size_t slab = size_t(pair) * kv.cap * HD;
@@ -165,13 +172,13 @@ attn_prefill_mfma_kernel(Shape s, const float *__restrict__ q, KvView kv, int ns
     }
 
     const int ntile = qlast_wg / BK + 1;
-    issue_tile<HD>(kslab, 0, n, lds, wave, lane);
-    issue_tile<HD>(vslab, 0, n, lds + TILE, wave, lane);
+    issue_tile<HD, C::DMA_W>(kslab, 0, n, lds, wave, lane);
+    issue_tile<HD, C::DMA_W>(vslab, 0, n, lds + TILE, wave, lane);
     for (int t = 0; t < ntile; ++t) {
         if (t + 1 < ntile) {
             float *next = lds + ((t + 1) & 1) * 2 * TILE;
-            issue_tile<HD>(kslab, (t + 1) * BK, n, next, wave, lane);
-            issue_tile<HD>(vslab, (t + 1) * BK, n, next + TILE, wave, lane);
+            issue_tile<HD, C::DMA_W>(kslab, (t + 1) * BK, n, next, wave, lane);
+            issue_tile<HD, C::DMA_W>(vslab, (t + 1) * BK, n, next + TILE, wave, lane);
             wait_vm<2 * C::DMA_W>();
         } else {
             wait_vm<0>();
@@ -398,18 +405,32 @@ bool attn_prefill_mfma_supported(const Shape &s, int rows_per_seq) {
 }
 
 void attn_prefill_mfma(const Shape &s, const float *q, KvView kv, int nseq, int rows_per_seq, float *y, int xsa,
-                       hipStream_t stream) {
+                       const int2 *range, hipStream_t stream) {
     const float scale_log2 = float(1.4426950408889634 / std::sqrt(double(s.hd)));
     auto launch = [&](auto kernel, int qt, int waves) {
         const int ntiles = (rows_per_seq + qt - 1) / qt;
         const int px = (nseq * s.H + 7) / 8;
         hipLaunchKernelGGL(kernel, dim3(8 * px * ntiles), dim3(64 * waves), 0, stream, s, q, kv, nseq,
-                           rows_per_seq, y, scale_log2, xsa);
+                           rows_per_seq, y, scale_log2, xsa, range);
     };
-    if (s.hd == 32)
-        launch(attn_prefill_mfma_kernel<32>, MfmaCfg<32>::QT, MfmaCfg<32>::WAVES);
+    // Queries of a workgroup (32 or 16 a wave).  Long sequences share each key
+    // tile among as many as fit: 8192 rows at head width 64, 23.7 ms a prefill
+    // with 256 queries and 24.0 with 128.  Shorter ones need workgroups to fill
+    // the GPU and lose on the diagonal and on waves without a query: 256
+    // sequences of 128 rows (4096 pairs, W1024, 12 blocks) take 11.37 ms with
+    // 256 queries, 9.10 with 128 in four waves, 9.33 with 64; 32 pairs of 512 rows
+    // (W512, 6 blocks) 0.79, 0.65 and 0.55; 72 of 1001 2.50, 1.80 and 1.73.
+    const bool longer = rows_per_seq >= 2048;
+    if (s.hd == 32 && longer)
+        launch(attn_prefill_mfma_kernel<32, 4, 2>, 128, 4);
+    else if (s.hd == 32)
+        launch(attn_prefill_mfma_kernel<32, 8, 1>, 128, 8);
+    else if (longer)
+        launch(attn_prefill_mfma_kernel<64, 8, 2>, 256, 8);
+    else if (nseq * s.H >= 1024)
+        launch(attn_prefill_mfma_kernel<64, 4, 2>, 128, 4);
     else
-        launch(attn_prefill_mfma_kernel<64>, MfmaCfg<64>::QT, MfmaCfg<64>::WAVES);
+        launch(attn_prefill_mfma_kernel<64, 4, 1>, 64, 4);
     (void)hipGetLastError();
 }
 

@@ -221,8 +221,18 @@ bool attn_prefill_mfma_supported(const Shape &s, int rows_per_seq);
 bool attn_prefill_short_supported(const Shape &s, int rows_per_seq);
 void attn_prefill_short(const Shape &s, const float *q, KvView kv, int nseq, int rows_per_seq, float *y, int xsa,
                         hipStream_t stream);
+// With `range` (from attn_split on the same rows) only the (sequence, head)
+// pairs that attn_split left.
 void attn_prefill_mfma(const Shape &s, const float *q, KvView kv, int nseq, int rows_per_seq, float *y, int xsa,
-                       hipStream_t stream);
+                       const int2 *range, hipStream_t stream);
+// The same for long sequences on FP16 matrix cores with every operand split
+// into two halves, at FP32 accuracy (attn_split.hip), in attn_split_bytes() of
+// scratch.  Pairs whose values span too wide a range for it are left to
+// attn_prefill_mfma, which takes the returned ranges.
+bool attn_split_supported(const Shape &s, int rows_per_seq);
+size_t attn_split_bytes(const Shape &s, int nseq, int rows_per_seq);
+const int2 *attn_split(const Shape &s, const float *q, KvView kv, int nseq, int rows_per_seq, float *y, int xsa,
+                       void *scratch, hipStream_t stream);
 // logits[i][t] = xn[i*row_mul+row_add] . E[t] (xn already RMS-normalised).
 void head(const Shape &s, const float *xn, int nrows, int row_mul, int row_add, const float *Et, int Vp,
           float *logits, int rt, hipStream_t stream);

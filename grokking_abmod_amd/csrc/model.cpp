@@ -126,6 +126,7 @@ struct MeshGpt::Impl {
 
     // Prefill / logits workspace, grown on demand.
     DevBuf wx, wxn, wq, wy, wtok, wlogits, wk, wv;
+    DevBuf wsplit;  // keys and values of one layer as attn_split's planes
 
     // Decode graphs replaying 1 and kGraphSteps steps.
     static constexpr size_t kGraphSteps = 8;
@@ -145,6 +146,7 @@ struct MeshGpt::Impl {
     bool persistent_ok = false;
     bool use_mfma_prefill = true;
     bool use_rows_prefill = true;
+    bool use_split_prefill = true;
     bool use_short_prefill = true;
 
     // Training (gpu.rs:1915-2003): the activations of the last forward, the
@@ -307,6 +309,7 @@ struct MeshGpt::Impl {
         row_decode = all_operators && env_int("MG_DISABLE_ROW_DECODE", 0) == 0 && kern::row_block_supported(shape);
         persistent_ok = row_decode && env_int("MG_DISABLE_PERSISTENT", 0) == 0;
         use_mfma_prefill = env_int("MG_DISABLE_MFMA_PREFILL", 0) == 0;
+        use_split_prefill = env_int("MG_DISABLE_SPLIT_PREFILL", 0) == 0;
         use_rows_prefill = env_int("MG_DISABLE_ROWS_PREFILL", 0) == 0;
         use_short_prefill = env_int("MG_DISABLE_SHORT_PREFILL", 0) == 0;
 
@@ -473,6 +476,11 @@ struct MeshGpt::Impl {
         // shape allows it (MG_DISABLE_MFMA_PREFILL=1 keeps the VALU kernel).
         const bool mfma_prefill = !decode && use_mfma_prefill &&
                                   kern::attn_prefill_mfma_supported(shape, rows.rows_per_seq);
+        // Long sequences: split FP16 operands for the (sequence, head) pairs
+        // whose values allow it (MG_DISABLE_SPLIT_PREFILL=1 keeps FP32).
+        const bool split_prefill =
+            mfma_prefill && use_split_prefill && kern::attn_split_supported(shape, rows.rows_per_seq);
+        if (split_prefill) wsplit.ensure(kern::attn_split_bytes(shape, nseq, rows.rows_per_seq));
         // Short sequences: one thread per (row, head) (MG_DISABLE_SHORT_PREFILL=1
         // keeps the VALU flash kernel).
         const bool short_prefill = !decode && use_short_prefill &&
@@ -534,7 +542,10 @@ struct MeshGpt::Impl {
                 kern::attn_decode(shape, q, kv_of(l), rows.len, rows.rows, nsplit, part_base, stream,
                                   events ? events[2 * l] : nullptr, events ? events[2 * l + 1] : nullptr);
             } else if (mfma_prefill) {
-                kern::attn_prefill_mfma(shape, q, kv_of(l), nseq, rows.rows_per_seq, y, cfg.xsa, stream);
+                const int2 *range = nullptr;
+                if (split_prefill)
+                    range = kern::attn_split(shape, q, kv_of(l), nseq, rows.rows_per_seq, y, cfg.xsa, wsplit.p, stream);
+                kern::attn_prefill_mfma(shape, q, kv_of(l), nseq, rows.rows_per_seq, y, cfg.xsa, range, stream);
             } else if (short_prefill) {
                 kern::attn_prefill_short(shape, q, kv_of(l), nseq, rows.rows_per_seq, y, cfg.xsa, stream);
             } else {
@@ -917,7 +928,7 @@ struct MeshGpt::Impl {
         size_t total = 0;
         for (const DevBuf *b : {&params, &codes, &E, &Et, &rope, &wdec, &Edec, &q0, &kc, &vc, &dx, &dx2, &dxn, &dq,
                                 &part, &dtokens, &dlen, &drng, &dlogits, &dflags, &drng_start, &drng_next, &pxch, &pabort, &wx,
-                                &wxn, &wq, &wy, &wtok, &wlogits, &wk, &wv, &tact, &tgrad, &tm, &tv, &tpart, &tin})
+                                &wxn, &wq, &wy, &wtok, &wlogits, &wk, &wv, &wsplit, &tact, &tgrad, &tm, &tv, &tpart, &tin})
             total += b->bytes;
         return total;
     }

@@ -566,3 +566,81 @@ def test_register_tile_prefill_matches_oracle_and_block_kernel(cfg, monkeypatch)
         assert_close(got["0"][0], ref, what=f"register-tile prefill logits n={n}")
         assert_close(got["0"][1], O.hidden_states(o, params, x, n), what=f"register-tile hidden n={n}")
         assert_close(got["0"][0], got["1"][0], what=f"register-tile vs block_kernel n={n}")
+
+
+def _prefill_error(got, ref):
+    return np.linalg.norm(got - ref) / np.linalg.norm(ref)
+
+
+# The matrix-core prefill around its dispatch lines: FP32 workgroups of 64 (head
+# width 64), 128 (head width 32) and, from 2048 rows, 256 queries; split FP16
+# from 288 rows, its 128- and 256-query workgroups; whole and ragged key tiles.
+@pytest.mark.parametrize("heads", [2, 4])
+@pytest.mark.parametrize("n", [64, 129, 287, 288, 320, 449, 2047, 2048, 2113])
+def test_long_prefill_matches_the_oracle(n, heads):
+    """Every row's logits against the f64 oracle in the 2-norm, split and FP32:
+    about forty f32 roundings of 2^-24 chain from a weight to a logit, 2.4e-6 if
+    all add up; four times that is allowed, and the split operands' error may
+    not pass 1.2 times the FP32 kernel's."""
+    kw = dict(vocab_size=64, context=n, width=128, heads=heads, layers=1, attention_mesh_depth=3, ffn_mesh_depth=3,
+              connectivity=1)
+    g, o = G.GptConfig(**kw), O.config(**kw)
+    params = G.normal_parameters(g, 5)
+    tokens = G.random_prompts(64, 2, n, 11).reshape(-1)
+    ref = np.concatenate([O.logits(o, params, t, n) for t in tokens.reshape(2, n)])
+    error = {}
+    for off in ("0", "1"):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setenv("MG_DISABLE_SPLIT_PREFILL", off)
+            with G.MeshGpt(0, g, 7) as model:
+                model.set_parameters(params)
+                error[off] = _prefill_error(model.logits(tokens, n), ref)
+    assert max(error.values()) <= 1e-5, error
+    assert error["0"] <= 1.2 * error["1"], error
+
+
+@pytest.mark.parametrize("wide", ["every head", "one head", "zero rows"])
+def test_split_prefill_leaves_wide_values_to_fp32(wide):
+    """Value rows of very different sizes: token 0's channels are all negative
+    (in one head or in every one) and saturate at -1 in a V mesh that grows
+    positive ones 2500 times.  Those pairs run on the FP32 kernel: with every
+    head affected the logits are its own bit for bit.  A V mesh of zeros keeps
+    the split kernels: rows without a size count for nothing."""
+    n, W, H = 300, 128, 2
+    kw = dict(vocab_size=16, context=n, width=W, heads=H, layers=1, attention_mesh_depth=3, ffn_mesh_depth=2,
+              embedding=1)
+    g, o = G.GptConfig(**kw), O.config(**kw)
+    params = O.initialize(o, 7)
+    rng = np.random.default_rng(3)
+    table = params[:16 * W].reshape(16, W)
+    table[:] = rng.choice([-1.0, 1.0], (16, W)) * rng.uniform(0.8, 1.2, (16, W))
+    table[0, :W if wide == "every head" else W // H] = -1.0
+    v = params[O.group_offsets(o)[3]:][:2 * W * 3].reshape(3, W, 2)
+    v[:, :, 1] = 0.0
+    v[:, :, 0] = 0.0 if wide == "zero rows" else np.array([50.0, 50.0, 1.0])[:, None]
+    tokens = rng.integers(0, 16, n).astype(np.uint32)
+    ref = O.logits(o, params, tokens, n)
+    got = {}
+    for off in ("0", "1"):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setenv("MG_DISABLE_SPLIT_PREFILL", off)
+            with G.MeshGpt(0, g, 7) as model:
+                model.set_parameters(params)
+                got[off] = model.logits(tokens, n)
+    assert _prefill_error(got["0"], ref) <= 1e-5 and _prefill_error(got["1"], ref) <= 1e-5
+    if wide == "every head":
+        assert np.array_equal(got["0"], got["1"])
+
+
+def test_split_prefill_reports_values_that_overflow():
+    n = 300
+    kw = dict(vocab_size=64, context=n, width=128, heads=4, layers=1, attention_mesh_depth=9, ffn_mesh_depth=2,
+              connectivity=1)
+    g, o = G.GptConfig(**kw), O.config(**kw)
+    params = O.initialize(o, 7)
+    params[O.group_offsets(o)[3]:][:2 * 128 * 9] = 3e38
+    with G.MeshGpt(0, g, 7) as model:
+        model.set_parameters(params)
+        with pytest.raises(G.MeshGptError) as err:
+            model.logits(G.random_prompts(64, 1, n, 7)[0], n, last_only=True)
+        assert err.value.status == G.MG_NONFINITE
