@@ -241,6 +241,29 @@ void head(const Shape &s, const float *xn, int nrows, int row_mul, int row_add, 
 void head_sample(const Shape &s, const float *xn, int batch, const float *Et, int Vp, float *logits,
                  float temperature, uint64_t *rng, uint32_t *tokens, int tok_stride, int *len, int *flags,
                  hipStream_t stream);
+// `steps` generated tokens of each of `batch` sequences in one launch, every
+// token from its whole window of the last `context` tokens (window.hip): the
+// shapes of window_supported(), contexts of at most kWindowRows.
+constexpr int kWindowRows = 64;
+struct WindowArgs {
+    const float *E;       // token vectors (V x W)
+    const float *w;       // block 0's query weights; the blocks follow one another
+    const float2 *rope;
+    uint32_t *tokens;     // appended to
+    int tok_stride;
+    int *len;             // each sequence's length, advanced
+    uint64_t *rng;        // sampler states, advanced when temperature > 0
+    float temperature;
+    float *logits;        // [batch][V] of the last token
+    int *flags;           // bit 0: non-finite logits
+    float *kc, *vc;       // when set: the KV cache, which receives the last window's rows
+    size_t layer_elems;
+    int cap;
+    int L, A, F, V, context, steps, butterfly, rotate, qk_norm, xsa;
+    float scale_log2;     // set by window_generate
+};
+bool window_supported(const Shape &s, size_t context);
+void window_generate(const Shape &s, WindowArgs a, int batch, hipStream_t stream);
 // Greedy / temperature sampling from logits rows; appends the token and bumps len.
 void sample(int V, int batch, const float *logits, float temperature, uint64_t *rng, uint32_t *tokens,
             int tok_stride, int *len, int *flags, hipStream_t stream);
