@@ -78,6 +78,7 @@ struct BlockArgs {
     const float *E;
     int embed;
     float *q;
+    int q_last;  // 1: only each sequence's last query is wanted (rows_block)
     KvView kv_pre;
     const float2 *rope;
     float *xn;  // when set: the final RMSNorm of x for the head
@@ -117,6 +118,15 @@ void block(const BlockArgs &a, bool staged, hipStream_t stream);
 // attention rows in a.ybuf (not split partials).
 bool rows_block_supported(const Shape &s);
 void rows_block(const BlockArgs &a, hipStream_t stream);
+// The last block of a prefill whose only output is each sequence's last row:
+// last_rows() gathers the last queries and residual rows of sequences of n rows
+// (and fills len with n), attn_decode() attends for them, last_merge() joins
+// its split states into attention rows with XSA, and rows_block() takes those as
+// sequences of one row.  Head widths up to 64.
+void last_rows(const float *q, const float *x, int nseq, int n, int W, float *q_out, float *x_out, int *len,
+               hipStream_t stream);
+void last_merge(const Shape &s, const float *part, int nsplit, KvView kv, int nseq, int n, int xsa, float *y,
+                hipStream_t stream);
 // Decode variant of block(): one row per sequence (rows_per_seq == 1), each
 // mesh of a row on one wavefront.  Supported for W a power of two in
 // [64, 1024] and a power-of-two head width >= 8.

@@ -126,6 +126,7 @@ struct MeshGpt::Impl {
 
     // Prefill / logits workspace, grown on demand.
     DevBuf wx, wxn, wq, wy, wtok, wlogits, wk, wv;
+    DevBuf wlast;   // the last block's rows of a prefill (run_blocks)
     DevBuf wsplit;  // keys and values of one layer as attn_split's planes
 
     // Decode graphs replaying 1 and kGraphSteps steps.
@@ -467,11 +468,14 @@ struct MeshGpt::Impl {
     // block's attention between them.  kv_of(l) is block l's cache view.  With
     // `events`, each decode-attention launch stamps its own begin and end into
     // events[2l] and events[2l+1].
-    template <class KvOf>
     // `part_base` is the decode attention's partial-state buffer (default: the
-    // start of `part`).
-    void run_blocks(const kern::Rows &rows, int nseq, KvOf kv_of, float *x, float *x2, float *q, float *y,
-                    float *xn, bool decode, hipEvent_t *events = nullptr, float *part_base = nullptr) {
+    // start of `part`).  With `last` (a prefill of which only each sequence's
+    // last row is wanted) the last block may run for those rows alone: then xn
+    // holds one row a sequence and the result is true.
+    template <class KvOf>
+    bool run_blocks(const kern::Rows &rows, int nseq, KvOf kv_of, float *x, float *x2, float *q, float *y,
+                    float *xn, bool decode, hipEvent_t *events = nullptr, float *part_base = nullptr,
+                    bool last = false) {
         if (!part_base) part_base = part.as<float>();
         const int nsplit = decode ? splits_for(size_t(rows.rows)) : 0;
         // Prefill attention on the matrix cores (XSA in its epilogue) where the
@@ -492,6 +496,23 @@ struct MeshGpt::Impl {
         const bool rows_prefill = use_rows_prefill && kern::rows_block_supported(shape) && rows.len == nullptr;
         const BlockTiling t = block_tiling(size_t(rows.rows), decode);
         const size_t L = cfg.layers;
+        // The last block for the last rows alone: two more launches (the
+        // gather and the merge) against that block's attention and half of its
+        // meshes for every other row.
+        const int n = rows.rows_per_seq;
+        const bool compact = last && !decode && rows_prefill && mfma_prefill && last_row_pays(rows.rows);
+        const int last_split = compact ? splits_for(size_t(nseq)) : 0;
+        float *last_q = nullptr, *last_x = nullptr, *last_y = nullptr, *last_part = nullptr;
+        int *last_len = nullptr;
+        if (compact) {
+            const size_t row = size_t(nseq) * cfg.width;
+            wlast.ensure((3 * row + size_t(nseq) * (cfg.heads * size_t(last_split) * (shape.hdp + 2) + 1)) * 4);
+            last_q = wlast.as<float>();
+            last_x = last_q + row;
+            last_y = last_x + row;
+            last_part = last_y + row;
+            last_len = reinterpret_cast<int *>(last_part + size_t(nseq) * cfg.heads * last_split * (shape.hdp + 2));
+        }
         const bool rows_order = decode && row_decode;
         auto weights = [&](size_t id) { return rows_order ? group_rows(id) : group(id); };
         // The row-order kernel reads the residual rows from one buffer and
@@ -525,8 +546,14 @@ struct MeshGpt::Impl {
                 a.q = q;
                 a.kv_pre = kv_of(l);
                 a.rope = rope.as<float2>();
+                a.q_last = compact && l + 1 == L;
             } else {
                 a.xn = xn;
+                if (compact) {
+                    a.ro = kern::Rows{nseq, 1, nullptr, rows.tokens, rows.tok_stride, rows.tok_offset};
+                    a.x = a.x_out = last_x;
+                    a.ybuf = last_y;
+                }
             }
             if (rows_order) {
                 if (xout == xin) throw Error("row-order decode needs two residual buffers", kDeviceError);
@@ -543,6 +570,10 @@ struct MeshGpt::Impl {
             if (decode) {
                 kern::attn_decode(shape, q, kv_of(l), rows.len, rows.rows, nsplit, part_base, stream,
                                   events ? events[2 * l] : nullptr, events ? events[2 * l + 1] : nullptr);
+            } else if (compact && l + 1 == L) {
+                kern::last_rows(q, x, nseq, n, shape.W, last_q, last_x, last_len, stream);
+                kern::attn_decode(shape, last_q, kv_of(l), last_len, nseq, last_split, last_part, stream);
+                kern::last_merge(shape, last_part, last_split, kv_of(l), nseq, n, cfg.xsa, last_y, stream);
             } else if (mfma_prefill) {
                 const int2 *range = nullptr;
                 if (split_prefill)
@@ -554,7 +585,14 @@ struct MeshGpt::Impl {
                 kern::attn_prefill(shape, q, kv_of(l), nseq, rows.rows_per_seq, y, stream);
             }
         }
+        return compact;
     }
+
+    // Measured with and without (us a prefill): W128, two blocks, 1 x 250 rows
+    // 127 and 111, 8 x 128 105 and 102; W512, six blocks, 1 x 64 331 and 304,
+    // 8 x 65 332 and 342, 8 x 512 523 and 571; W1024, twelve blocks, 4 x 64 670
+    // and 704; W512, four blocks, 8 x 8192 7264 and 9058.
+    bool last_row_pays(int rows) const { return size_t(rows) * cfg.width >= size_t(1) << 18; }
 
     // Rows of each cached slab that decode attention reads with the default
     // cache policy (kern::kv_keep_rows; MG_KV_KEEP_ROWS overrides it).
@@ -569,14 +607,15 @@ struct MeshGpt::Impl {
 
     // Forward over a flat batch of sequences with a one-layer KV workspace
     // (each block's keys are consumed before the next block overwrites them).
-    void forward_rows(const uint32_t *tokens, size_t n, size_t sequence, size_t out_rows) {
+    // With `last` only the last rows' xn is wanted; true when it holds those alone.
+    bool forward_rows(const uint32_t *tokens, size_t n, size_t sequence, size_t out_rows, bool last = false) {
         ensure_workspace(n, out_rows, true);
         check(hipMemcpyAsync(wtok.p, tokens, n * 4, hipMemcpyHostToDevice, stream), "upload tokens");
         mark_call(0);
         kern::Rows rows{int(n), int(sequence), nullptr, wtok.as<uint32_t>(), int(sequence), 0};
         const kern::KvView kv{wk.as<float>(), wv.as<float>(), int(sequence)};
-        run_blocks(rows, int(n / sequence), [&](size_t) { return kv; }, wx.as<float>(), nullptr, wq.as<float>(),
-                   wy.as<float>(), wxn.as<float>(), false);
+        return run_blocks(rows, int(n / sequence), [&](size_t) { return kv; }, wx.as<float>(), nullptr,
+                          wq.as<float>(), wy.as<float>(), wxn.as<float>(), false, nullptr, nullptr, last);
     }
 
     std::vector<float> logits(const uint32_t *tokens, size_t n, size_t sequence, bool last_only) {
@@ -616,9 +655,10 @@ struct MeshGpt::Impl {
             a.scale = float(1.0 / std::sqrt(double(cfg.width / cfg.heads)));
             T::short_forward(a, int(n / sequence), stream);
         } else {
-            forward_rows(tokens, n, sequence, out_rows);
-            kern::head(shape, wxn.as<float>(), int(out_rows), last_only ? int(sequence) : 1,
-                       last_only ? int(sequence) - 1 : 0, Et.as<float>(), vpad, wlogits.as<float>(), head_rows(),
+            const bool compact = forward_rows(tokens, n, sequence, out_rows, last_only);
+            const bool strided = last_only && !compact;
+            kern::head(shape, wxn.as<float>(), int(out_rows), strided ? int(sequence) : 1,
+                       strided ? int(sequence) - 1 : 0, Et.as<float>(), vpad, wlogits.as<float>(), head_rows(),
                        stream);
         }
         mark_call(1);
@@ -930,7 +970,7 @@ struct MeshGpt::Impl {
         size_t total = 0;
         for (const DevBuf *b : {&params, &codes, &E, &Et, &rope, &wdec, &Edec, &q0, &kc, &vc, &dx, &dx2, &dxn, &dq,
                                 &part, &dtokens, &dlen, &drng, &dlogits, &dflags, &drng_start, &drng_next, &pxch, &pabort, &wx,
-                                &wxn, &wq, &wy, &wtok, &wlogits, &wk, &wv, &wsplit, &tact, &tgrad, &tm, &tv, &tpart, &tin})
+                                &wxn, &wq, &wy, &wtok, &wlogits, &wk, &wv, &wsplit, &wlast, &tact, &tgrad, &tm, &tv, &tpart, &tin})
             total += b->bytes;
         return total;
     }
@@ -1162,9 +1202,10 @@ struct MeshGpt::Impl {
     void prefill_step(size_t start, size_t n) {
         ensure_workspace(batch * n, 1, false);
         const kern::Rows rows{int(batch * n), int(n), nullptr, dtokens.as<uint32_t>(), int(tcap), int(start)};
-        run_blocks(rows, int(batch), [&](size_t l) { return cache_layer(l); }, wx.as<float>(), nullptr,
-                   wq.as<float>(), wy.as<float>(), wxn.as<float>(), false);
-        head_and_sample(wxn.as<float>(), int(n), int(n) - 1);
+        const bool compact = run_blocks(rows, int(batch), [&](size_t l) { return cache_layer(l); }, wx.as<float>(),
+                                        nullptr, wq.as<float>(), wy.as<float>(), wxn.as<float>(), false, nullptr,
+                                        nullptr, true);
+        head_and_sample(wxn.as<float>(), compact ? 1 : int(n), compact ? 0 : int(n) - 1);
     }
 
     // One generated token for every sequence (gpu.rs:2025-2050).

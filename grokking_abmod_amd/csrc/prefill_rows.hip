@@ -288,7 +288,8 @@ __global__ void __launch_bounds__(256) rows_block_kernel(BlockArgs a) {
 
     // Q, K and V meshes, one after another, each from the normalised rows.
     const size_t meshw = size_t(s.A) * W;
-    for (int m = 0; m < 3; ++m) {
+    const bool no_q = a.q_last && (r0 + C::R) / rps == r0 / rps && r0 + C::R < a.ro.rows;  // no sequence ends here
+    for (int m = no_q ? 1 : 0; m < 3; ++m) {
         const float *wm = m == 0 ? a.wq : (m == 1 ? a.wk : a.wv);
         float v[CPT][RG];
 #pragma unroll
@@ -330,6 +331,43 @@ __global__ void __launch_bounds__(256) rows_block_kernel(BlockArgs a) {
     }
 }
 
+// The last rows of `nseq` sequences of n rows, for attention over whole
+// sequences and blocks over single rows: q and x gathered, len filled with n.
+__global__ void __launch_bounds__(256)
+last_rows_kernel(const float *__restrict__ q, const float *__restrict__ x, int n, int W, float *__restrict__ q_out,
+                 float *__restrict__ x_out, int *__restrict__ len) {
+    const size_t from = (size_t(blockIdx.x) * n + n - 1) * W, to = size_t(blockIdx.x) * W;
+    for (int c = 4 * int(threadIdx.x); c < W; c += 1024) {
+        *reinterpret_cast<float4 *>(q_out + to + c) = *reinterpret_cast<const float4 *>(q + from + c);
+        *reinterpret_cast<float4 *>(x_out + to + c) = *reinterpret_cast<const float4 *>(x + from + c);
+    }
+    if (threadIdx.x == 0) len[blockIdx.x] = n;
+}
+
+// The split states (acc[hdp], m, l; log2 domain) of one (sequence, head) per
+// wave merged into its attention row, then XSA against the value row at n - 1
+// (reference.rs:577-603).
+__global__ void __launch_bounds__(256)
+last_merge_kernel(Shape s, const float *__restrict__ part, int nsplit, KvView kv, int n, int pairs, int xsa,
+                  float *__restrict__ y) {
+    const int pair = (int(blockIdx.x) * 256 + int(threadIdx.x)) >> 6, lane = int(threadIdx.x) & 63;
+    if (pair >= pairs) return;
+    const float *p = part + size_t(pair) * nsplit * (s.hdp + 2);
+    float top = -INFINITY;
+    for (int i = 0; i < nsplit; ++i) top = fmaxf(top, p[size_t(i) * (s.hdp + 2) + s.hdp]);
+    float sum = 0.0f, acc = 0.0f;
+    for (int i = 0; i < nsplit; ++i) {
+        const float *state = p + size_t(i) * (s.hdp + 2);
+        const float scale = __builtin_amdgcn_exp2f(state[s.hdp] - top);
+        sum = fmaf(state[s.hdp + 1], scale, sum);
+        if (lane < s.hd) acc = fmaf(state[lane], scale, acc);
+    }
+    acc /= sum;
+    const float v = lane < s.hd ? kv.v[(size_t(pair) * kv.cap + n - 1) * s.hdp + lane] : 0.0f;
+    const float vv = wave_sum(v * v), yv = wave_sum(acc * v), iv = rsqrtf(fmaxf(vv, kXsaNormFloor));
+    if (lane < s.hd) y[size_t(pair) * s.hd + lane] = xsa ? acc - (yv * iv) * (v * iv) : acc;
+}
+
 }  // namespace
 
 bool rows_block_supported(const Shape &s) {
@@ -355,6 +393,20 @@ void rows_block(const BlockArgs &a, hipStream_t stream) {
     case 512: launch_rows_block<512>(a, stream); break;
     default: launch_rows_block<1024>(a, stream); break;
     }
+    (void)hipGetLastError();
+}
+
+void last_rows(const float *q, const float *x, int nseq, int n, int W, float *q_out, float *x_out, int *len,
+               hipStream_t stream) {
+    hipLaunchKernelGGL(last_rows_kernel, dim3(nseq), dim3(256), 0, stream, q, x, n, W, q_out, x_out, len);
+    (void)hipGetLastError();
+}
+
+void last_merge(const Shape &s, const float *part, int nsplit, KvView kv, int nseq, int n, int xsa, float *y,
+                hipStream_t stream) {
+    const int pairs = nseq * s.H;
+    hipLaunchKernelGGL(last_merge_kernel, dim3((pairs + 3) / 4), dim3(256), 0, stream, s, part, nsplit, kv, n, pairs,
+                       xsa, y);
     (void)hipGetLastError();
 }
 

@@ -644,3 +644,30 @@ def test_split_prefill_reports_values_that_overflow():
         with pytest.raises(G.MeshGptError) as err:
             model.logits(G.random_prompts(64, 1, n, 7)[0], n, last_only=True)
         assert err.value.status == G.MG_NONFINITE
+
+
+# The last block for the last rows alone (from 2^18 channels of rows on): a
+# tile of rows that ends inside, at and across sequences, one and several key
+# splits, each register-tile width, against the same rows with every output
+# wanted; and one sequence fewer than the rule asks for.
+@pytest.mark.parametrize("W,H,n,batch", [(128, 4, 64, 32), (128, 4, 65, 32), (128, 2, 97, 22), (128, 2, 96, 22),
+                                         (256, 8, 129, 8), (256, 4, 1025, 1), (512, 8, 70, 8), (512, 8, 320, 2),
+                                         (1024, 16, 64, 4), (1024, 16, 259, 1), (512, 8, 511, 1), (512, 8, 513, 1)])
+def test_last_rows_alone_match_all_rows(W, H, n, batch):
+    """The last rows' logits: 1e-5 of their 2-norm, four times forty f32 roundings."""
+    kw = dict(vocab_size=64, context=n + 1, width=W, heads=H, layers=2, attention_mesh_depth=5, ffn_mesh_depth=4,
+              connectivity=1)
+    g = G.GptConfig(**kw)
+    tokens = G.random_prompts(64, batch, n, 11)
+    with G.MeshGpt(0, g, 7, max_batch=batch) as model:
+        model.set_parameters(G.normal_parameters(g, 3))
+        every = model.logits(tokens.reshape(-1), n).reshape(batch, n, 64)[:, -1]
+        last = model.logits(tokens.reshape(-1), n, last_only=True)
+        assert _prefill_error(last, every) <= 1e-5
+        model.prefill(tokens, 0.0, 7, reserve=n + 2)
+        assert _prefill_error(model.last_logits(batch), every) <= 1e-5
+        assert np.array_equal(model.read_tokens(batch)[:, -1], model.last_logits(batch).argmax(1))
+        model.decode(1)  # the cache of the last block is whole
+        again = np.concatenate([tokens, model.read_tokens(batch, n + 1)[:, n:]], 1)
+        again = model.logits(again.reshape(-1), n + 1, last_only=True)
+        assert _prefill_error(model.last_logits(batch), again) <= 1e-5
