@@ -177,7 +177,7 @@ int mg_model_config(const mg_model *model, mg_config *out) {
 }
 
 int mg_parameters(mg_model *model, float *out, size_t n) {
-    return guarded([&] { copy_out(model_of(model).parameters(), out, n); });
+    return guarded([&] { model_of(model).parameters(out, n); });
 }
 
 int mg_set_parameters(mg_model *model, const float *values, size_t n) {
@@ -192,7 +192,7 @@ int mg_logits(mg_model *model, const uint32_t *tokens, size_t n, size_t sequence
     return guarded([&] {
         require(tokens != nullptr || n == 0, "tokens must not be null");
         static const uint32_t none = 0;
-        copy_out(model_of(model).logits(tokens ? tokens : &none, n, sequence, last_only != 0), out, out_len);
+        model_of(model).logits(tokens ? tokens : &none, n, sequence, last_only != 0, out, out_len);
     });
 }
 
@@ -244,10 +244,7 @@ int mg_loss_and_gradient(mg_model *model, const uint32_t *inputs, const uint32_t
                          size_t sequence, double *loss, float *gradient, size_t n_gradient) {
     return guarded([&] {
         require(inputs != nullptr && targets != nullptr && loss != nullptr, "inputs, targets and loss must not be null");
-        std::vector<float> g;
-        const double l = model_of(model).loss_and_gradient(inputs, targets, n, sequence, g);
-        copy_out(g, gradient, n_gradient);
-        *loss = l;
+        *loss = model_of(model).loss_and_gradient(inputs, targets, n, sequence, gradient, n_gradient);
     });
 }
 
@@ -275,7 +272,7 @@ int mg_hidden_states(mg_model *model, const uint32_t *tokens, size_t n, size_t s
     return guarded([&] {
         require(tokens != nullptr || n == 0, "tokens must not be null");
         static const uint32_t none = 0;
-        copy_out(model_of(model).hidden_states(tokens ? tokens : &none, n, sequence), out, out_len);
+        model_of(model).hidden_states(tokens ? tokens : &none, n, sequence, out, out_len);
     });
 }
 
@@ -353,7 +350,7 @@ int mg_read_tokens(mg_model *model, uint32_t *out, size_t batch, size_t length) 
 }
 
 int mg_last_logits(mg_model *model, float *out, size_t n) {
-    return guarded([&] { copy_out(model_of(model).last_logits(), out, n); });
+    return guarded([&] { model_of(model).last_logits(out, n); });
 }
 
 void *mg_model_stream(mg_model *model) { return model ? static_cast<void *>(model->model.stream()) : nullptr; }

@@ -284,6 +284,14 @@ constexpr int kNoAllocRows = 65536;
 hipError_t noalloc_scratch(int device, int **out);
 // p[0..n) = value, by a kernel (no memset node when a caller captures the stream).
 void fill_int(int *p, int value, int n, hipStream_t stream);
+// The decode state of a new batch: row b of `tokens` (`stride` apart) begins with
+// the n tokens at prompts + b n, len[b] = n, rng[b] = seed + b, *flags = 0.
+void start_rows(const uint32_t *prompts, int batch, int n, uint32_t *tokens, size_t stride, int *len, uint64_t *rng,
+                uint64_t seed, int *flags, hipStream_t stream);
+// out[b n ..) = the first n tokens of row b.
+void gather_rows(const uint32_t *tokens, size_t stride, int batch, int n, uint32_t *out, hipStream_t stream);
+// *flag = 1 when a value of x[0..n) is not finite, else 0.
+void nonfinite(const float *x, size_t n, int *flag, hipStream_t stream);
 // y[i] = the sampler's f32 exp of x[i] (for verification).
 void device_expf(const float *x, float *y, size_t n, hipStream_t stream);
 // dst[i] = src[i] for n float4 elements (bandwidth calibration).

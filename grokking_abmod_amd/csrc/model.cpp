@@ -126,6 +126,14 @@ struct MeshGpt::Impl {
 
     // Prefill / logits workspace, grown on demand.
     DevBuf wx, wxn, wq, wy, wtok, wlogits, wk, wv;
+    // Transfers: pinned staging of uploads and downloads (a model's own, fixed
+    // in size), contiguous tokens on the device, and the finiteness flag.
+    static constexpr size_t kUpload = size_t(1) << 20, kChunk = size_t(512) << 10, kChunks = 4, kWords = 256;
+    PinnedBuf hup, hdown;
+    DevBuf dstage, dbad;
+    hipEvent_t chunk_ev[kChunks] = {};
+    bool upload_busy = false;    // hup may still be read by the stream
+    int known_flags = -1;        // dflags' value when the host has it
     DevBuf wlast;   // the last block's rows of a prefill (run_blocks)
     DevBuf wsplit;  // keys and values of one layer as attn_split's planes
 
@@ -191,6 +199,8 @@ struct MeshGpt::Impl {
         drop_graph();
         drop_train_graph();
         for (hipEvent_t e : call_ev)
+            if (e) (void)hipEventDestroy(e);
+        for (hipEvent_t e : chunk_ev)
             if (e) (void)hipEventDestroy(e);
         for (int i = 0; i < kMaxSlices - 1; ++i) {
             if (join_ev[i]) (void)hipEventDestroy(join_ev[i]);
@@ -286,6 +296,10 @@ struct MeshGpt::Impl {
         kern::configure_lds(lds_limit);
         check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
         for (hipEvent_t &e : call_ev) check(hipEventCreate(&e), "hipEventCreate");
+        for (hipEvent_t &e : chunk_ev) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+        hup.ensure(kUpload);
+        hdown.ensure(kChunk * kChunks + kWords);
+        dbad.ensure(4);
         use_graph = env_int("MG_DISABLE_GRAPH", 0) == 0;
 
         const size_t W = cfg.width, hd = cfg.head_width();
@@ -400,6 +414,89 @@ struct MeshGpt::Impl {
     void sync() {
         check(hipGetLastError(), "kernel launch");
         check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        upload_busy = false;
+    }
+
+    // dst[0..bytes) = src on the stream.  Staged in pinned memory where it
+    // fits, so that src is free when this returns; a larger upload waits.
+    void upload(void *dst, const void *src, size_t bytes, const char *what) {
+        if (bytes <= kUpload) {
+            if (upload_busy) sync();
+            std::memcpy(hup.p, src, bytes);
+            check(hipMemcpyAsync(dst, hup.p, bytes, hipMemcpyHostToDevice, stream), what);
+            upload_busy = true;
+        } else {
+            check(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream), what);
+            sync();
+        }
+    }
+
+    // A word of host memory that the stream may write; valid until the next
+    // sync() has passed and another call of the same slot.
+    int *word(int slot) const { return reinterpret_cast<int *>(hdown.as<char>() + kChunk * kChunks) + slot; }
+    enum { kFlagsWord = 0, kBadWord = 1, kStatusWord = 2 };
+
+    // out[0..bytes) = src once the stream has reached this point: pinned chunks,
+    // the copy out of one beside the transfers of the next ones.  `ready` runs
+    // after the first transfer has arrived and before out is written (it may
+    // throw; what the stream did before this call is then known to the host).
+    template <class Ready>
+    void download(void *out, const void *src, size_t bytes, const char *what, Ready ready) {
+        const size_t chunks = (bytes + kChunk - 1) / kChunk;
+        auto size = [&](size_t i) { return std::min(kChunk, bytes - i * kChunk); };
+        auto issue = [&](size_t i) {
+            check(hipMemcpyAsync(hdown.as<char>() + i % kChunks * kChunk, static_cast<const char *>(src) + i * kChunk,
+                                 size(i), hipMemcpyDeviceToHost, stream),
+                  what);
+            if (chunks > 1) check(hipEventRecord(chunk_ev[i % kChunks], stream), "hipEventRecord");
+        };
+        for (size_t i = 0; i < std::min(chunks, kChunks); ++i) issue(i);
+        if (chunks <= 1) {
+            sync();
+            ready();
+        }
+        for (size_t i = 0; i < chunks; ++i) {
+            if (chunks > 1) {
+                check(hipEventSynchronize(chunk_ev[i % kChunks]), "hipEventSynchronize");
+                if (i == 0) {
+                    try {
+                        ready();
+                    } catch (...) {
+                        (void)hipStreamSynchronize(stream);
+                        throw;
+                    }
+                }
+            }
+            std::memcpy(static_cast<char *>(out) + i * kChunk, hdown.as<char>() + i % kChunks * kChunk, size(i));
+            if (i + kChunks < chunks) issue(i + kChunks);
+        }
+        if (chunks > 1) sync();
+    }
+
+    // The same for n floats that must be finite (validate_finite's error).
+    template <class Ready>
+    void download_finite(float *out, const float *src, size_t n, const char *name, Ready ready) {
+        // Few values are looked through here (12288: 4 us), more where they lie
+        // (two launches and a word's copy, 15 us).
+        constexpr size_t kHostCheck = 32768;
+        static_assert(kHostCheck * 4 <= kChunk, "in one chunk");
+        if (n <= kHostCheck) {
+            download(out, src, n * 4, "download", [&] {
+                ready();
+                validate_finite(hdown.as<float>(), n, name);
+            });
+            return;
+        }
+        kern::nonfinite(src, n, dbad.as<int>(), stream);
+        check(hipMemcpyAsync(word(kBadWord), dbad.p, 4, hipMemcpyDeviceToHost, stream), "download check");
+        download(out, src, n * 4, "download", [&] {
+            ready();
+            if (*word(kBadWord)) throw Error(std::string(name) + " must contain only finite values", kNonfinite);
+        });
+    }
+
+    static void check_capacity(const float *out, size_t capacity, size_t n) {
+        if (out == nullptr || capacity < n) throw Error("output buffer is too small");
     }
 
     void ensure_decode(size_t b, size_t t) {
@@ -610,7 +707,7 @@ struct MeshGpt::Impl {
     // With `last` only the last rows' xn is wanted; true when it holds those alone.
     bool forward_rows(const uint32_t *tokens, size_t n, size_t sequence, size_t out_rows, bool last = false) {
         ensure_workspace(n, out_rows, true);
-        check(hipMemcpyAsync(wtok.p, tokens, n * 4, hipMemcpyHostToDevice, stream), "upload tokens");
+        upload(wtok.p, tokens, n * 4, "upload tokens");
         mark_call(0);
         kern::Rows rows{int(n), int(sequence), nullptr, wtok.as<uint32_t>(), int(sequence), 0};
         const kern::KvView kv{wk.as<float>(), wv.as<float>(), int(sequence)};
@@ -618,17 +715,18 @@ struct MeshGpt::Impl {
                           wq.as<float>(), wy.as<float>(), wxn.as<float>(), false, nullptr, nullptr, last);
     }
 
-    std::vector<float> logits(const uint32_t *tokens, size_t n, size_t sequence, bool last_only) {
+    void logits(const uint32_t *tokens, size_t n, size_t sequence, bool last_only, float *out, size_t capacity) {
         cfg.validate_tokens(tokens, n, sequence);
+        const size_t out_rows = last_only ? n / sequence : n;
+        check_capacity(out, capacity, out_rows * cfg.vocab_size);
         activate();
         ensure_derived();
-        const size_t out_rows = last_only ? n / sequence : n;
         namespace T = kern::train;
         if (T::short_forward_fits(int(cfg.width), int(cfg.heads), cfg.vocab_size, int(sequence))) {
             // Sequences of up to 16 rows: the whole forward and the head in one
             // launch, a workgroup per sequence.
             ensure_workspace(n, out_rows, true);
-            check(hipMemcpyAsync(wtok.p, tokens, n * 4, hipMemcpyHostToDevice, stream), "upload tokens");
+            upload(wtok.p, tokens, n * 4, "upload tokens");
             mark_call(0);
             T::ShortForward a{};
             a.E = E.as<float>();
@@ -662,27 +760,17 @@ struct MeshGpt::Impl {
                        stream);
         }
         mark_call(1);
-        std::vector<float> out(out_rows * cfg.vocab_size);
-        check(hipMemcpyAsync(out.data(), wlogits.p, out.size() * 4, hipMemcpyDeviceToHost, stream),
-              "download logits");
-        sync();
-        close_call();
-        validate_finite(out.data(), out.size(), "logits");
-        return out;
+        download_finite(out, wlogits.as<float>(), out_rows * cfg.vocab_size, "logits", [&] { close_call(); });
     }
 
-    std::vector<float> hidden_states(const uint32_t *tokens, size_t n, size_t sequence) {
+    void hidden_states(const uint32_t *tokens, size_t n, size_t sequence, float *out, size_t capacity) {
         cfg.validate_tokens(tokens, n, sequence);
+        check_capacity(out, capacity, n * cfg.width);
         activate();
         ensure_derived();
         forward_rows(tokens, n, sequence, 1);
         mark_call(1);
-        std::vector<float> out(n * cfg.width);
-        check(hipMemcpyAsync(out.data(), wx.p, out.size() * 4, hipMemcpyDeviceToHost, stream), "download");
-        sync();
-        close_call();
-        validate_finite(out.data(), out.size(), "features");
-        return out;
+        download_finite(out, wx.as<float>(), n * cfg.width, "features", [&] { close_call(); });
     }
 
     // ---- training -------------------------------------------------------------
@@ -969,7 +1057,7 @@ struct MeshGpt::Impl {
     size_t allocated_device_bytes() const {
         size_t total = 0;
         for (const DevBuf *b : {&params, &codes, &E, &Et, &rope, &wdec, &Edec, &q0, &kc, &vc, &dx, &dx2, &dxn, &dq,
-                                &part, &dtokens, &dlen, &drng, &dlogits, &dflags, &drng_start, &drng_next, &pxch, &pabort, &wx,
+                                &part, &dtokens, &dlen, &drng, &dlogits, &dflags, &drng_start, &drng_next, &dstage, &dbad, &pxch, &pabort, &wx,
                                 &wxn, &wq, &wy, &wtok, &wlogits, &wk, &wv, &wsplit, &wlast, &tact, &tgrad, &tm, &tv, &tpart, &tin})
             total += b->bytes;
         return total;
@@ -998,12 +1086,7 @@ struct MeshGpt::Impl {
         return train_loss(n, supervised);
     }
 
-    std::vector<float> gradient() {
-        std::vector<float> out(layout.count());
-        check(hipMemcpy(out.data(), tgrad.p, out.size() * 4, hipMemcpyDeviceToHost), "download gradients");
-        validate_finite(out.data(), out.size(), "gradients");
-        return out;
-    }
+    void gradient(float *out) { download_finite(out, tgrad.as<float>(), layout.count(), "gradients", [] {}); }
 
     // gpu.rs:1971-2003: the gradient, then one AdamW update of every group
     // (the embedding group stays when the geometry is frozen).  The whole
@@ -1058,15 +1141,11 @@ struct MeshGpt::Impl {
         activate();
         ensure_derived();
         ensure_decode(b, std::max(reserve, p));
-        check(hipMemcpy2DAsync(dtokens.p, tcap * 4, prompts, p * 4, p * 4, b, hipMemcpyHostToDevice, stream),
-              "upload prompts");
-        std::vector<int> lens(b, int(p));
-        std::vector<uint64_t> states(b);
-        for (size_t i = 0; i < b; ++i) states[i] = seed + i;
-        check(hipMemcpyAsync(dlen.p, lens.data(), b * 4, hipMemcpyHostToDevice, stream), "upload lengths");
-        check(hipMemcpyAsync(drng.p, states.data(), b * 8, hipMemcpyHostToDevice, stream), "upload rng");
-        check(hipMemsetAsync(dflags.p, 0, 4, stream), "clear flags");
-        sync();
+        dstage.ensure(b * std::max(reserve, p) * 4);
+        upload(dstage.p, prompts, b * p * 4, "upload prompts");
+        kern::start_rows(dstage.as<uint32_t>(), int(b), int(p), dtokens.as<uint32_t>(), tcap, dlen.as<int>(),
+                         drng.as<uint64_t>(), seed, dflags.as<int>(), stream);
+        known_flags = -1;
         batch = b;
         length = p;
         cached = 0;
@@ -1161,6 +1240,7 @@ struct MeshGpt::Impl {
     }
 
     void launch_decode_step(hipEvent_t *events = nullptr) {
+        known_flags = -1;
         const kern::Rows rows{int(batch), 1, dlen.as<int>(), dtokens.as<uint32_t>(), int(tcap), 0};
         run_blocks(rows, int(batch), [&](size_t l) { return cache_layer(l); }, dx.as<float>(), dx2.as<float>(),
                    dq.as<float>(), nullptr, dxn.as<float>(), true, events);
@@ -1170,6 +1250,7 @@ struct MeshGpt::Impl {
     // `n` decode steps (1 or kGraphSteps) as one graph replay; the graphs are
     // captured on first use for the current batch and temperature.
     void decode_steps(size_t n) {
+        known_flags = -1;
         const int slices = decode_slices();
         auto enqueue = [&] {
             if (slices > 1)
@@ -1211,6 +1292,7 @@ struct MeshGpt::Impl {
     // One generated token for every sequence (gpu.rs:2025-2050).
     void step() {
         if (length + 1 > tcap) throw Error("generation exceeds the reserved token capacity");
+        known_flags = -1;
         if (length <= cfg.context && cached == length - 1) {
             decode_step();
             cached = length;
@@ -1234,6 +1316,7 @@ struct MeshGpt::Impl {
     // decode to that length leaves it.
     void window(size_t steps) {
         if (length + steps > tcap) throw Error("generation exceeds the reserved token capacity");
+        known_flags = -1;
         constexpr size_t kLaunchSteps = 4096;  // bounds a launch to some tens of milliseconds
         for (size_t done = 0; done < steps;) {
             const size_t n = std::min(steps - done, kLaunchSteps), before = length + n - 1;
@@ -1270,19 +1353,34 @@ struct MeshGpt::Impl {
         }
     }
 
-    void finish() {
-        sync();
-        int flags = 0;
-        check(hipMemcpy(&flags, dflags.p, 4, hipMemcpyDeviceToHost), "download flags");
-        if (flags) throw Error("logits must contain only finite values", kNonfinite);
+    void fetch_flags() {
+        check(hipMemcpyAsync(word(kFlagsWord), dflags.p, 4, hipMemcpyDeviceToHost, stream), "download flags");
+    }
+    void check_flags() const {
+        if (known_flags > 0) throw Error("logits must contain only finite values", kNonfinite);
     }
 
-    void read_tokens(uint32_t *out, size_t b, size_t len) {
+    void finish() {
+        if (known_flags < 0) {
+            fetch_flags();
+            sync();
+            known_flags = *word(kFlagsWord);
+        }
+        check_flags();
+    }
+
+    // The first len tokens of b sequences; with `checked`, finish() on the way.
+    void read_tokens(uint32_t *out, size_t b, size_t len, bool checked = false) {
         if (b > batch || len > length) throw Error("requested tokens exceed the generated sequences");
         activate();
-        check(hipMemcpy2DAsync(out, len * 4, dtokens.p, tcap * 4, len * 4, b, hipMemcpyDeviceToHost, stream),
-              "download tokens");
-        sync();
+        dstage.ensure(b * len * 4);
+        kern::gather_rows(dtokens.as<uint32_t>(), tcap, int(b), int(len), dstage.as<uint32_t>(), stream);
+        const bool ask = checked && known_flags < 0;
+        if (ask) fetch_flags();
+        download(out, dstage.p, b * len * 4, "download tokens", [&] {
+            if (ask) known_flags = *word(kFlagsWord);
+            if (checked) check_flags();
+        });
     }
 
     bool decodable(size_t steps) const {
@@ -1364,10 +1462,11 @@ struct MeshGpt::Impl {
         }
         check(launched, "persistent decode launch");
         mark_call(1);
+        int *status = word(kStatusWord);
+        check(hipMemcpyAsync(status, pabort.p, 8, hipMemcpyDeviceToHost, stream), "download abort flag");
+        fetch_flags();
         sync();
         close_call();
-        int status[2] = {0, 0};
-        check(hipMemcpy(status, pabort.p, 8, hipMemcpyDeviceToHost), "download abort flag");
         if (status[0]) {
             // Every sequence back at the launch's starting length; the sampler
             // states in drng were not touched.
@@ -1379,6 +1478,7 @@ struct MeshGpt::Impl {
         std::swap(drng.p, drng_next.p);
         std::swap(drng.bytes, drng_next.bytes);
         if (status[1]) check(hipMemsetD32Async(hipDeviceptr_t(dflags.p), 1, 1, stream), "flag non-finite logits");
+        known_flags = *word(kFlagsWord) | status[1];
         cached = length + steps - 1;
         length += steps;
         return true;
@@ -1395,17 +1495,29 @@ MeshGpt::~MeshGpt() = default;
 const GptConfig &MeshGpt::config() const { return impl_->cfg; }
 
 std::vector<float> MeshGpt::parameters() const {
-    impl_->activate();
     std::vector<float> out(impl_->layout.count());
-    check(hipMemcpy(out.data(), impl_->params.p, out.size() * 4, hipMemcpyDeviceToHost), "download parameters");
-    validate_finite(out.data(), out.size(), "parameters");
+    parameters(out.data(), out.size());
     return out;
+}
+
+void MeshGpt::parameters(float *out, size_t capacity) const {
+    Impl &m = *impl_;
+    Impl::check_capacity(out, capacity, m.layout.count());
+    m.activate();
+    m.download_finite(out, m.params.as<float>(), m.layout.count(), "parameters", [] {});
 }
 
 void MeshGpt::set_parameters(const float *values, size_t n) { impl_->set_parameters(values, n); }
 
 std::vector<float> MeshGpt::logits(const uint32_t *tokens, size_t n, size_t sequence, bool last_only) {
-    return impl_->logits(tokens, n, sequence, last_only);
+    impl_->cfg.validate_tokens(tokens, n, sequence);
+    std::vector<float> out((last_only ? n / sequence : n) * impl_->cfg.vocab_size);
+    impl_->logits(tokens, n, sequence, last_only, out.data(), out.size());
+    return out;
+}
+
+void MeshGpt::logits(const uint32_t *tokens, size_t n, size_t sequence, bool last_only, float *out, size_t capacity) {
+    impl_->logits(tokens, n, sequence, last_only, out, capacity);
 }
 
 std::vector<float> MeshGpt::token_embeddings() {
@@ -1423,8 +1535,15 @@ double MeshGpt::cross_entropy(const uint32_t *inputs, const uint32_t *targets, s
 
 double MeshGpt::loss_and_gradient(const uint32_t *inputs, const uint32_t *targets, size_t n, size_t sequence,
                                   std::vector<float> &gradient) {
+    gradient.resize(impl_->layout.count());
+    return loss_and_gradient(inputs, targets, n, sequence, gradient.data(), gradient.size());
+}
+
+double MeshGpt::loss_and_gradient(const uint32_t *inputs, const uint32_t *targets, size_t n, size_t sequence,
+                                  float *gradient, size_t capacity) {
     const double loss = impl_->train_pass(inputs, targets, n, sequence, true);
-    gradient = impl_->gradient();
+    Impl::check_capacity(gradient, capacity, impl_->layout.count());
+    impl_->gradient(gradient);
     return loss;
 }
 
@@ -1436,7 +1555,14 @@ double MeshGpt::train_batch(const uint32_t *inputs, const uint32_t *targets, siz
 size_t MeshGpt::allocated_device_bytes() const { return impl_->allocated_device_bytes(); }
 
 std::vector<float> MeshGpt::hidden_states(const uint32_t *tokens, size_t n, size_t sequence) {
-    return impl_->hidden_states(tokens, n, sequence);
+    impl_->cfg.validate_tokens(tokens, n, sequence);
+    std::vector<float> out(n * impl_->cfg.width);
+    impl_->hidden_states(tokens, n, sequence, out.data(), out.size());
+    return out;
+}
+
+void MeshGpt::hidden_states(const uint32_t *tokens, size_t n, size_t sequence, float *out, size_t capacity) {
+    impl_->hidden_states(tokens, n, sequence, out, capacity);
 }
 
 void MeshGpt::generate_tokens(const uint32_t *prompts, size_t batch, size_t prompt_len, size_t count,
@@ -1463,8 +1589,7 @@ void MeshGpt::generate_tokens(const uint32_t *prompts, size_t batch, size_t prom
         done = count;
     }
     for (; done < count; ++done) m.step();
-    m.finish();
-    m.read_tokens(out, batch, prompt_len + count);
+    m.read_tokens(out, batch, prompt_len + count, true);
 }
 
 std::string MeshGpt::generate(const CharacterTokenizer &tokenizer, const std::string &prompt, size_t count,
@@ -1487,11 +1612,10 @@ void MeshGpt::prefill(const uint32_t *prompts, size_t batch, size_t prompt_len, 
     m.mark_call(0);
     m.step();
     m.mark_call(1);
+    check(hipMemcpyAsync(m.drng_start.p, m.drng.p, m.batch * 8, hipMemcpyDeviceToDevice, m.stream), "save rng");
     m.finish();
     m.close_call();
-    check(hipMemcpyAsync(m.drng_start.p, m.drng.p, m.batch * 8, hipMemcpyDeviceToDevice, m.stream), "save rng");
     m.start_length = m.length;
-    m.sync();
 }
 
 void MeshGpt::rewind() {
@@ -1575,11 +1699,17 @@ float MeshGpt::last_call_ms() const { return impl_->call_ms; }
 void MeshGpt::read_tokens(uint32_t *out, size_t batch, size_t length) { impl_->read_tokens(out, batch, length); }
 
 std::vector<float> MeshGpt::last_logits() {
-    Impl &m = *impl_;
-    m.activate();
-    std::vector<float> out(m.batch * m.cfg.vocab_size);
-    check(hipMemcpy(out.data(), m.dlogits.p, out.size() * 4, hipMemcpyDeviceToHost), "download logits");
+    std::vector<float> out(impl_->batch * impl_->cfg.vocab_size);
+    last_logits(out.data(), out.size());
     return out;
+}
+
+void MeshGpt::last_logits(float *out, size_t capacity) {
+    Impl &m = *impl_;
+    const size_t n = m.batch * m.cfg.vocab_size;
+    Impl::check_capacity(out, capacity, n);
+    m.activate();
+    if (n) m.download(out, m.dlogits.p, n * 4, "download logits", [] {});
 }
 
 hipStream_t MeshGpt::stream() const { return impl_->stream; }

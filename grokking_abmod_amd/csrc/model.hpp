@@ -28,6 +28,12 @@ class MeshGpt {
     void set_parameters(const float *values, size_t n);     // gpu.rs:1856-1872
     // gpu.rs:1875-1887: logits of every row (or only each sequence's last row)
     std::vector<float> logits(const uint32_t *tokens, size_t n, size_t sequence, bool last_only = false);
+    // The results of the calls of the same names, written to out, which holds
+    // `capacity` floats.  On an error out is as it was.
+    void logits(const uint32_t *tokens, size_t n, size_t sequence, bool last_only, float *out, size_t capacity);
+    void parameters(float *out, size_t capacity) const;
+    void hidden_states(const uint32_t *tokens, size_t n, size_t sequence, float *out, size_t capacity);
+    void last_logits(float *out, size_t capacity);
     std::vector<float> token_embeddings();                  // gpu.rs:2056-2068, V x W
     std::vector<float> hidden_states(const uint32_t *tokens, size_t n, size_t sequence);  // gpu.rs:2070
     // Training (gpu.rs:1915-2003).  Targets equal to kIgnoreTarget are not
@@ -38,6 +44,8 @@ class MeshGpt {
     double cross_entropy(const uint32_t *inputs, const uint32_t *targets, size_t n, size_t sequence);
     double loss_and_gradient(const uint32_t *inputs, const uint32_t *targets, size_t n, size_t sequence,
                              std::vector<float> &gradient);
+    double loss_and_gradient(const uint32_t *inputs, const uint32_t *targets, size_t n, size_t sequence,
+                             float *gradient, size_t capacity);
     double train_batch(const uint32_t *inputs, const uint32_t *targets, size_t n, size_t sequence,
                        const AdamWOptions &options);
     // Bytes of device memory the model holds (gpu.rs allocated_device_bytes).
