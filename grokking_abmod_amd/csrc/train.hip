@@ -577,7 +577,11 @@ __global__ void __launch_bounds__(kThreads) rmsnorm_backward_kernel(const float 
     }
 }
 
-// ---- one wave per (row, head), lanes over the head's dims (dim lane + 64 e)
+// ---- one group of G lanes per (row, head), lanes over the head's dims (dim
+// lane + 64 e, G = 64 where a lane holds more than one): heads of up to 8, 16 or
+// 32 dims share a wave, so that its lanes are used and one load brings 64 / G
+// rows.  The sums over a group add what the sum over a wave with zeros in the
+// other lanes adds, in the same order.
 
 template <int EPL>
 __device__ __forceinline__ void lanes_load(const float *row, int hd, int lane, float (&v)[EPL]) {
@@ -592,16 +596,17 @@ __device__ __forceinline__ void lanes_store(float *row, int hd, int lane, const 
         if (lane + 64 * e < hd) row[lane + 64 * e] = v[e];
 }
 
-template <int EPL>
+template <int G, int EPL>
 __device__ __forceinline__ float lanes_dot(const float (&a)[EPL], const float (&b)[EPL]) {
     float acc = 0.0f;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) acc = fmaf(a[e], b[e], acc);
-    return wave_sum(acc);
+    if constexpr (G == 64) return wave_sum(acc);
+    return group_sum<G>(acc);
 }
 
 // The RoPE partner of each lane's dims (d + half or d - half).
-template <int EPL>
+template <int G, int EPL>
 __device__ __forceinline__ void lanes_partner(const float (&x)[EPL], int hd, int lane, float (&out)[EPL]) {
     const int half = hd / 2;
     if (EPL > 1 && half % 64 == 0) {
@@ -618,13 +623,14 @@ __device__ __forceinline__ void lanes_partner(const float (&x)[EPL], int hd, int
         }
         return;
     }
+    const int base = int(threadIdx.x) & 63 & ~(G - 1);
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
         const int d = lane + 64 * e, pd = d < half ? d + half : d - half;
         float v = 0.0f;
 #pragma unroll
         for (int f = 0; f < EPL; ++f) {
-            const float t = __shfl(x[f], pd & 63, 64);
+            const float t = __shfl(x[f], base + (pd & (G - 1)), 64);
             if ((pd >> 6) == f) v = t;
         }
         out[e] = d < hd ? v : 0.0f;
@@ -632,29 +638,36 @@ __device__ __forceinline__ void lanes_partner(const float (&x)[EPL], int hd, int
 }
 
 __device__ __forceinline__ int row_wave() { return int((blockIdx.x * kThreads + threadIdx.x) >> 6); }
+template <int G>
+__device__ __forceinline__ int row_group() { return int((blockIdx.x * kThreads + threadIdx.x) / G); }
+
+// Keys (or queries) whose rows a group loads before it works through them in
+// order: their loads and products overlap, the sums stay in row order.
+template <int EPL>
+constexpr int kBatch = EPL <= 2 ? 4 : 1;
 
 // QK-Norm (per-head RMSNorm) then RoPE of row r, head h, in place; inv keeps
 // the norm's factor (reference.rs:174-193, 392-409, 462-482).
-template <int EPL>
+template <int EPL, int G>
 __global__ void __launch_bounds__(kThreads) qk_forward_kernel(QkSet set, const float2 *__restrict__ table, int rows,
                                                               int sequence, int W, int H, int norm, int rotate) {
     float *x = set.out[blockIdx.y];
     const float *__restrict__ pre = set.pre[blockIdx.y];
     float *__restrict__ inv = set.inv[blockIdx.y];
-    const int t = row_wave(), lane = threadIdx.x & 63;
+    const int t = row_group<G>(), lane = threadIdx.x & (G - 1);
     if (t >= rows * H) return;
     const int r = t / H, h = t % H, hd = W / H, half = hd / 2;
     float v[EPL];
     lanes_load(pre + size_t(r) * W + h * hd, hd, lane, v);
     if (norm) {
-        const float iv = rsqrtf(lanes_dot(v, v) * (1.0f / float(hd)) + kRmsEps);
+        const float iv = rsqrtf(lanes_dot<G>(v, v) * (1.0f / float(hd)) + kRmsEps);
 #pragma unroll
         for (int e = 0; e < EPL; ++e) v[e] *= iv;
         if (lane == 0) inv[t] = iv;
     }
     if (rotate) {
         float o[EPL];
-        lanes_partner(v, hd, lane, o);
+        lanes_partner<G>(v, hd, lane, o);
 #pragma unroll
         for (int e = 0; e < EPL; ++e) {
             const int d = lane + 64 * e;
@@ -667,13 +680,13 @@ __global__ void __launch_bounds__(kThreads) qk_forward_kernel(QkSet set, const f
 
 // Its backward in place on g: the transposed rotation, then the norm's
 // backward against the pre-norm rows `pre`.
-template <int EPL>
+template <int EPL, int G>
 __global__ void __launch_bounds__(kThreads) qk_backward_kernel(QkSet set, const float2 *__restrict__ table, int rows,
                                                                int sequence, int W, int H, int norm, int rotate) {
     float *g = set.out[blockIdx.y];
     const float *__restrict__ pre = set.pre[blockIdx.y];
     const float *__restrict__ inv = set.inv[blockIdx.y];
-    const int t = row_wave(), lane = threadIdx.x & 63;
+    const int t = row_group<G>(), lane = threadIdx.x & (G - 1);
     if (t >= rows * H) return;
     const int r = t / H, h = t % H, hd = W / H, half = hd / 2;
     float *row = g + size_t(r) * W + h * hd;
@@ -681,7 +694,7 @@ __global__ void __launch_bounds__(kThreads) qk_backward_kernel(QkSet set, const 
     lanes_load(row, hd, lane, v);
     if (rotate) {
         float o[EPL];
-        lanes_partner(v, hd, lane, o);
+        lanes_partner<G>(v, hd, lane, o);
 #pragma unroll
         for (int e = 0; e < EPL; ++e) {
             const int d = lane + 64 * e;
@@ -692,7 +705,7 @@ __global__ void __launch_bounds__(kThreads) qk_backward_kernel(QkSet set, const 
     if (norm) {
         float x[EPL];
         lanes_load(pre + size_t(r) * W + h * hd, hd, lane, x);
-        const float iv = inv[t], k = lanes_dot(v, x) * iv * iv * iv * (1.0f / float(hd));
+        const float iv = inv[t], k = lanes_dot<G>(v, x) * iv * iv * iv * (1.0f / float(hd));
 #pragma unroll
         for (int e = 0; e < EPL; ++e) v[e] = iv * v[e] - x[e] * k;
     }
@@ -702,13 +715,13 @@ __global__ void __launch_bounds__(kThreads) qk_backward_kernel(QkSet set, const 
 // Causal attention for short sequences: one wave per query row and head.
 // XSA of one (row, head) in a wave's lanes (reference.rs:577-603): y minus
 // its component along u = v / max(|v|, 1e-12), in place.
-template <int EPL>
+template <int G, int EPL>
 __device__ __forceinline__ void lanes_xsa(float (&yv)[EPL], const float (&v)[EPL]) {
     float u[EPL];
-    const float inv = rsqrtf(fmaxf(lanes_dot(v, v), kXsaFloor));
+    const float inv = rsqrtf(fmaxf(lanes_dot<G>(v, v), kXsaFloor));
 #pragma unroll
     for (int e = 0; e < EPL; ++e) u[e] = v[e] * inv;
-    const float s = lanes_dot(yv, u);
+    const float s = lanes_dot<G>(yv, u);
 #pragma unroll
     for (int e = 0; e < EPL; ++e) yv[e] -= s * u[e];
 }
@@ -716,49 +729,59 @@ __device__ __forceinline__ void lanes_xsa(float (&yv)[EPL], const float (&v)[EPL
 // Its backward from g = d loss / d z: g becomes d loss / d y = g - (g.u) u,
 // and dv = inv (du - u (u.du)) above the norm floor (inv du below it) with
 // du = -((y.u) g + (g.u) y).
-template <int EPL>
+template <int G, int EPL>
 __device__ __forceinline__ void lanes_xsa_backward(const float (&yv)[EPL], const float (&v)[EPL], float (&g)[EPL],
                                                    float (&dv)[EPL]) {
     float u[EPL];
-    const float sq = lanes_dot(v, v), inv = rsqrtf(fmaxf(sq, kXsaFloor));
+    const float sq = lanes_dot<G>(v, v), inv = rsqrtf(fmaxf(sq, kXsaFloor));
 #pragma unroll
     for (int e = 0; e < EPL; ++e) u[e] = v[e] * inv;
-    const float s = lanes_dot(yv, u), tg = lanes_dot(g, u);
+    const float s = lanes_dot<G>(yv, u), tg = lanes_dot<G>(g, u);
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
         dv[e] = -(s * g[e] + tg * yv[e]);
         g[e] = g[e] - tg * u[e];
     }
-    const float udu = sq >= kXsaFloor ? lanes_dot(u, dv) : 0.0f;
+    const float udu = sq >= kXsaFloor ? lanes_dot<G>(u, dv) : 0.0f;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) dv[e] = inv * (dv[e] - u[e] * udu);
 }
 
-// Causal attention of one (row, head) per wave, then (XSA) the exclusive
+// Causal attention of one (row, head) per group, then (XSA) the exclusive
 // projection against the row's own value: y and z = xsa(y) (or y) stored.
-template <int EPL, bool XSA>
+template <int EPL, int G, bool XSA>
 __global__ void __launch_bounds__(kThreads) attention_forward_wave(const float *__restrict__ q,
                                                                    const float *__restrict__ k,
                                                                    const float *__restrict__ v, float *__restrict__ y,
                                                                    float *__restrict__ z, float *__restrict__ lse,
                                                                    int rows, int sequence, int W, int H,
                                                                    float scale) {
-    const int t = row_wave(), lane = threadIdx.x & 63;
+    const int t = row_group<G>(), lane = threadIdx.x & (G - 1);
     if (t >= rows * H) return;
     const int r = t / H, h = t % H, hd = W / H, pos = r % sequence, first = r - pos;
     float qr[EPL], acc[EPL] = {};
     lanes_load(q + size_t(r) * W + h * hd, hd, lane, qr);
     float m = -INFINITY, l = 0.0f;
-    for (int j = 0; j <= pos; ++j) {
-        float kr[EPL], vr[EPL];
-        lanes_load(k + size_t(first + j) * W + h * hd, hd, lane, kr);
-        lanes_load(v + size_t(first + j) * W + h * hd, hd, lane, vr);
-        const float s = lanes_dot(qr, kr) * scale;
-        const float mn = fmaxf(m, s), alpha = expf(m - mn), p = expf(s - mn);
-        l = l * alpha + p;
+    constexpr int U = kBatch<EPL>;
+    for (int j0 = 0; j0 <= pos; j0 += U) {
+        float kr[U][EPL], vr[U][EPL], sc[U];
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) acc[e] = fmaf(p, vr[e], acc[e] * alpha);
-        m = mn;
+        for (int u = 0; u < U; ++u) {
+            const size_t o = size_t(first + min(j0 + u, pos)) * W + h * hd;
+            lanes_load(k + o, hd, lane, kr[u]);
+            lanes_load(v + o, hd, lane, vr[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) sc[u] = lanes_dot<G>(qr, kr[u]) * scale;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (j0 + u > pos) break;
+            const float mn = fmaxf(m, sc[u]), alpha = expf(m - mn), p = expf(sc[u] - mn);
+            l = l * alpha + p;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) acc[e] = fmaf(p, vr[u][e], acc[e] * alpha);
+            m = mn;
+        }
     }
     const float il = 1.0f / l;
 #pragma unroll
@@ -769,7 +792,7 @@ __global__ void __launch_bounds__(kThreads) attention_forward_wave(const float *
     if (XSA) {
         float vs[EPL];
         lanes_load(v + o, hd, lane, vs);
-        lanes_xsa(acc, vs);
+        lanes_xsa<G>(acc, vs);
     }
     lanes_store(z + o, hd, lane, acc);
 }
@@ -777,7 +800,7 @@ __global__ void __launch_bounds__(kThreads) attention_forward_wave(const float *
 // From dz = d loss / d z: (XSA) its backward first, storing dy and the XSA's
 // part of dv; without XSA dy is dz and dv starts at zero.  Then dq and the
 // row's dy . y (dsum), which the key-side kernel needs.
-template <int EPL, bool XSA>
+template <int EPL, int G, bool XSA>
 __global__ void __launch_bounds__(kThreads) attention_dq_wave(const float *__restrict__ q, const float *__restrict__ k,
                                                               const float *__restrict__ v, const float *__restrict__ y,
                                                               const float *__restrict__ lse,
@@ -785,7 +808,7 @@ __global__ void __launch_bounds__(kThreads) attention_dq_wave(const float *__res
                                                               float *__restrict__ dv, float *__restrict__ dq,
                                                               float *__restrict__ dsum, int rows, int sequence, int W,
                                                               int H, float scale) {
-    const int t = row_wave(), lane = threadIdx.x & 63;
+    const int t = row_group<G>(), lane = threadIdx.x & (G - 1);
     if (t >= rows * H) return;
     const int r = t / H, h = t % H, hd = W / H, pos = r % sequence, first = r - pos;
     const size_t o = size_t(r) * W + h * hd;
@@ -797,18 +820,28 @@ __global__ void __launch_bounds__(kThreads) attention_dq_wave(const float *__res
     if (XSA) {
         float vs[EPL];
         lanes_load(v + o, hd, lane, vs);
-        lanes_xsa_backward(yv, vs, g, dvs);
+        lanes_xsa_backward<G>(yv, vs, g, dvs);
         lanes_store(dy + o, hd, lane, g);
     }
     lanes_store(dv + o, hd, lane, dvs);
-    const float D = lanes_dot(g, yv), L = lse[t];
-    for (int j = 0; j <= pos; ++j) {
-        float kr[EPL], vr[EPL];
-        lanes_load(k + size_t(first + j) * W + h * hd, hd, lane, kr);
-        lanes_load(v + size_t(first + j) * W + h * hd, hd, lane, vr);
-        const float ds = expf(lanes_dot(qr, kr) * scale - L) * (lanes_dot(g, vr) - D);
+    const float D = lanes_dot<G>(g, yv), L = lse[t];
+    constexpr int U = kBatch<EPL>;
+    for (int j0 = 0; j0 <= pos; j0 += U) {
+        float kr[U][EPL], vr[U][EPL], ds[U];
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) acc[e] = fmaf(ds, kr[e], acc[e]);
+        for (int u = 0; u < U; ++u) {
+            const size_t at = size_t(first + min(j0 + u, pos)) * W + h * hd;
+            lanes_load(k + at, hd, lane, kr[u]);
+            lanes_load(v + at, hd, lane, vr[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) ds[u] = expf(lanes_dot<G>(qr, kr[u]) * scale - L) * (lanes_dot<G>(g, vr[u]) - D);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (j0 + u > pos) break;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) acc[e] = fmaf(ds[u], kr[u][e], acc[e]);
+        }
     }
 #pragma unroll
     for (int e = 0; e < EPL; ++e) acc[e] *= scale;
@@ -816,7 +849,7 @@ __global__ void __launch_bounds__(kThreads) attention_dq_wave(const float *__res
     if (lane == 0) dsum[t] = D;
 }
 
-template <int EPL>
+template <int EPL, int G>
 __global__ void __launch_bounds__(kThreads) attention_dkv_wave(const float *__restrict__ q,
                                                                const float *__restrict__ k,
                                                                const float *__restrict__ v,
@@ -825,23 +858,37 @@ __global__ void __launch_bounds__(kThreads) attention_dkv_wave(const float *__re
                                                                const float *__restrict__ dsum, float *__restrict__ dk,
                                                                float *dv, int rows, int sequence, int W, int H,
                                                                float scale) {
-    const int t = row_wave(), lane = threadIdx.x & 63;
+    const int t = row_group<G>(), lane = threadIdx.x & (G - 1);
     if (t >= rows * H) return;
     const int j = t / H, h = t % H, hd = W / H, pos = j % sequence, last = j - pos + sequence;
     const size_t o = size_t(j) * W + h * hd;
     float kr[EPL], vr[EPL], ak[EPL] = {}, av[EPL] = {};
     lanes_load(k + o, hd, lane, kr);
     lanes_load(v + o, hd, lane, vr);
-    for (int i = j; i < last; ++i) {
-        float qi[EPL], gi[EPL];
-        lanes_load(q + size_t(i) * W + h * hd, hd, lane, qi);
-        lanes_load(dy + size_t(i) * W + h * hd, hd, lane, gi);
-        const float p = expf(lanes_dot(qi, kr) * scale - lse[size_t(i) * H + h]);
-        const float ds = p * (lanes_dot(gi, vr) - dsum[size_t(i) * H + h]);
+    constexpr int U = kBatch<EPL>;
+    for (int i0 = j; i0 < last; i0 += U) {
+        float qi[U][EPL], gi[U][EPL], p[U], ds[U];
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) {
-            av[e] = fmaf(p, gi[e], av[e]);
-            ak[e] = fmaf(ds, qi[e], ak[e]);
+        for (int u = 0; u < U; ++u) {
+            const int i = min(i0 + u, last - 1);
+            lanes_load(q + size_t(i) * W + h * hd, hd, lane, qi[u]);
+            lanes_load(dy + size_t(i) * W + h * hd, hd, lane, gi[u]);
+            p[u] = lse[size_t(i) * H + h];
+            ds[u] = dsum[size_t(i) * H + h];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            p[u] = expf(lanes_dot<G>(qi[u], kr) * scale - p[u]);
+            ds[u] = p[u] * (lanes_dot<G>(gi[u], vr) - ds[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (i0 + u >= last) break;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) {
+                av[e] = fmaf(p[u], gi[u][e], av[e]);
+                ak[e] = fmaf(ds[u], qi[u][e], ak[e]);
+            }
         }
     }
     float old[EPL];
@@ -860,7 +907,7 @@ __global__ void __launch_bounds__(kThreads) attention_dkv_wave(const float *__re
 // blockIdx.y = 1 a key row each (dk and dv, as attention_dkv_wave), which
 // form each later query's XSA backward and dy . y themselves instead of
 // waiting for the query waves: the same arithmetic on the same operands.
-template <int EPL, bool XSA>
+template <int EPL, int G, bool XSA>
 __global__ void __launch_bounds__(kThreads) attention_backward_wave(const float *__restrict__ q,
                                                                     const float *__restrict__ k,
                                                                     const float *__restrict__ v,
@@ -870,7 +917,7 @@ __global__ void __launch_bounds__(kThreads) attention_backward_wave(const float 
                                                                     float *__restrict__ dq, float *__restrict__ dk,
                                                                     float *__restrict__ dv, int rows, int sequence,
                                                                     int W, int H, float scale) {
-    const int t = row_wave(), lane = threadIdx.x & 63;
+    const int t = row_group<G>(), lane = threadIdx.x & (G - 1);
     if (t >= rows * H) return;
     const int r = t / H, h = t % H, hd = W / H, pos = r % sequence, first = r - pos;
     // d loss / d y of row i (XSA's backward when on) and its dy . y.
@@ -884,22 +931,32 @@ __global__ void __launch_bounds__(kThreads) attention_backward_wave(const float 
         if (XSA) {
             float vs[EPL];
             lanes_load(v + oi, hd, lane, vs);
-            lanes_xsa_backward(yv, vs, g, dvs);
+            lanes_xsa_backward<G>(yv, vs, g, dvs);
         }
-        return lanes_dot(g, yv);
+        return lanes_dot<G>(g, yv);
     };
     const size_t o = size_t(r) * W + h * hd;
     if (blockIdx.y == 0) {
         float qr[EPL], g[EPL], dvs[EPL], acc[EPL] = {};
         lanes_load(q + o, hd, lane, qr);
         const float D = output_grad(r, g, dvs), L = lse[t];
-        for (int j = 0; j <= pos; ++j) {
-            float kr[EPL], vr[EPL];
-            lanes_load(k + size_t(first + j) * W + h * hd, hd, lane, kr);
-            lanes_load(v + size_t(first + j) * W + h * hd, hd, lane, vr);
-            const float ds = expf(lanes_dot(qr, kr) * scale - L) * (lanes_dot(g, vr) - D);
+        constexpr int U = kBatch<EPL>;
+        for (int j0 = 0; j0 <= pos; j0 += U) {
+            float kr[U][EPL], vr[U][EPL], ds[U];
 #pragma unroll
-            for (int e = 0; e < EPL; ++e) acc[e] = fmaf(ds, kr[e], acc[e]);
+            for (int u = 0; u < U; ++u) {
+                const size_t at = size_t(first + min(j0 + u, pos)) * W + h * hd;
+                lanes_load(k + at, hd, lane, kr[u]);
+                lanes_load(v + at, hd, lane, vr[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) ds[u] = expf(lanes_dot<G>(qr, kr[u]) * scale - L) * (lanes_dot<G>(g, vr[u]) - D);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (j0 + u > pos) break;
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) acc[e] = fmaf(ds[u], kr[u][e], acc[e]);
+            }
         }
 #pragma unroll
         for (int e = 0; e < EPL; ++e) acc[e] *= scale;
@@ -914,16 +971,30 @@ __global__ void __launch_bounds__(kThreads) attention_backward_wave(const float 
         float g[EPL];
         output_grad(r, g, own);  // this row's own XSA part of dv
     }
-    for (int i = r; i < last; ++i) {
-        float qi[EPL], gi[EPL], unused[EPL];
-        lanes_load(q + size_t(i) * W + h * hd, hd, lane, qi);
-        const float D = output_grad(i, gi, unused);
-        const float p = expf(lanes_dot(qi, kr) * scale - lse[size_t(i) * H + h]);
-        const float ds = p * (lanes_dot(gi, vr) - D);
+    constexpr int U = kBatch<EPL>;
+    for (int i0 = r; i0 < last; i0 += U) {
+        float qi[U][EPL], gi[U][EPL], p[U], ds[U];
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) {
-            av[e] = fmaf(p, gi[e], av[e]);
-            ak[e] = fmaf(ds, qi[e], ak[e]);
+        for (int u = 0; u < U; ++u) {
+            const int i = min(i0 + u, last - 1);
+            lanes_load(q + size_t(i) * W + h * hd, hd, lane, qi[u]);
+            p[u] = lse[size_t(i) * H + h];
+            float unused[EPL];
+            ds[u] = output_grad(i, gi[u], unused);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            p[u] = expf(lanes_dot<G>(qi[u], kr) * scale - p[u]);
+            ds[u] = p[u] * (lanes_dot<G>(gi[u], vr) - ds[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (i0 + u >= last) break;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) {
+                av[e] = fmaf(p[u], gi[u][e], av[e]);
+                ak[e] = fmaf(ds[u], qi[u][e], ak[e]);
+            }
         }
     }
 #pragma unroll
@@ -937,14 +1008,14 @@ __global__ void __launch_bounds__(kThreads) attention_backward_wave(const float 
 
 // What the matrix-core backward needs of one (row, head): dy (XSA's backward
 // of dz), the XSA's part of dv (zero without XSA) and D = dy . y.
-template <int EPL, bool XSA>
+template <int EPL, int G, bool XSA>
 __global__ void __launch_bounds__(kThreads) attention_output_grad_wave(const float *__restrict__ y,
                                                                        const float *__restrict__ v,
                                                                        const float *__restrict__ dz,
                                                                        float *__restrict__ dy, float *__restrict__ dv,
                                                                        float *__restrict__ dsum, int rows, int W,
                                                                        int H) {
-    const int t = row_wave(), lane = threadIdx.x & 63;
+    const int t = row_group<G>(), lane = threadIdx.x & (G - 1);
     if (t >= rows * H) return;
     const int hd = W / H;
     const size_t o = size_t(t / H) * W + (t % H) * hd;
@@ -954,26 +1025,35 @@ __global__ void __launch_bounds__(kThreads) attention_output_grad_wave(const flo
     if (XSA) {
         float vs[EPL];
         lanes_load(v + o, hd, lane, vs);
-        lanes_xsa_backward(yv, vs, g, d);
+        lanes_xsa_backward<G>(yv, vs, g, d);
         lanes_store(dy + o, hd, lane, g);
     }
     lanes_store(dv + o, hd, lane, d);
-    const float D = lanes_dot(g, yv);
+    const float D = lanes_dot<G>(g, yv);
     if (lane == 0) dsum[t] = D;
 }
 
+// f(registers a lane, lanes) of a (row, head)'s group.
 template <class F>
 void by_lanes(int hd, F &&f) {
-    if (hd <= 64)
-        f(std::integral_constant<int, 1>{});
+    auto call = [&](auto e, auto g) { f(e, g); };
+    using std::integral_constant;
+    if (hd <= 8)
+        call(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+    else if (hd <= 16)
+        call(integral_constant<int, 1>{}, integral_constant<int, 16>{});
+    else if (hd <= 32)
+        call(integral_constant<int, 1>{}, integral_constant<int, 32>{});
+    else if (hd <= 64)
+        call(integral_constant<int, 1>{}, integral_constant<int, 64>{});
     else if (hd <= 128)
-        f(std::integral_constant<int, 2>{});
+        call(integral_constant<int, 2>{}, integral_constant<int, 64>{});
     else if (hd <= 256)
-        f(std::integral_constant<int, 4>{});
+        call(integral_constant<int, 4>{}, integral_constant<int, 64>{});
     else if (hd <= 512)
-        f(std::integral_constant<int, 8>{});
+        call(integral_constant<int, 8>{}, integral_constant<int, 64>{});
     else
-        f(std::integral_constant<int, 16>{});
+        call(integral_constant<int, 16>{}, integral_constant<int, 64>{});
 }
 
 // Whether a shape takes the matrix-core attention kernels, which work on 16 x 16
@@ -1826,14 +1906,14 @@ void attention_forward(const float *q, const float *k, const float *v, float *y,
         matrix_attention_forward(q, k, v, y, z, lse, rows, sequence, W, H, xsa, stream);
         return;
     }
-    by_lanes(W / H, [&](auto e) {
-        constexpr int EPL = decltype(e)::value;
-        const dim3 grid(blocks_for(size_t(rows) * H * 64));
+    by_lanes(W / H, [&](auto e, auto lanes) {
+        constexpr int EPL = decltype(e)::value, G = decltype(lanes)::value;
+        const dim3 grid(blocks_for(size_t(rows) * H * G));
         if (xsa)
-            hipLaunchKernelGGL((attention_forward_wave<EPL, true>), grid, dim3(kThreads), 0, stream, q, k, v, y, z,
+            hipLaunchKernelGGL((attention_forward_wave<EPL, G, true>), grid, dim3(kThreads), 0, stream, q, k, v, y, z,
                                lse, rows, sequence, W, H, scale);
         else
-            hipLaunchKernelGGL((attention_forward_wave<EPL, false>), grid, dim3(kThreads), 0, stream, q, k, v, y, z,
+            hipLaunchKernelGGL((attention_forward_wave<EPL, G, false>), grid, dim3(kThreads), 0, stream, q, k, v, y, z,
                                lse, rows, sequence, W, H, scale);
     });
 }
@@ -1845,42 +1925,42 @@ void attention_backward(const float *q, const float *k, const float *v, const fl
     // Without XSA the attention's output gradient is dz itself.
     const float *g = xsa ? dy : dz;
     if (sequence <= kMergedBackwardMax) {
-        by_lanes(W / H, [&](auto e) {
-            constexpr int EPL = decltype(e)::value;
-            const dim3 grid(blocks_for(size_t(rows) * H * 64), 2);
+        by_lanes(W / H, [&](auto e, auto lanes) {
+            constexpr int EPL = decltype(e)::value, G = decltype(lanes)::value;
+            const dim3 grid(blocks_for(size_t(rows) * H * G), 2);
             if (xsa)
-                hipLaunchKernelGGL((attention_backward_wave<EPL, true>), grid, dim3(kThreads), 0, stream, q, k, v, y,
+                hipLaunchKernelGGL((attention_backward_wave<EPL, G, true>), grid, dim3(kThreads), 0, stream, q, k, v, y,
                                    lse, dz, dq, dk, dv, rows, sequence, W, H, scale);
             else
-                hipLaunchKernelGGL((attention_backward_wave<EPL, false>), grid, dim3(kThreads), 0, stream, q, k, v, y,
+                hipLaunchKernelGGL((attention_backward_wave<EPL, G, false>), grid, dim3(kThreads), 0, stream, q, k, v, y,
                                    lse, dz, dq, dk, dv, rows, sequence, W, H, scale);
         });
         return;
     }
     if (matrix_attention(sequence, W / H)) {
-        by_lanes(W / H, [&](auto e) {
-            constexpr int EPL = decltype(e)::value;
-            const dim3 grid(blocks_for(size_t(rows) * H * 64));
+        by_lanes(W / H, [&](auto e, auto lanes) {
+            constexpr int EPL = decltype(e)::value, G = decltype(lanes)::value;
+            const dim3 grid(blocks_for(size_t(rows) * H * G));
             if (xsa)
-                hipLaunchKernelGGL((attention_output_grad_wave<EPL, true>), grid, dim3(kThreads), 0, stream, y, v, dz,
+                hipLaunchKernelGGL((attention_output_grad_wave<EPL, G, true>), grid, dim3(kThreads), 0, stream, y, v, dz,
                                    dy, dv, dsum, rows, W, H);
             else
-                hipLaunchKernelGGL((attention_output_grad_wave<EPL, false>), grid, dim3(kThreads), 0, stream, y, v,
+                hipLaunchKernelGGL((attention_output_grad_wave<EPL, G, false>), grid, dim3(kThreads), 0, stream, y, v,
                                    dz, dy, dv, dsum, rows, W, H);
         });
         matrix_attention_backward(q, k, v, lse, g, dsum, dq, dk, dv, rows, sequence, W, H, stream);
         return;
     }
-    by_lanes(W / H, [&](auto e) {
-        constexpr int EPL = decltype(e)::value;
-        const dim3 grid(blocks_for(size_t(rows) * H * 64));
+    by_lanes(W / H, [&](auto e, auto lanes) {
+        constexpr int EPL = decltype(e)::value, G = decltype(lanes)::value;
+        const dim3 grid(blocks_for(size_t(rows) * H * G));
         if (xsa)
-            hipLaunchKernelGGL((attention_dq_wave<EPL, true>), grid, dim3(kThreads), 0, stream, q, k, v, y, lse, dz,
+            hipLaunchKernelGGL((attention_dq_wave<EPL, G, true>), grid, dim3(kThreads), 0, stream, q, k, v, y, lse, dz,
                                dy, dv, dq, dsum, rows, sequence, W, H, scale);
         else
-            hipLaunchKernelGGL((attention_dq_wave<EPL, false>), grid, dim3(kThreads), 0, stream, q, k, v, y, lse, dz,
+            hipLaunchKernelGGL((attention_dq_wave<EPL, G, false>), grid, dim3(kThreads), 0, stream, q, k, v, y, lse, dz,
                                dy, dv, dq, dsum, rows, sequence, W, H, scale);
-        hipLaunchKernelGGL(attention_dkv_wave<EPL>, grid, dim3(kThreads), 0, stream, q, k, v, lse, g, dsum, dk, dv,
+        hipLaunchKernelGGL((attention_dkv_wave<EPL, G>), grid, dim3(kThreads), 0, stream, q, k, v, lse, g, dsum, dk, dv,
                            rows, sequence, W, H, scale);
     });
 }
@@ -1893,9 +1973,10 @@ void qk_forward(int count, const float *const *pre, float *const *out, float *co
         set.out[i] = out[i];
         set.inv[i] = inv[i];
     }
-    by_lanes(W / H, [&](auto e) {
-        hipLaunchKernelGGL(qk_forward_kernel<decltype(e)::value>,
-                           dim3(blocks_for(size_t(rows) * H * 64), unsigned(count)), dim3(kThreads), 0, stream, set,
+    by_lanes(W / H, [&](auto e, auto lanes) {
+        constexpr int EPL = decltype(e)::value, G = decltype(lanes)::value;
+        hipLaunchKernelGGL((qk_forward_kernel<EPL, G>),
+                           dim3(blocks_for(size_t(rows) * H * G), unsigned(count)), dim3(kThreads), 0, stream, set,
                            table, rows, sequence, W, H, int(norm), int(rotate));
     });
 }
@@ -1908,9 +1989,10 @@ void qk_backward(int count, float *const *g, const float *const *pre, const floa
         set.out[i] = g[i];
         set.inv[i] = const_cast<float *>(inv[i]);  // read only in the backward
     }
-    by_lanes(W / H, [&](auto e) {
-        hipLaunchKernelGGL(qk_backward_kernel<decltype(e)::value>,
-                           dim3(blocks_for(size_t(rows) * H * 64), unsigned(count)), dim3(kThreads), 0, stream, set,
+    by_lanes(W / H, [&](auto e, auto lanes) {
+        constexpr int EPL = decltype(e)::value, G = decltype(lanes)::value;
+        hipLaunchKernelGGL((qk_backward_kernel<EPL, G>),
+                           dim3(blocks_for(size_t(rows) * H * G), unsigned(count)), dim3(kThreads), 0, stream, set,
                            table, rows, sequence, W, H, int(norm), int(rotate));
     });
 }
