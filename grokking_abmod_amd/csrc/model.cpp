@@ -127,12 +127,14 @@ struct MeshGpt::Impl {
     // Prefill / logits workspace, grown on demand.
     DevBuf wx, wxn, wq, wy, wtok, wlogits, wk, wv;
     // Transfers: pinned staging of uploads and downloads (a model's own, fixed
-    // in size), contiguous tokens on the device, and the finiteness flag.
-    static constexpr size_t kUpload = size_t(1) << 20, kChunk = size_t(512) << 10, kChunks = 4, kWords = 256;
-    PinnedBuf hup, hdown;
-    DevBuf dstage, dbad;
+    // in size) and contiguous tokens on the device.  A chunk costs some 14 us
+    // of submission and waiting: 3.7 MB of logits take 450 us in all with
+    // chunks of 256 KiB, 347 with 512, 325 with 1 MiB, 343 with 2 MiB.
+    static constexpr size_t kUpload = size_t(1) << 20, kChunk = size_t(1) << 20, kChunks = 2, kWords = 256;
+    PinnedBuf hio;  // the upload, then the download chunks, then single words
+    DevBuf dstage;
     hipEvent_t chunk_ev[kChunks] = {};
-    bool upload_busy = false;    // hup may still be read by the stream
+    bool upload_busy = false;    // hio's upload may still be read by the stream
     int known_flags = -1;        // dflags' value when the host has it
     DevBuf wlast;   // the last block's rows of a prefill (run_blocks)
     DevBuf wsplit;  // keys and values of one layer as attn_split's planes
@@ -158,6 +160,7 @@ struct MeshGpt::Impl {
     bool use_split_prefill = true;
     bool use_short_prefill = true;
     bool use_window = true;
+    bool use_chain = true;
 
     // Training (gpu.rs:1915-2003): the activations of the last forward, the
     // gradient, AdamW's moments and the running powers of its betas (reset
@@ -297,9 +300,7 @@ struct MeshGpt::Impl {
         check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
         for (hipEvent_t &e : call_ev) check(hipEventCreate(&e), "hipEventCreate");
         for (hipEvent_t &e : chunk_ev) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
-        hup.ensure(kUpload);
-        hdown.ensure(kChunk * kChunks + kWords);
-        dbad.ensure(4);
+        hio.ensure(kUpload + kChunk * kChunks + kWords);
         use_graph = env_int("MG_DISABLE_GRAPH", 0) == 0;
 
         const size_t W = cfg.width, hd = cfg.head_width();
@@ -328,6 +329,7 @@ struct MeshGpt::Impl {
         use_split_prefill = env_int("MG_DISABLE_SPLIT_PREFILL", 0) == 0;
         use_rows_prefill = env_int("MG_DISABLE_ROWS_PREFILL", 0) == 0;
         use_window = env_int("MG_DISABLE_WINDOW", 0) == 0;
+        use_chain = env_int("MG_DISABLE_TRAIN_CHAIN", 0) == 0;
         use_short_prefill = env_int("MG_DISABLE_SHORT_PREFILL", 0) == 0;
 
         const size_t C = cfg.context;
@@ -422,8 +424,8 @@ struct MeshGpt::Impl {
     void upload(void *dst, const void *src, size_t bytes, const char *what) {
         if (bytes <= kUpload) {
             if (upload_busy) sync();
-            std::memcpy(hup.p, src, bytes);
-            check(hipMemcpyAsync(dst, hup.p, bytes, hipMemcpyHostToDevice, stream), what);
+            std::memcpy(hio.p, src, bytes);
+            check(hipMemcpyAsync(dst, hio.p, bytes, hipMemcpyHostToDevice, stream), what);
             upload_busy = true;
         } else {
             check(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream), what);
@@ -433,7 +435,8 @@ struct MeshGpt::Impl {
 
     // A word of host memory that the stream may write; valid until the next
     // sync() has passed and another call of the same slot.
-    int *word(int slot) const { return reinterpret_cast<int *>(hdown.as<char>() + kChunk * kChunks) + slot; }
+    int *word(int slot) const { return reinterpret_cast<int *>(hio.as<char>() + kUpload + kChunk * kChunks) + slot; }
+    char *chunk(size_t i) const { return hio.as<char>() + kUpload + i % kChunks * kChunk; }
     enum { kFlagsWord = 0, kBadWord = 1, kStatusWord = 2 };
 
     // out[0..bytes) = src once the stream has reached this point: pinned chunks,
@@ -445,7 +448,7 @@ struct MeshGpt::Impl {
         const size_t chunks = (bytes + kChunk - 1) / kChunk;
         auto size = [&](size_t i) { return std::min(kChunk, bytes - i * kChunk); };
         auto issue = [&](size_t i) {
-            check(hipMemcpyAsync(hdown.as<char>() + i % kChunks * kChunk, static_cast<const char *>(src) + i * kChunk,
+            check(hipMemcpyAsync(chunk(i), static_cast<const char *>(src) + i * kChunk,
                                  size(i), hipMemcpyDeviceToHost, stream),
                   what);
             if (chunks > 1) check(hipEventRecord(chunk_ev[i % kChunks], stream), "hipEventRecord");
@@ -467,7 +470,7 @@ struct MeshGpt::Impl {
                     }
                 }
             }
-            std::memcpy(static_cast<char *>(out) + i * kChunk, hdown.as<char>() + i % kChunks * kChunk, size(i));
+            std::memcpy(static_cast<char *>(out) + i * kChunk, chunk(i), size(i));
             if (i + kChunks < chunks) issue(i + kChunks);
         }
         if (chunks > 1) sync();
@@ -483,12 +486,12 @@ struct MeshGpt::Impl {
         if (n <= kHostCheck) {
             download(out, src, n * 4, "download", [&] {
                 ready();
-                validate_finite(hdown.as<float>(), n, name);
+                validate_finite(reinterpret_cast<float *>(chunk(0)), n, name);
             });
             return;
         }
-        kern::nonfinite(src, n, dbad.as<int>(), stream);
-        check(hipMemcpyAsync(word(kBadWord), dbad.p, 4, hipMemcpyDeviceToHost, stream), "download check");
+        kern::nonfinite(src, n, dflags.as<int>() + 1, stream);
+        check(hipMemcpyAsync(word(kBadWord), dflags.as<int>() + 1, 4, hipMemcpyDeviceToHost, stream), "download check");
         download(out, src, n * 4, "download", [&] {
             ready();
             if (*word(kBadWord)) throw Error(std::string(name) + " must contain only finite values", kNonfinite);
@@ -528,7 +531,7 @@ struct MeshGpt::Impl {
             drng_start.ensure(batch_cap * 8);
             drng_next.ensure(batch_cap * 8);
             dlogits.ensure(batch_cap * cfg.vocab_size * 4);
-            dflags.ensure(4);
+            dflags.ensure(8);  // non-finite logits of the decode, of a downloaded result
             if (persistent_ok) {
                 pxch.ensure(batch_cap * kern::persistent_exchange_words(shape) * 8);
                 pabort.ensure(8);  // abort flag, then the launch's non-finite flag
@@ -954,35 +957,85 @@ struct MeshGpt::Impl {
             T::geometry_forward(Eraw, codes.as<float>(), at(p.eg), at(p.er), V, W, radius, normalize, preserve, stream);
             Ev = at(p.eg);
         }
-        T::gather(Ev, tok, at(p.x), R, W, stream);
         auto X = [&](int b) { return at(p.x) + size_t(b) * RW; };
         auto last = [&](size_t o, int depth) { return at(o) + size_t(depth - 1) * RW; };
-        for (int b = 0; b < L; ++b) {
+        const bool chain = use_chain && T::chain_fits(ma, mf, H);
+        auto attend = [&](int b) {
             const TrainBlock &k = p.blocks[b];
-            const Block &g = layout.blocks[b];
-            // n1 = rmsnorm(x_b), x_b = xm + ffn of the block below (its residual
-            // add and this norm are formed in front of the meshes), then Q, K
-            // and V of n1 in one launch, then QK-Norm and RoPE of q and k in
-            // one (reference.rs:174-193, each when switched on).
-            const float *qkv_w[3] = {w + group(g.query), w + group(g.key), w + group(g.value)};
-            float *qkv[3] = {at(k.qs), at(k.ks), at(k.vs)};
-            const T::NormIn n1 = b == 0 ? T::NormIn{X(0), nullptr, nullptr, at(k.n1), at(k.inv1)}
-                                        : T::NormIn{at(p.blocks[b - 1].xm), last(p.blocks[b - 1].fs, F), X(b),
-                                                    at(k.n1), at(k.inv1)};
-            const T::QkOut qk{{at(k.qr), at(k.kr)}, {at(k.qinv), at(k.kinv)}, table, seq, H, cfg.qk_norm, cfg.rope};
-            T::norm_mesh_forward_qkv(ma, n1, qkv, qkv_w, qk, R, stream);
             T::attention_forward(at(k.qr), at(k.kr), last(k.vs, A), at(k.y), at(k.z), at(k.lse), R, seq, W, H,
                                  cfg.xsa, stream);
-            T::mesh_forward(ma, at(k.z), at(k.ps), w + group(g.projection), R, stream);
-            // xm = x_b + proj and n2 = rmsnorm(xm), formed in front of the FFN mesh.
-            float *fs = at(k.fs);
-            const float *wf = w + group(g.ffn);
-            T::norm_mesh_forward_set(mf, 1, T::NormIn{X(b), last(k.ps, A), at(k.xm), at(k.n2), at(k.inv2)}, &fs, &wf,
-                                     R, stream);
+        };
+        if (chain) {
+            // A launch before, between and after the attentions.
+            for (int b = 0; b <= L; ++b) {
+                T::ForwardChain c{};
+                c.rows = R;
+                c.ma = ma;
+                c.mf = mf;
+                c.x_out = X(b);
+                if (b == 0) {
+                    c.E = Ev;
+                    c.tokens = tok;
+                } else {
+                    const TrainBlock &k = p.blocks[b - 1];
+                    const Block &g = layout.blocks[b - 1];
+                    c.z = at(k.z);
+                    c.x_in = X(b - 1);
+                    c.wproj = w + group(g.projection);
+                    c.wffn = w + group(g.ffn);
+                    c.ps = at(k.ps);
+                    c.xm = at(k.xm);
+                    c.n2 = at(k.n2);
+                    c.inv2 = at(k.inv2);
+                    c.fs = at(k.fs);
+                }
+                if (b < L) {
+                    const TrainBlock &k = p.blocks[b];
+                    const Block &g = layout.blocks[b];
+                    c.n = at(k.n1);
+                    c.inv = at(k.inv1);
+                    const size_t id[3] = {g.query, g.key, g.value};
+                    float *stacks[3] = {at(k.qs), at(k.ks), at(k.vs)};
+                    for (int y = 0; y < 3; ++y) {
+                        c.wqkv[y] = w + group(id[y]);
+                        c.qkv[y] = stacks[y];
+                    }
+                    c.qk = T::QkOut{{at(k.qr), at(k.kr)}, {at(k.qinv), at(k.kinv)}, table, seq, H, cfg.qk_norm, cfg.rope};
+                } else {
+                    c.n = at(p.nf);
+                    c.inv = at(p.invf);
+                }
+                T::forward_chain(c, stream);
+                if (b < L) attend(b);
+            }
+        } else {
+            T::gather(Ev, tok, at(p.x), R, W, stream);
+            for (int b = 0; b < L; ++b) {
+                const TrainBlock &k = p.blocks[b];
+                const Block &g = layout.blocks[b];
+                // n1 = rmsnorm(x_b), x_b = xm + ffn of the block below (its residual
+                // add and this norm are formed in front of the meshes), then Q, K
+                // and V of n1 in one launch, then QK-Norm and RoPE of q and k in
+                // one (reference.rs:174-193, each when switched on).
+                const float *qkv_w[3] = {w + group(g.query), w + group(g.key), w + group(g.value)};
+                float *qkv[3] = {at(k.qs), at(k.ks), at(k.vs)};
+                const T::NormIn n1 = b == 0 ? T::NormIn{X(0), nullptr, nullptr, at(k.n1), at(k.inv1)}
+                                            : T::NormIn{at(p.blocks[b - 1].xm), last(p.blocks[b - 1].fs, F), X(b),
+                                                        at(k.n1), at(k.inv1)};
+                const T::QkOut qk{{at(k.qr), at(k.kr)}, {at(k.qinv), at(k.kinv)}, table, seq, H, cfg.qk_norm, cfg.rope};
+                T::norm_mesh_forward_qkv(ma, n1, qkv, qkv_w, qk, R, stream);
+                attend(b);
+                T::mesh_forward(ma, at(k.z), at(k.ps), w + group(g.projection), R, stream);
+                // xm = x_b + proj and n2 = rmsnorm(xm), formed in front of the FFN mesh.
+                float *fs = at(k.fs);
+                const float *wf = w + group(g.ffn);
+                T::norm_mesh_forward_set(mf, 1, T::NormIn{X(b), last(k.ps, A), at(k.xm), at(k.n2), at(k.inv2)}, &fs, &wf,
+                                         R, stream);
+            }
+            // x_L = xm + ffn of the top block, and the final norm.
+            T::add_rmsnorm_forward(at(p.blocks[L - 1].xm), last(p.blocks[L - 1].fs, F), X(L), at(p.nf), at(p.invf), R, W,
+                                   stream);
         }
-        // x_L = xm + ffn of the top block, and the final norm.
-        T::add_rmsnorm_forward(at(p.blocks[L - 1].xm), last(p.blocks[L - 1].fs, F), X(L), at(p.nf), at(p.invf), R, W,
-                               stream);
         T::head_logits(at(p.nf), Ev, at(p.logits), R, W, V, stream);
         T::cross_entropy(at(p.logits), tgt, at(p.dlogits), at(p.loss), R, V, sc, stream);
         if (!backward) return;
@@ -1006,33 +1059,94 @@ struct MeshGpt::Impl {
                                  &gp, rows, stream, &reductions);
         };
         T::head_backward(at(p.dlogits), Ev, dn, R, W, V, stream);
-        T::rmsnorm_backward(X(L), at(p.invf), dn, dx, false, R, W, 1, stream);
-        for (int b = L - 1; b >= 0; --b) {
+        auto attend_back = [&](int b) {
             const TrainBlock &k = p.blocks[b];
-            const Block &g = layout.blocks[b];
-            // x_{b+1} = xm + ffn(rmsnorm(xm)); xm = x_b + proj(attention)
-            T::mesh_backward_norm(mf, at(k.n2), at(k.fs), dx, T::NormGrad{at(k.xm), at(k.inv2), dx}, dn,
-                                  w + group(g.ffn), region(T::mesh_partial_floats(mf, R)), grad + group(g.ffn), R,
-                                  stream, &reductions);
-            mesh_backward(ma, at(k.z), at(k.ps), dx, dt, group(g.projection), R);
             T::attention_backward(at(k.qr), at(k.kr), last(k.vs, A), at(k.y), at(k.lse), dt, dy, dq, dk, dv,
                                   at(p.dsum), R, seq, W, H, cfg.xsa, stream);
-            if (cfg.rope || cfg.qk_norm) {
-                float *qk_g[2] = {dq, dk};
-                const float *qk_pre[2] = {last(k.qs, A), last(k.ks, A)}, *qk_inv[2] = {at(k.qinv), at(k.kinv)};
-                T::qk_backward(2, qk_g, qk_pre, qk_inv, table, R, seq, W, H, cfg.qk_norm, cfg.rope, stream);
+        };
+        if (chain) {
+            for (int b = L; b >= 0; --b) {
+                T::BackwardChain c{};
+                float *out[5] = {};
+                c.rows = R;
+                c.ma = ma;
+                c.mf = mf;
+                c.dx = dx;
+                if (b == L) {
+                    c.dn = dn;
+                    c.x_last = X(L);
+                    c.inv_last = at(p.invf);
+                } else {
+                    const TrainBlock &k = p.blocks[b];
+                    const Block &g = layout.blocks[b];
+                    const size_t id[3] = {g.query, g.key, g.value};
+                    const float *stacks[3] = {at(k.qs), at(k.ks), at(k.vs)}, *dout[3] = {dq, dk, dv};
+                    for (int y = 0; y < 3; ++y) {
+                        c.dqkv[y] = dout[y];
+                        c.wqkv[y] = w + group(id[y]);
+                        c.qkv[y] = stacks[y];
+                        c.part_qkv[y] = region(T::mesh_partial_floats(ma, R));
+                        out[y] = grad + group(id[y]);
+                    }
+                    c.qk_inv[0] = at(k.qinv);
+                    c.qk_inv[1] = at(k.kinv);
+                    c.n1 = at(k.n1);
+                    c.x_below = X(b);
+                    c.inv1 = at(k.inv1);
+                    c.table = table;
+                    c.sequence = seq;
+                    c.H = H;
+                    c.norm = cfg.qk_norm;
+                    c.rotate = cfg.rope;
+                }
+                if (b > 0) {
+                    const TrainBlock &k = p.blocks[b - 1];
+                    const Block &g = layout.blocks[b - 1];
+                    c.wffn = w + group(g.ffn);
+                    c.wproj = w + group(g.projection);
+                    c.n2 = at(k.n2);
+                    c.fs = at(k.fs);
+                    c.xm = at(k.xm);
+                    c.inv2 = at(k.inv2);
+                    c.z = at(k.z);
+                    c.ps = at(k.ps);
+                    c.dt = dt;
+                    c.part_ffn = region(T::mesh_partial_floats(mf, R));
+                    c.part_proj = region(T::mesh_partial_floats(ma, R));
+                    out[3] = grad + group(g.ffn);
+                    out[4] = grad + group(g.projection);
+                }
+                T::backward_chain(c, &reductions, out, stream);
+                if (b > 0) attend_back(b - 1);
             }
-            // The Q, K and V meshes' backward in one launch, each into its own
-            // rows; the norm's backward adds them (in that order).
-            const float *n1 = at(k.n1);
-            const float *qkv_in[3] = {n1, n1, n1}, *qkv[3] = {at(k.qs), at(k.ks), at(k.vs)};
-            const float *qkv_dout[3] = {dq, dk, dv};
-            const float *qkv_w[3] = {w + group(g.query), w + group(g.key), w + group(g.value)};
-            float *qkv_din[3] = {dn, at(p.dnk), at(p.dnv)};
-            float *qkv_grad[3] = {grad + group(g.query), grad + group(g.key), grad + group(g.value)};
-            T::mesh_backward_set(ma, 3, qkv_in, qkv, qkv_dout, qkv_din, false, qkv_w,
-                                 region(3 * T::mesh_partial_floats(ma, R)), qkv_grad, R, stream, &reductions);
-            T::rmsnorm_backward_sum3(X(b), at(k.inv1), dn, at(p.dnk), at(p.dnv), dx, true, R, W, stream);
+        } else {
+            T::rmsnorm_backward(X(L), at(p.invf), dn, dx, false, R, W, 1, stream);
+            for (int b = L - 1; b >= 0; --b) {
+                const TrainBlock &k = p.blocks[b];
+                const Block &g = layout.blocks[b];
+                // x_{b+1} = xm + ffn(rmsnorm(xm)); xm = x_b + proj(attention)
+                T::mesh_backward_norm(mf, at(k.n2), at(k.fs), dx, T::NormGrad{at(k.xm), at(k.inv2), dx}, dn,
+                                      w + group(g.ffn), region(T::mesh_partial_floats(mf, R)), grad + group(g.ffn), R,
+                                      stream, &reductions);
+                mesh_backward(ma, at(k.z), at(k.ps), dx, dt, group(g.projection), R);
+                attend_back(b);
+                if (cfg.rope || cfg.qk_norm) {
+                    float *qk_g[2] = {dq, dk};
+                    const float *qk_pre[2] = {last(k.qs, A), last(k.ks, A)}, *qk_inv[2] = {at(k.qinv), at(k.kinv)};
+                    T::qk_backward(2, qk_g, qk_pre, qk_inv, table, R, seq, W, H, cfg.qk_norm, cfg.rope, stream);
+                }
+                // The Q, K and V meshes' backward in one launch, each into its own
+                // rows; the norm's backward adds them (in that order).
+                const float *n1 = at(k.n1);
+                const float *qkv_in[3] = {n1, n1, n1}, *qkv[3] = {at(k.qs), at(k.ks), at(k.vs)};
+                const float *qkv_dout[3] = {dq, dk, dv};
+                const float *qkv_w[3] = {w + group(g.query), w + group(g.key), w + group(g.value)};
+                float *qkv_din[3] = {dn, at(p.dnk), at(p.dnv)};
+                float *qkv_grad[3] = {grad + group(g.query), grad + group(g.key), grad + group(g.value)};
+                T::mesh_backward_set(ma, 3, qkv_in, qkv, qkv_dout, qkv_din, false, qkv_w,
+                                     region(3 * T::mesh_partial_floats(ma, R)), qkv_grad, R, stream, &reductions);
+                T::rmsnorm_backward_sum3(X(b), at(k.inv1), dn, at(p.dnk), at(p.dnv), dx, true, R, W, stream);
+            }
         }
         // The tied vectors collect the head's gradient and the gathered rows'.
         T::embedding_gradient(at(p.dlogits), at(p.nf), tok, dx, at(p.dE), region(T::embedding_partial_floats(R, W, V)),
@@ -1057,7 +1171,7 @@ struct MeshGpt::Impl {
     size_t allocated_device_bytes() const {
         size_t total = 0;
         for (const DevBuf *b : {&params, &codes, &E, &Et, &rope, &wdec, &Edec, &q0, &kc, &vc, &dx, &dx2, &dxn, &dq,
-                                &part, &dtokens, &dlen, &drng, &dlogits, &dflags, &drng_start, &drng_next, &dstage, &dbad, &pxch, &pabort, &wx,
+                                &part, &dtokens, &dlen, &drng, &dlogits, &dflags, &drng_start, &drng_next, &dstage, &pxch, &pabort, &wx,
                                 &wxn, &wq, &wy, &wtok, &wlogits, &wk, &wv, &wsplit, &wlast, &tact, &tgrad, &tm, &tv, &tpart, &tin})
             total += b->bytes;
         return total;
@@ -1729,7 +1843,7 @@ bool sample_logits(int device, const float *logits, size_t rows, size_t vocab, f
     drng.ensure(rows * 8);
     dtok.ensure(rows * 4);
     dlen.ensure(rows * 4);
-    dflags.ensure(4);
+    dflags.ensure(8);  // non-finite logits of the decode, of a downloaded result
     check(hipMemcpy(dl.p, logits, rows * vocab * 4, hipMemcpyHostToDevice), "upload logits");
     check(hipMemcpy(drng.p, rng_states, rows * 8, hipMemcpyHostToDevice), "upload rng");
     check(hipMemset(dlen.p, 0, rows * 4), "clear lengths");

@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "dpp.hpp"
+#include "mesh_wave.hpp"
 #include "train.hpp"
 
 namespace meshgpt::kern::train {
@@ -46,18 +47,7 @@ struct QkSet {
     float *inv[kMaxSet];
 };
 
-constexpr float kRmsEps = 1e-5f;                                         // src/gpt/mod.rs:38
 constexpr float kXsaFloor = float(double(1e-12f) * double(1e-12f));      // XSA_EPSILON^2
-constexpr int kThreads = 256;
-
-__device__ __forceinline__ float elu(float z) { return z >= 0.0f ? z : expm1f(z); }
-
-__device__ __forceinline__ int stride_of(const Mesh &m, int l) {
-    return m.butterfly ? 1 << ((m.layer0 + l) % m.log2w) : 1;
-}
-
-// Whether layer l of a launch applies the ELU (every layer but the stack's last).
-__device__ __forceinline__ bool elu_layer(const Mesh &m, int l) { return l + 1 < m.depth || !m.linear_top; }
 
 int block_for(int W) { return std::max(64, (W + 63) / 64 * 64); }
 
@@ -208,61 +198,6 @@ int mesh_groups(const Mesh &m, int rows) {
 
 // ---- mesh stacks of width <= 64 or 128: one wave per row, channel
 // lane + 64 j in register j, partners by lane shuffles (no barriers).
-
-// Lane l gets v of lane (l + 1) mod 64 (DPP wave_rol:1) or of lane (l - 1)
-// mod 64 (DPP wave_ror:1): no LDS round trip.
-__device__ __forceinline__ float lanes_rol1(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x134, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float lanes_ror1(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x13C, 0xf, 0xf, false));
-}
-
-// out[j] = the value of channel (lane + 64 j + d) mod W, for 0 <= d < W.
-// Width 128 (CPL 2): a shift by 64 + d' renames the registers and shifts by
-// d'; for d' < 64 every lane reads lane (lane + d') mod 64, whose lanes below
-// d' offer their other register (their readers wrapped past lane 63), one lane
-// read per register, a DPP rotation for d' = 1 or 63 (the neighbour mesh and
-// its backward).
-template <int CPL>
-__device__ __forceinline__ void channel_shift(const float (&x)[CPL], int d, int W, int lane, float (&out)[CPL]) {
-    static_assert(CPL == 1 || CPL == 2, "wave mesh kernels take widths up to 128");
-    if constexpr (CPL == 1) {
-        if (W == 64 && d == 1) {
-            out[0] = lanes_rol1(x[0]);
-        } else if (W == 64 && d == 63) {
-            out[0] = lanes_ror1(x[0]);
-        } else {
-            int src = lane + d;
-            if (src >= W) src -= W;
-            out[0] = __shfl(x[0], src & 63, 64);
-        }
-    } else {
-        const bool swap = d >= 64;
-        const float y0 = swap ? x[1] : x[0], y1 = swap ? x[0] : x[1];
-        d &= 63;
-        if (d == 0) {
-            out[0] = y0;
-            out[1] = y1;
-            return;
-        }
-        const bool next = lane < d;
-        const float o0 = next ? y1 : y0, o1 = next ? y0 : y1;
-        if (d == 1) {
-            out[0] = lanes_rol1(o0);
-            out[1] = lanes_rol1(o1);
-        } else if (d == 63) {
-            out[0] = lanes_ror1(o0);
-            out[1] = lanes_ror1(o1);
-        } else {
-            const int src = (lane + d) & 63;
-            out[0] = __shfl(o0, src, 64);
-            out[1] = __shfl(o1, src, 64);
-        }
-    }
-}
-
-constexpr int kMeshWaveRows = 2;  // rows per wave of the wave-per-row mesh backward
 
 // D: the layers a launch may hold (registers are sized for it; the launch's
 // own depth is at most D).
@@ -517,13 +452,6 @@ __global__ void __launch_bounds__(kThreads) mesh_backward_wave(Mesh m, MeshGradS
         for (int k = 0; k < kThreads / 64; ++k) acc += sums[size_t(k) * n + i];
         partials[size_t(blockIdx.x) * n + i] = acc;
     }
-}
-
-int mesh_wave_cpl(int W) { return W <= 64 ? 1 : (W == 128 ? 2 : 0); }
-
-int mesh_wave_groups(int rows) {
-    const int per = kMeshWaveRows * (kThreads / 64);
-    return std::max(1, std::min((rows + per - 1) / per, 256));
 }
 
 // ---- norms (one wave per (row, group))
@@ -1197,26 +1125,51 @@ __global__ void __launch_bounds__(kThreads) gemm_tile_kernel(const float *__rest
     const int m0 = wave / tiles_n * 16, n0 = wave % tiles_n * 16, i = lane & 15, g = lane >> 4;
     const int m = m0 + i, n = n0 + i, kb = int(blockIdx.y) * kspan, ke = min(K, kb + kspan);
     v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k0 = kb; k0 < ke; k0 += 16) {
-        float a[4], b[4];
+    // Four 16-wide slices of K on their way at once: a wave has a handful of
+    // them, and waited for memory at each.
+    constexpr int U = 4;
+    for (int k0 = kb; k0 < ke; k0 += 16 * U) {
+        float a[U][4], b[U][4];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int k = k0 + 4 * g + s;
-            const bool ok = k < ke;
-            a[s] = ok && m < M ? (AK ? A[size_t(m) * lda + k] : A[size_t(k) * lda + m]) : 0.0f;
-            b[s] = ok && n < N ? (BK ? B[size_t(n) * ldb + k] : B[size_t(k) * ldb + n]) : 0.0f;
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int k = k0 + 16 * u + 4 * g + s;
+                const bool ok = k < ke;
+                a[u][s] = ok && m < M ? (AK ? A[size_t(m) * lda + k] : A[size_t(k) * lda + m]) : 0.0f;
+                b[u][s] = ok && n < N ? (BK ? B[size_t(n) * ldb + k] : B[size_t(k) * ldb + n]) : 0.0f;
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k0 + 16 * u >= ke) break;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][s], b[u][s], acc, 0, 0, 0);
         }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], acc, 0, 0, 0);
     }
     if (tokens) {
-        for (int r = kb; r < ke; ++r) {
-            const int t = int(tokens[r]) - m0;  // the same for every lane
-            if (t < 0 || t >= 16 || (t >> 2) != g || n >= N) continue;
-            const float d = dx[size_t(r) * N + n];
+        // The slice's rows whose token is one of the tile's, found for 64 rows at
+        // once and loaded four at a time, then added in row order.
+        for (int r0 = kb; r0 < ke; r0 += 64) {
+            const int mine = r0 + lane < ke ? int(tokens[r0 + lane]) - m0 : -1;
+            uint64_t hits = __ballot(mine >= 0 && mine < 16);
+            while (hits) {
+                int t[4];
+                float d[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if ((t & 3) == j) acc[j] += d;
+                for (int u = 0; u < 4; ++u) {
+                    const int at = hits ? int(__builtin_ctzll(hits)) : 0;
+                    t[u] = hits ? __builtin_amdgcn_readlane(mine, at) : -1;
+                    d[u] = t[u] >= 0 && n < N ? dx[size_t(r0 + at) * N + n] : 0.0f;
+                    hits &= hits - 1;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (t[u] < 0 || (t[u] >> 2) != g || n >= N) continue;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if ((t[u] & 3) == j) acc[j] += d[u];
+                }
+            }
         }
     }
     float *out = C + size_t(blockIdx.y) * cstride;

@@ -91,6 +91,50 @@ void mesh_backward_set(const Mesh &m, int count, const float *const *in, const f
                        float *partials, float *const *grad, int rows, hipStream_t stream,
                        std::vector<GradReduce> *deferred);
 
+// The row-local operators between two attentions as one launch each way
+// (train_chain.hip), bit for bit the separate kernels' results, for the shapes of
+// chain_fits() (widths up to 128, head widths a power of two up to 64, stacks of
+// few layers).  Rows are x_b -> xm -> x_{b+1} of block b; null pointers leave a
+// part out.
+bool chain_fits(const Mesh &ma, const Mesh &mf, int H);
+struct ForwardChain {
+    int rows;
+    Mesh ma, mf;
+    // x_out is the gathered rows E[tokens] (E set), or block b's post half: from
+    // the attention output z and x_in.
+    const float *E;
+    const uint32_t *tokens;
+    const float *z, *x_in, *wproj, *wffn;
+    float *ps, *xm, *n2, *inv2, *fs, *x_out;
+    // n = RMSNorm(x_out) with its factor, then (wqkv set) the next block's Q, K
+    // and V stacks, QK-Norm and RoPE.
+    float *n, *inv;
+    const float *wqkv[3];
+    float *qkv[3];
+    QkOut qk;
+};
+void forward_chain(const ForwardChain &a, hipStream_t stream);
+struct BackwardChain {
+    int rows;
+    Mesh ma, mf;
+    float *dx;  // d loss / d residual, read (unless dn is set) and written
+    // The final norm's backward from dn = d loss / d its output.
+    const float *dn, *x_last, *inv_last;
+    // Block b + 1's pre half: from dqkv (d loss / d rotated q and k, and v) to
+    // its input rows x_below, normalised n1.
+    const float *dqkv[3], *wqkv[3], *qkv[3], *qk_inv[2], *n1, *x_below, *inv1;
+    const float2 *table;
+    int sequence, H, norm, rotate;
+    // Block b's post half down to dt = d loss / d its attention output.
+    const float *wffn, *wproj, *n2, *fs, *xm, *inv2, *z, *ps;
+    float *dt;
+    float *part_qkv[3], *part_ffn, *part_proj;  // mesh_partial_floats each
+};
+// Appends the reductions of the stacks it ran, into grad[0..2] (Q, K, V),
+// grad[3] (FFN) and grad[4] (projection).
+void backward_chain(const BackwardChain &a, std::vector<GradReduce> *reductions, float *const *grad,
+                    hipStream_t stream);
+
 // RMSNorm over `groups` equal groups of each row (reference.rs:392-409):
 // y = x / sqrt(mean(x^2) + 1e-5); inv[row * groups + g] keeps the factor.
 void rmsnorm_forward(const float *x, float *y, float *inv, int rows, int W, int groups, hipStream_t stream);

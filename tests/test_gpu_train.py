@@ -169,6 +169,38 @@ def test_a_later_row_that_overflows_leaves_earlier_losses():
             model.cross_entropy(x, y, s)
 
 
+# The launches that chain the row-local operators between attentions: widths of
+# one and two registers a lane (whole, ragged), both depth limits and past them
+# (where the separate launches run either way), one and three blocks, each
+# switch, head widths from 2 to 64, few rows and more rows than waves.
+CHAIN = [(dict(width=32, heads=4, layers=2), 8, 32), (dict(width=128, heads=4, layers=2), 600, 4),
+         (dict(width=128, heads=2, layers=1, attention_mesh_depth=1, ffn_mesh_depth=1), 1, 1),
+         (dict(width=64, heads=8, layers=3, attention_mesh_depth=8, ffn_mesh_depth=8, connectivity=1), 3, 40),
+         (dict(width=24, heads=3, layers=2, attention_mesh_depth=5), 5, 7), (dict(width=8, heads=4, layers=2), 43, 3),
+         (dict(width=128, heads=8, layers=2, connectivity=1, rope=0), 9, 9),
+         (dict(width=128, heads=4, layers=2, qk_norm=0), 9, 9), (dict(width=64, heads=1, layers=2, xsa=0), 4, 70),
+         (dict(width=128, heads=4, layers=2, attention_mesh_depth=5), 9, 9),
+         (dict(width=32, heads=4, layers=2, ffn_mesh_depth=9), 9, 9), (dict(width=32, heads=4, embedding=1), 700, 3)]
+
+
+@pytest.mark.parametrize("cfg,b,s", CHAIN, ids=[f"{i}-W{c['width']}-{b}x{s}" for i, (c, b, s) in enumerate(CHAIN)])
+def test_chained_launches_give_the_separate_launches_bits(cfg, b, s, monkeypatch):
+    g = G.GptConfig(vocab_size=11, context=s, **cfg)
+    rng = np.random.default_rng(b)
+    x, y = (rng.integers(0, 11, b * s).astype(np.uint32) for _ in range(2))
+    got = {}
+    for off in ("0", "1"):
+        monkeypatch.setenv("MG_DISABLE_TRAIN_CHAIN", off)
+        with G.MeshGpt(0, g, 7) as model:
+            model.set_parameters(np.random.default_rng(3).uniform(
+                -1.0, 1.0, G.parameter_count(g)).astype(np.float32))
+            first = model.loss_and_gradient(x, y, s)
+            losses = [model.train_batch(x, y, s) for _ in range(3)]
+            got[off] = (first[0], first[1], losses, model.parameters(), model.cross_entropy(x, y, s))
+    assert got["0"][0] == got["1"][0] and got["0"][2] == got["1"][2] and got["0"][4] == got["1"][4]
+    assert np.array_equal(got["0"][1], got["1"][1]) and np.array_equal(got["0"][3], got["1"][3])
+
+
 # Stacks deeper than the 16 layers of one kernel launch, in the wave (width
 # <= 128) and the LDS (wider) mesh kernels, both connectivities, the mesh
 # embedding included.
