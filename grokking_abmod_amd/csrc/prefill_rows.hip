@@ -16,6 +16,17 @@
 // used for all of its rows.  Row reductions (RMSNorm) go through a small LDS
 // scratch; head reductions (QK-Norm, XSA) and the RoPE pair exchange stay
 // inside a wave (a head is hd <= 64 consecutive channels = consecutive lanes).
+//
+// What bounds it is instruction issue: five VALU instructions a value and layer
+// (product, multiply-add, exponential, multiply-add, maximum; values are carried
+// times log2(e), or it is six) and an LDS write and read of the value, behind a
+// barrier each layer that only other workgroups' waves on the SIMD can fill.
+// Widths 512 and 1024 keep to 128 registers for four waves a SIMD; 128 and 256,
+// with 16 rows a thread, would spill and keep three.  A prefill of 256 x 128 rows
+// (W1024, 12 blocks, 13 launches of this kernel, 527 us each at first): 8.84 ms,
+// 7.94 with the scaled values alone, 7.63 with four waves as well.
+// Not kept: strides of 256 and 512 from the
+// thread's own registers (7.73 ms), weights loaded two layers ahead (7.74).
 #include <hip/hip_runtime.h>
 
 #include "dpp.hpp"
@@ -28,11 +39,14 @@ constexpr float kEps = 1e-5f;  // src/gpt/mod.rs:38
 // (f64(1e-12f))^2 rounded to f32: the XSA norm floor of reference.rs:591.
 constexpr float kXsaNormFloor = float(double(1e-12f) * double(1e-12f));
 
-__device__ __forceinline__ float elu_f(float z) {
-    // max(z, clamp(exp(z), 0, 1) - 1) with the NaN-propagating maximum, which
-    // keeps a NaN z NaN (kernels.hip's elu)
-    const float e = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(z * 1.4426950408889634f), 0.0f, 1.0f);
-    return __builtin_elementwise_maximum(z, e - 1.0f);
+constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
+
+// The ELU of a value t carried times log2(e): max(t, log2(e) (clamp(2^t, 0, 1)
+// - 1)) with the NaN-propagating maximum, which keeps a NaN t NaN
+// (kernels.hip's elu).
+__device__ __forceinline__ float elu_log2(float t) {
+    const float e = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(t), 0.0f, 1.0f);
+    return __builtin_elementwise_maximum(t, __builtin_fmaf(e, kLog2e, -kLog2e));
 }
 
 template <int W>
@@ -46,6 +60,7 @@ struct RowsCfg {
     static constexpr int NCH = R / 4;             // 16-byte chunks of a channel
     static constexpr int ROT = R >= 64 ? 1 : 64 / R;  // channels per chunk rotation step
     static constexpr int TILE = W * R;            // floats of one LDS buffer
+    static constexpr int WAVES = CPT > 1 ? 4 : 3;  // of a SIMD
     static constexpr int WAVES_G = T / 64 > 0 ? T / 64 : 1;  // waves per row group
     static_assert(RG % 4 == 0 && W % 64 == 0, "tile geometry");
 };
@@ -95,40 +110,47 @@ struct Tile {
     }
     __device__ void flip() { parity ^= 1; }
 
+    // One layer on v in place: v[c] w0 + p[c] w1, and the ELU unless LAST.
+    template <bool LAST>
+    __device__ __forceinline__ void update(float (&v)[CPT][RG], const float (&p)[CPT][RG], const float2 (&w)[CPT]) {
+#pragma unroll
+        for (int k = 0; k < CPT; ++k)
+#pragma unroll
+            for (int i = 0; i < RG; ++i) {
+                const float t = v[k][i] * w[k].x + p[k][i] * w[k].y;
+                v[k][i] = LAST ? t : elu_log2(t);
+            }
+    }
+    template <bool LAST>
+    __device__ __forceinline__ void layer(float (&v)[CPT][RG], const float2 (&w)[CPT], int st) {
+        float p[CPT][RG];
+        put(v);
+        __syncthreads();
+        partner(st, p);
+        update<LAST>(v, p, w);
+        flip();
+    }
+
     // A mesh stack on v in place: layer l maps v[c] to v[c] w0 + v[c + st] w1
     // with ELU on every layer but the last (reference.rs:422-453).
     // Butterfly strides double from 1 and wrap at W (W is a power of two).
+    // Values are carried times log2(e), which the ELU's exponential would
+    // otherwise multiply in.
     __device__ void mesh(float (&v)[CPT][RG], const float2 *__restrict__ w, int depth, const Shape &s) {
         float2 wc[CPT];
 #pragma unroll
         for (int k = 0; k < CPT; ++k) wc[k] = w[chan(k)];
         int st = 1;
-        for (int l = 0; l < depth; ++l) {
-            put(v);
-            __syncthreads();
+        for (int l = 0; l + 1 < depth; ++l) {
             float2 wn[CPT];
-            if (l + 1 < depth) {
 #pragma unroll
-                for (int k = 0; k < CPT; ++k) wn[k] = w[size_t(l + 1) * W + chan(k)];
-            }
-            float p[CPT][RG];
-            partner(st, p);
-            if (l + 1 < depth) {
+            for (int k = 0; k < CPT; ++k) wn[k] = w[size_t(l + 1) * W + chan(k)];
+            layer<false>(v, wc, st);
 #pragma unroll
-                for (int k = 0; k < CPT; ++k)
-#pragma unroll
-                    for (int i = 0; i < RG; ++i) v[k][i] = elu_f(v[k][i] * wc[k].x + p[k][i] * wc[k].y);
-#pragma unroll
-                for (int k = 0; k < CPT; ++k) wc[k] = wn[k];
-            } else {
-#pragma unroll
-                for (int k = 0; k < CPT; ++k)
-#pragma unroll
-                    for (int i = 0; i < RG; ++i) v[k][i] = v[k][i] * wc[k].x + p[k][i] * wc[k].y;
-            }
-            flip();
+            for (int k = 0; k < CPT; ++k) wc[k] = wn[k];
             st = s.butterfly ? (2 * st == W ? 1 : 2 * st) : 1;
         }
+        layer<true>(v, wc, st);
     }
 
     // inv[i] = 1 / sqrt(mean over the row's W channels of v^2 + eps) for the
@@ -173,7 +195,7 @@ __device__ __forceinline__ float head_sum(float v, int hd) {
 // whole prefill sequences (Rows.len is null: a row's position is its index
 // within its sequence).
 template <int W, int HD>
-__global__ void __launch_bounds__(256) rows_block_kernel(BlockArgs a) {
+__global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(BlockArgs a) {
     using C = RowsCfg<W>;
     constexpr int CPT = C::CPT, RG = C::RG;
     __shared__ __align__(16) float lds[2 * C::TILE];
@@ -238,23 +260,27 @@ __global__ void __launch_bounds__(256) rows_block_kernel(BlockArgs a) {
                 }
             }
         }
+#pragma unroll
+        for (int k = 0; k < CPT; ++k)
+#pragma unroll
+            for (int i = 0; i < RG; ++i) y[k][i] *= kLog2e;
         t.mesh(y, reinterpret_cast<const float2 *>(a.wproj), s.A, s);
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) x[k][i] += y[k][i];
+            for (int i = 0; i < RG; ++i) x[k][i] = __builtin_fmaf(y[k][i], kLn2, x[k][i]);
         float inv[RG];
         t.row_inv_rms(x, inv);
         float n[CPT][RG];
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * inv[i];
+            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * (inv[i] * kLog2e);
         t.mesh(n, reinterpret_cast<const float2 *>(a.wffn), s.F, s);
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) x[k][i] += n[k][i];
+            for (int i = 0; i < RG; ++i) x[k][i] = __builtin_fmaf(n[k][i], kLn2, x[k][i]);
     }
     if (post || a.embed) {
 #pragma unroll
@@ -266,25 +292,26 @@ __global__ void __launch_bounds__(256) rows_block_kernel(BlockArgs a) {
     }
     if (!a.xn && !pre) return;
 
-    // The next RMSNorm: the final one for the head, or the block's pre-norm.
+    // The next RMSNorm: the final one for the head, or the block's pre-norm,
+    // whose rows enter the meshes times log2(e).
     float n[CPT][RG];
     {
         float inv[RG];
         t.row_inv_rms(x, inv);
+        if (a.xn) {
+#pragma unroll
+            for (int i = 0; i < RG; ++i)
+                if (live(i)) {
+#pragma unroll
+                    for (int k = 0; k < CPT; ++k) a.xn[grow(i) * W + t.chan(k)] = x[k][i] * inv[i];
+                }
+        }
+        if (!pre) return;
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * inv[i];
+            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * (inv[i] * kLog2e);
     }
-    if (a.xn) {
-#pragma unroll
-        for (int i = 0; i < RG; ++i)
-            if (live(i)) {
-#pragma unroll
-                for (int k = 0; k < CPT; ++k) a.xn[grow(i) * W + t.chan(k)] = n[k][i];
-            }
-    }
-    if (!pre) return;
 
     // Q, K and V meshes, one after another, each from the normalised rows.
     const size_t meshw = size_t(s.A) * W;
@@ -298,9 +325,14 @@ __global__ void __launch_bounds__(256) rows_block_kernel(BlockArgs a) {
             for (int i = 0; i < RG; ++i) v[k][i] = n[k][i];
         t.mesh(v, reinterpret_cast<const float2 *>(wm), s.A, s);
         (void)meshw;
+        // Addresses and RoPE factors are formed here for each mesh: hoisted out of
+        // the loop they would hold up to 60 registers through every layer.  (With
+        // 16 rows a thread, widths 128 and 256, forming them spills.)
+        int here = 0;
+        if constexpr (CPT > 1) asm volatile("" : "+v"(here));
 #pragma unroll
         for (int k = 0; k < CPT; ++k) {
-            const int c = t.chan(k), h = c / s.hd, d = c - h * s.hd;
+            const int c = t.chan(k) + here, h = c / s.hd, d = c - h * s.hd;
             if (m < 2) {
                 // QK-Norm per head, then RoPE at the row's position, each when
                 // its switch is on (reference.rs:174-193); the pair partner
@@ -308,7 +340,7 @@ __global__ void __launch_bounds__(256) rows_block_kernel(BlockArgs a) {
 #pragma unroll
                 for (int i = 0; i < RG; ++i) {
                     float q = v[k][i];
-                    if (s.qk_norm) q *= rsqrtf(head_sum<HD>(q * q, s.hd) * (1.0f / float(s.hd)) + kEps);
+                    q *= s.qk_norm ? rsqrtf(head_sum<HD>(q * q, s.hd) * (1.0f / float(s.hd)) + kEps * kLog2e * kLog2e) : kLn2;
                     if (s.rope) {
                         const float p = __shfl_xor(q, s.half, 64);
                         const float2 cs = a.rope[size_t(posof(i)) * s.half + (d < s.half ? d : d - s.half)];
@@ -316,6 +348,9 @@ __global__ void __launch_bounds__(256) rows_block_kernel(BlockArgs a) {
                     }
                     v[k][i] = q;
                 }
+            } else {
+#pragma unroll
+                for (int i = 0; i < RG; ++i) v[k][i] *= kLn2;
             }
 #pragma unroll
             for (int i = 0; i < RG; ++i) {

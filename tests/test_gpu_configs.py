@@ -671,3 +671,24 @@ def test_last_rows_alone_match_all_rows(W, H, n, batch):
         again = np.concatenate([tokens, model.read_tokens(batch, n + 1)[:, n:]], 1)
         again = model.logits(again.reshape(-1), n + 1, last_only=True)
         assert _prefill_error(model.last_logits(batch), again) <= 1e-5
+
+
+# The row-tile blocks at each register-tile width: tiles of 4096 / W rows with
+# one row more and one less, both connectivities, stacks of one layer (no ELU),
+# and QK-Norm off (the only factor that takes log2(e) from q and k) or on.
+@pytest.mark.parametrize("switch", [dict(), dict(qk_norm=0), dict(rope=0), dict(qk_norm=0, rope=0, xsa=0)],
+                         ids=["all", "no-qk", "no-rope", "none"])
+@pytest.mark.parametrize("W,H,n,A,F,butterfly", [(128, 4, 31, 7, 1, 1), (128, 8, 33, 1, 5, 0), (256, 4, 17, 8, 8, 1),
+                                                 (512, 8, 17, 9, 1, 1), (512, 16, 24, 1, 10, 0),
+                                                 (1024, 16, 19, 11, 1, 1), (1024, 32, 17, 3, 10, 1)])
+def test_row_tiles_match_the_oracle(W, H, n, A, F, butterfly, switch):
+    kw = dict(vocab_size=40, context=n, width=W, heads=H, layers=2, attention_mesh_depth=A, ffn_mesh_depth=F,
+              connectivity=butterfly, **switch)
+    o = O.config(**kw)
+    params = O.initialize(o, 7)
+    tokens = G.random_prompts(40, 3, n, 11).reshape(-1)
+    with G.MeshGpt(0, G.GptConfig(**kw), 7) as model:
+        model.set_parameters(params)
+        got = model.logits(tokens, n)
+    # the 2-norm allowance of _prefill_error's other uses: forty f32 roundings, four times
+    assert _prefill_error(got, O.logits(o, params, tokens, n)) <= 1e-5
