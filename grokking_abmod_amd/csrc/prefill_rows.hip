@@ -23,7 +23,7 @@
 // barrier each layer that only other workgroups' waves on the SIMD can fill.
 // Widths 512 and 1024 keep to 128 registers for four waves a SIMD; 128 and 256,
 // with 16 rows a thread, would spill and keep three.  A prefill of 256 x 128 rows
-// (W1024, 12 blocks, 13 launches of this kernel, 527 us each at first): 8.84 ms,
+// (W1024, 12 blocks, 13 launches of this kernel, 527 us each before and 446 now): 8.84 ms,
 // 7.94 with the scaled values alone, 7.63 with four waves as well.
 // Not kept: strides of 256 and 512 from the thread's own registers (7.73 ms), weights
 // loaded two layers ahead (7.74).
