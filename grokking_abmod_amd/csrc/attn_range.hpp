@@ -9,7 +9,8 @@ namespace meshgpt::kern {
 
 constexpr int kSplitKeys = 64;     // keys of a tile
 constexpr int kSplitSpread = 10;   // see attn_split.hip
-constexpr int kBadRange = 4096;    // a tile whose values have no usable exponent
+constexpr int kSplitTiny = 4;      // see attn_split.hip
+constexpr int kBadRange = 4096;    // a tile whose values need the FP32 kernel
 constexpr int kNoRow = 2048;       // a tile of zeros
 
 // The exponent E of the largest |v| of a pair (v < 2^E) from its tiles' ranges

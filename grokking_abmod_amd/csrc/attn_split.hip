@@ -16,10 +16,18 @@
 //    2^-13 times a typical one still keep 24 bits;
 //  - v by 2^(14 - e), e the exponent of its key tile's largest |v|, and the
 //    probability by 2^(14 + e - E), E the largest e of the (sequence, head),
-//    so that every tile adds in the same units.
-// This needs the rows of v to be of similar size.  Where the smallest row's
-// largest entry lies more than 2^kSplitSpread below the largest of all, or an
-// entry is not finite, the (sequence, head) runs in the FP32 kernel instead.
+//    so that every tile adds in the same units;
+//  - v's second half by 2^11 more, and the probability's first half by 2^-11
+//    where it meets it: one scale serves all of a tile's channels, and so an
+//    entry keeps 24 bits down to 2^-26 of the tile's largest and not to 2^-15.
+// A (sequence, head) runs in the FP32 kernel instead where that is not enough:
+//  - its smallest row's largest entry lies more than 2^kSplitSpread below the
+//    largest of all (the probabilities' scale then takes their low bits);
+//  - a tile holds more than kSplitTiny entries below 2^(e - 26), as a channel
+//    that is small in every row does.  (Normally distributed values have such
+//    an entry once in some 2500 tiles, by chance, and it is off by less than
+//    2^-50 of the tile's largest);
+//  - an entry is not finite.
 //
 // attn_split_prepare_kernel writes k and v of a key tile once as f16 planes in
 // the order the products read them: k as [key][dim], v as [dim][key].  Each
@@ -29,17 +37,23 @@
 // first product (keys 8 a + 4 (lane / 32) + b of query lane % 32) are, in
 // order, the operand of the second.  The planes are as large as k and v.
 //
-// Measured on 64 pairs of 8192 rows of 64 dims (0.55 TFLOP a launch): 1.58 ms,
-// 1.04 PFLOP/s of FP16 products, where a large bf16 matrix product of a library
-// reaches 1.21 on the same card; the FP32 kernel takes 5.25 ms.  More waves on a
-// SIMD (128 registers, four waves) are slower (9.99 against 9.07 ms a prefill).
-// The probability's scale multiplies the exponential's result: added to its
-// argument it cost no instruction, but arguments near 14 round to 2^-21 and put
-// a tenth on the logits' error (1.60 and 1.65 ms a launch traced, 7.51 a prefill both).  The error against 64 bits
-// is now the FP32 kernel's or less (8 x 8192 rows, seeded weights, three draws:
-// 1.8e-7 and 1.8e-7, 2.1e-7 and 2.1e-7, 1.9e-7 and 2.0e-7).  Forming the next
+// Measured on 64 pairs of 8192 rows of 64 dims (0.55 TFLOP a launch): 1.66 ms,
+// 0.99 PFLOP/s of FP16 products, where a large bf16 matrix product of a library
+// reaches 1.21 on the same card; the FP32 kernel takes 5.25 ms.  (v's second
+// half without its own scale: 1.65 ms.)  More waves on a SIMD (128 registers,
+// four waves) are slower (9.99 against 9.07 ms a prefill).  Forming the next
 // tile's scores beside this one's softmax in each wave gains nothing (7.6-7.9 ms
 // a prefill against 7.5): two waves a SIMD already overlap the two.
+//
+// The error against 64 bits is the FP32 kernel's with seeded and with normally
+// distributed weights (8 x 8192 rows, three draws: 1.8e-7 and 1.8e-7, 2.1e-7 and
+// 2.1e-7, 1.9e-7 and 2.0e-7; 320 rows with every third value channel 2^-12 of the
+// others' size and grown back behind the attention: 9.2e-8 both).  Where XSA
+// takes away all but rounding, the operands' own rounding shows: up to 1.7 times
+// the FP32 kernel's error with sixteen token vectors that differ in signs only.
+// The probability's scale multiplies the exponential's result: added to its
+// argument it cost no instruction, but arguments near 14 round to 2^-21 and put
+// a tenth on the logits' error.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -66,6 +80,7 @@ constexpr int kBK = kSplitKeys;
 // rows 0.51 and 0.47 ms, 16 x 449 0.99 and 1.16; W1024, 12 blocks: 16 x 300
 // 2.21 and 2.32).
 constexpr int kSplitRows = 288;
+constexpr float kLowScale = 2048.0f;  // of v's second half
 constexpr float kQScale = 16384.0f, kKScale = 4096.0f, kScoreUnit = 1.0f / (16384.0f * 4096.0f);
 
 template <int HD>
@@ -87,12 +102,13 @@ __device__ __forceinline__ v16f mfma(h8 a, h8 b, v16f c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ void split(const float (&x)[8], h8 &h, h8 &m) {
+// x as h + m / low.
+__device__ __forceinline__ void split(const float (&x)[8], h8 &h, h8 &m, float low = 1.0f) {
 #pragma unroll
     for (int i = 0; i < 8; i += 2) {
         const f2 v = {x[i], x[i + 1]};
         const h2 a = __builtin_convertvector(v, h2);
-        const f2 r = {x[i] - float(a[0]), x[i + 1] - float(a[1])};
+        const f2 r = {(x[i] - float(a[0])) * low, (x[i + 1] - float(a[1])) * low};
         const h2 b = __builtin_convertvector(r, h2);
         h[i] = a[0];
         h[i + 1] = a[1];
@@ -108,13 +124,15 @@ __device__ __forceinline__ int exponent_of(float x) {
 }
 
 // The planes of one tile, and its range (pair_splits): the exponent of its
-// largest |v| and of its smallest row's, kBadRange when an entry is not finite
-// or all are below 2^-100.  A row of zeros has no size and counts for neither.
+// largest |v| and of its smallest row's, kBadRange when an entry is not finite,
+// all are below 2^-100 or more than kSplitTiny are too small beside the largest.
+// Zeros have no size: they count for none of these.
 template <int HD>
 __global__ void __launch_bounds__(256)
 attn_split_prepare_kernel(KvView kv, int n, int tiles, _Float16 *__restrict__ planes, int2 *__restrict__ range) {
     using C = Split<HD>;
     __shared__ float big[4], small[4];
+    __shared__ int tiny[4];
     const int tile = int(blockIdx.x) % tiles, pair = int(blockIdx.x) / tiles, t0 = tile * kBK;
     const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
     const size_t slab = size_t(pair) * kv.cap * HD;
@@ -173,19 +191,26 @@ attn_split_prepare_kernel(KvView kv, int n, int tiles, _Float16 *__restrict__ pl
     const int e = isfinite(top) && top > 0.0f ? exponent_of(top) : 0;
     const bool good = isfinite(top) && e >= -100;
     const float scale = good ? ldexpf(1.0f, 14 - e) : 0.0f;
+    int few = 0;
 #pragma unroll
     for (int u = 0; u < VP; ++u) {
         const int d = lane % HD, c = (u * 4 + wave) * PER + lane / HD;
         float y[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) y[i] = x[u][i] * scale;
+        for (int i = 0; i < 8; ++i) {
+            y[i] = x[u][i] * scale;
+            few += int(__popcll(__ballot(fabsf(y[i]) < 0x1p-12f && x[u][i] != 0.0f)));
+        }
         h8 h, m;
-        split(y, h, m);
+        split(y, h, m, kLowScale);
         *reinterpret_cast<h8 *>(out + 2 * C::KPLANE + slot_at<8>(d, c)) = h;
         *reinterpret_cast<h8 *>(out + 3 * C::KPLANE + slot_at<8>(d, c)) = m;
     }
+    if (lane == 0) tiny[wave] = few;
+    __syncthreads();
+    const bool even = tiny[0] + tiny[1] + tiny[2] + tiny[3] <= kSplitTiny;
     if (threadIdx.x == 0)
-        range[blockIdx.x] = !good                ? make_int2(kBadRange, 0)
+        range[blockIdx.x] = !good || !even       ? make_int2(kBadRange, 0)
                             : isfinite(low)      ? make_int2(e, exponent_of(low))
                                                  : make_int2(-kNoRow, kNoRow);
 }
@@ -331,6 +356,7 @@ attn_split_kernel(Shape s, const float *__restrict__ q, KvView kv, const _Float1
                 for (int i = 0; i < 8; ++i) p[i] = sc[k / 2][8 * (k % 2) + i] * up;
                 h8 ph, pm;
                 split(p, ph, pm);
+                const h8 pl = ph * _Float16(1.0f / kLowScale);
                 h8 vh[C::DB], vm[C::DB];
 #pragma unroll
                 for (int d = 0; d < C::DB; ++d) {
@@ -338,7 +364,7 @@ attn_split_kernel(Shape s, const float *__restrict__ q, KvView kv, const _Float1
                     vm[d] = *reinterpret_cast<const h8 *>(vp + C::KPLANE + slot_at<8>(32 * d + jq, 2 * k + hf));
                 }
 #pragma unroll
-                for (int d = 0; d < C::DB; ++d) acc[d] = mfma(vm[d], ph, acc[d]);
+                for (int d = 0; d < C::DB; ++d) acc[d] = mfma(vm[d], pl, acc[d]);
 #pragma unroll
                 for (int d = 0; d < C::DB; ++d) acc[d] = mfma(vh[d], pm, acc[d]);
 #pragma unroll

@@ -599,37 +599,82 @@ def test_long_prefill_matches_the_oracle(n, heads):
     assert error["0"] <= 1.2 * error["1"], error
 
 
-@pytest.mark.parametrize("wide", ["every head", "one head", "zero rows"])
-def test_split_prefill_leaves_wide_values_to_fp32(wide):
+def _split_and_fp32(kw, params, tokens, n):
+    """The logits with long prefills on split FP16 operands where they fit, and on FP32 ones."""
+    got = []
+    for off in ("0", "1"):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setenv("MG_DISABLE_SPLIT_PREFILL", off)
+            with G.MeshGpt(0, G.GptConfig(**kw), 7) as model:
+                model.set_parameters(params)
+                got.append(model.logits(tokens, n))
+    return got
+
+
+# 128- and 256-query workgroups of the FP32 kernel that takes the pairs left to it
+@pytest.mark.parametrize("n", [300, 2100])
+@pytest.mark.parametrize("H", [2, 4])
+@pytest.mark.parametrize("wide", ["every head", "one head", "within", "zero rows"])
+def test_split_prefill_leaves_wide_values_to_fp32(wide, H, n):
     """Value rows of very different sizes: token 0's channels are all negative
     (in one head or in every one) and saturate at -1 in a V mesh that grows
     positive ones 2500 times.  Those pairs run on the FP32 kernel: with every
-    head affected the logits are its own bit for bit.  A V mesh of zeros keeps
-    the split kernels: rows without a size count for nothing."""
-    n, W, H = 300, 128, 2
+    head affected the logits are its own bit for bit.  Grown 484 times, rows
+    580 to 1 in size are split, and a V mesh of zeros is: rows without a size
+    count for nothing.  Sixteen vectors make all rows, so XSA takes most of an
+    attention row away and what is left shows the products' own rounding: each
+    operand's (2^-23 at most, none in FP32) beside the sums' (2^-24 an addition),
+    twice the FP32 kernel's error at most."""
+    W = 128
     kw = dict(vocab_size=16, context=n, width=W, heads=H, layers=1, attention_mesh_depth=3, ffn_mesh_depth=2,
               embedding=1)
-    g, o = G.GptConfig(**kw), O.config(**kw)
+    o = O.config(**kw)
     params = O.initialize(o, 7)
     rng = np.random.default_rng(3)
     table = params[:16 * W].reshape(16, W)
     table[:] = rng.choice([-1.0, 1.0], (16, W)) * rng.uniform(0.8, 1.2, (16, W))
-    table[0, :W if wide == "every head" else W // H] = -1.0
+    table[0, :W // H if wide == "one head" else W] = -1.0
     v = params[O.group_offsets(o)[3]:][:2 * W * 3].reshape(3, W, 2)
     v[:, :, 1] = 0.0
-    v[:, :, 0] = 0.0 if wide == "zero rows" else np.array([50.0, 50.0, 1.0])[:, None]
+    grow = {"zero rows": 0.0, "within": 22.0}.get(wide, 50.0)
+    v[:, :, 0] = np.array([grow, grow, 1.0 if grow else 0.0])[:, None]
     tokens = rng.integers(0, 16, n).astype(np.uint32)
     ref = O.logits(o, params, tokens, n)
-    got = {}
-    for off in ("0", "1"):
-        with pytest.MonkeyPatch.context() as mp:
-            mp.setenv("MG_DISABLE_SPLIT_PREFILL", off)
-            with G.MeshGpt(0, g, 7) as model:
-                model.set_parameters(params)
-                got[off] = model.logits(tokens, n)
-    assert _prefill_error(got["0"], ref) <= 1e-5 and _prefill_error(got["1"], ref) <= 1e-5
+    split, fp32 = _split_and_fp32(kw, params, tokens, n)
+    # forty f32 roundings, four times, as in test_long_prefill_matches_the_oracle
+    assert _prefill_error(split, ref) <= 1e-5 and _prefill_error(fp32, ref) <= 1e-5
     if wide == "every head":
-        assert np.array_equal(got["0"], got["1"])
+        assert np.array_equal(split, fp32)
+    else:
+        assert _prefill_error(split, ref) <= 2 * _prefill_error(fp32, ref)
+
+
+@pytest.mark.parametrize("H", [2, 4])
+@pytest.mark.parametrize("below", [6, 12, 16, 20, 24, 30, 60])
+def test_split_prefill_keeps_small_channels(below, H):
+    """Every third value channel 2^-below times its size, grown back (exactly) by
+    the projection's first layer: its bits count as much as the others'.  The
+    split operands' error may not pass 1.2 times the FP32 kernel's."""
+    n, W, A = 320, 128, 3
+    kw = dict(vocab_size=64, context=n, width=W, heads=H, layers=1, attention_mesh_depth=A, ffn_mesh_depth=2,
+              embedding=1)
+    o = O.config(**kw)
+    params = G.normal_parameters(G.GptConfig(**kw), 5)
+    size = np.where(np.arange(W) % 3 == 1, 2.0 ** -below, 1.0)
+    stack = 2 * W * A
+    offsets = O.group_offsets(o)
+    v = params[offsets[3]:][:stack].reshape(A, W, 2)
+    v[-1] *= size[:, None]
+    projection = params[offsets[4]:][:stack].reshape(A, W, 2)
+    projection[0, :, 0] /= size
+    projection[0, :, 1] /= np.roll(size, -1)
+    tokens = G.random_prompts(64, 1, n, 11)[0]
+    ref = O.logits(o, params, tokens, n)
+    split, fp32 = _split_and_fp32(kw, params, tokens, n)
+    error = _prefill_error(split, ref), _prefill_error(fp32, ref)
+    assert max(error) <= 1e-5 and error[0] <= 1.2 * error[1], error
+    if below >= 24:
+        assert np.array_equal(split, fp32)
 
 
 def test_split_prefill_reports_values_that_overflow():
