@@ -397,7 +397,6 @@ void attn_prefill_short(const Shape &s, const float *q, KvView kv, int nseq, int
     else
         hipLaunchKernelGGL(attn_short_kernel<64>, dim3(blocks), dim3(256), 0, stream, s, q, kv, rows, rows_per_seq,
                            y, scale_log2, xsa);
-    (void)hipGetLastError();
 }
 
 bool attn_prefill_mfma_supported(const Shape &s, int rows_per_seq) {
@@ -431,7 +430,6 @@ void attn_prefill_mfma(const Shape &s, const float *q, KvView kv, int nseq, int 
         launch(attn_prefill_mfma_kernel<64, 4, 2>, 128, 4);
     else
         launch(attn_prefill_mfma_kernel<64, 4, 1>, 64, 4);
-    (void)hipGetLastError();
 }
 
 }  // namespace meshgpt::kern

@@ -443,7 +443,6 @@ const int2 *attn_split(const Shape &s, const float *q, KvView kv, int nseq, int 
     else
         longer ? launch(attn_split_prepare_kernel<64>, attn_split_kernel<64, 8>, 8)
                : launch(attn_split_prepare_kernel<64>, attn_split_kernel<64, 4>, 4);
-    (void)hipGetLastError();
     return range;
 }
 

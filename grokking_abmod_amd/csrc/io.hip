@@ -41,13 +41,11 @@ void start_rows(const uint32_t *prompts, int batch, int n, uint32_t *tokens, siz
                 uint64_t seed, int *flags, hipStream_t stream) {
     hipLaunchKernelGGL(start_rows_kernel, dim3(batch), dim3(256), 0, stream, prompts, n, tokens, stride, len, rng, seed,
                        flags);
-    (void)hipGetLastError();
 }
 
 void gather_rows(const uint32_t *tokens, size_t stride, int batch, int n, uint32_t *out, hipStream_t stream) {
     if (batch && n)
         hipLaunchKernelGGL(gather_rows_kernel, dim3(batch), dim3(256), 0, stream, tokens, stride, n, out);
-    (void)hipGetLastError();
 }
 
 void nonfinite(const float *x, size_t n, int *flag, hipStream_t stream) {
@@ -55,7 +53,6 @@ void nonfinite(const float *x, size_t n, int *flag, hipStream_t stream) {
     const size_t blocks = n / 1024 + 1;
     hipLaunchKernelGGL(nonfinite_kernel, dim3(unsigned(blocks < 1024 ? blocks : 1024)), dim3(256), 0, stream, x, n,
                        flag);
-    (void)hipGetLastError();
 }
 
 }  // namespace meshgpt::kern

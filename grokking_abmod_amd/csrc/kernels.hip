@@ -39,7 +39,6 @@ constexpr float kRmsEps = 1e-5f;  // src/gpt/mod.rs:38
 typedef __attribute__((address_space(1))) uint64_t global_u64;
 constexpr float kXsaFloor = float(double(1e-12f) * double(1e-12f));
 
-#define HIP_LAUNCH_CHECK() (void)hipGetLastError()
 
 
 template <int CTRL, int ROW_MASK = 0xf>
@@ -3807,7 +3806,6 @@ void launch_decode_t(const Shape &s, const float *q, KvView kv, const int *len, 
         hipLaunchKernelGGL(attn_decode_kernel<HDP>, grid, dim3(DecodeCfg<HDP>::THREADS), 0, stream, s, q, kv,
                            len, nsplit, part, scale_log2);
     }
-    HIP_LAUNCH_CHECK();
 }
 
 template <int HDP>
@@ -3818,7 +3816,6 @@ void launch_prefill_t(const Shape &s, const float *q, KvView kv, int nseq, int r
     dim3 grid(ntiles * nseq, s.H);
     hipLaunchKernelGGL(attn_prefill_kernel<HDP>, grid, dim3(kThreads), 0, stream, s, q, kv, rows_per_seq,
                        y, scale_log2);
-    HIP_LAUNCH_CHECK();
 }
 
 template <class F>
@@ -3899,20 +3896,17 @@ void mesh_rows(const Shape &s, const float *in, float *out, int rows, const floa
         hipLaunchKernelGGL(mesh_rows_kernel<decltype(c)::value>, grid, dim3(team_threads(s.W)),
                            mesh_lds_bytes(s, rpw), stream, s, in, out, rows, w, depth, rpw);
     });
-    HIP_LAUNCH_CHECK();
 }
 
 void embedding_geometry(float *E, const float *codes, int V, int W, float radius, int normalize, int keep,
                         hipStream_t stream) {
     hipLaunchKernelGGL(embedding_geometry_kernel, dim3(V), dim3(kThreads), 0, stream, E, codes, W, radius, normalize,
                        keep);
-    HIP_LAUNCH_CHECK();
 }
 
 void transpose(const float *E, float *Et, int V, int Vp, int W, hipStream_t stream) {
     dim3 grid((Vp + 31) / 32, (W + 31) / 32);
     hipLaunchKernelGGL(transpose_kernel, grid, dim3(kThreads), 0, stream, E, Et, V, Vp, W);
-    HIP_LAUNCH_CHECK();
 }
 
 void block(const BlockArgs &a, bool staged, hipStream_t stream) {
@@ -3929,7 +3923,6 @@ void block(const BlockArgs &a, bool staged, hipStream_t stream) {
             else hipLaunchKernelGGL((block_kernel<C, false, 1>), grid, threads, lds, stream, a);
         }
     });
-    HIP_LAUNCH_CHECK();
 }
 
 bool block_decode_supported(const Shape &s) {
@@ -3956,7 +3949,6 @@ void block_decode(const BlockArgs &a, hipStream_t stream) {
             }
         });
     }
-    HIP_LAUNCH_CHECK();
 }
 
 int row_waves(int W) { return W >= 256 ? 4 : 2; }
@@ -4039,12 +4031,10 @@ void row_block(const BlockArgs &a, hipStream_t stream) {
     const bool fixed = s.butterfly && s.A == s.F && s.hd == 64;
     if (fixed && s.W == 512 && s.A == 9) {
         launch_row_block_rows<4, 2, 16, 9>(a, teams, stream);
-        HIP_LAUNCH_CHECK();
         return;
     }
     if (fixed && s.W == 1024 && s.A == 10) {
         launch_row_block_rows<4, 4, 16, 10>(a, teams, stream);
-        HIP_LAUNCH_CHECK();
         return;
     }
     const dim3 grid(a.ro.rows * teams);
@@ -4054,7 +4044,6 @@ void row_block(const BlockArgs &a, hipStream_t stream) {
     case 512: launch_row_block<4, 2>(a, grid, stream); break;
     default: launch_row_block<4, 4>(a, grid, stream); break;
     }
-    HIP_LAUNCH_CHECK();
 }
 
 void row_order(const float *src, float *dst, int rows, int W, bool pairs, hipStream_t stream) {
@@ -4067,7 +4056,6 @@ void row_order(const float *src, float *dst, int rows, int W, bool pairs, hipStr
     else
         hipLaunchKernelGGL(row_order_kernel<float>, dim3(blocks), dim3(kThreads), 0, stream, src, dst, rows, W,
                            row_waves(W));
-    HIP_LAUNCH_CHECK();
 }
 
 // The persistent kernel instantiation for a shape, or nullptr.
@@ -4126,8 +4114,11 @@ bool persistent_fits(const Shape &s, int batch, int device) {
     const void *f = persistent_kernel(s);
     if (!f) return false;
     int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, 64 * row_waves(s.W), 0) != hipSuccess) return false;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return false;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, 64 * row_waves(s.W), 0) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+        (void)hipGetLastError();  // answered here, no launch error
+        return false;
+    }
     return persistent_blocks(s, batch) <= per_cu * cus;
 }
 
@@ -4162,7 +4153,6 @@ bool persistent_layer0(const Shape &s, const float *E, const float *w, size_t bl
         constexpr int NW = decltype(nw)::value;
         hipLaunchKernelGGL((layer0_kernel<NW, decltype(cpl)::value, decltype(gl)::value, decltype(depth)::value>),
                            dim3(3 * s.V), dim3(64 * NW), 0, stream, s, E, w, block0, q0);
-        HIP_LAUNCH_CHECK();
         (void)hdp;
     });
 }
@@ -4210,7 +4200,6 @@ void head(const Shape &s, const float *xn, int nrows, int row_mul, int row_add, 
     dim3 grid((s.V + kHeadTokens - 1) / kHeadTokens, (nrows + rt - 1) / rt);
     hipLaunchKernelGGL(head_kernel, grid, dim3(kThreads), head_lds_bytes(s, rt), stream, s, xn, nrows, row_mul,
                        row_add, Et, Vp, logits, rt);
-    HIP_LAUNCH_CHECK();
 }
 
 void head_sample(const Shape &s, const float *xn, int batch, const float *Et, int Vp, float *logits,
@@ -4218,20 +4207,17 @@ void head_sample(const Shape &s, const float *xn, int batch, const float *Et, in
                  hipStream_t stream) {
     hipLaunchKernelGGL(head_sample_kernel, dim3(batch), dim3(kHsThreads), head_sample_lds_bytes(s), stream, s, xn,
                        Et, Vp, logits, temperature, rng, tokens, tok_stride, len, flags);
-    HIP_LAUNCH_CHECK();
 }
 
 void device_expf(const float *x, float *y, size_t n, hipStream_t stream) {
     const int blocks = int(std::min<size_t>((n + kThreads - 1) / kThreads, 4096));
     if (blocks > 0) hipLaunchKernelGGL(expf_kernel, dim3(blocks), dim3(kThreads), 0, stream, x, y, n);
-    HIP_LAUNCH_CHECK();
 }
 
 void calibration_copy(const float4 *src, float4 *dst, size_t n, hipStream_t stream) {
     const size_t blocks = std::min<size_t>((n + kThreads - 1) / kThreads, 256 * 16);
     hipLaunchKernelGGL(calibration_copy_kernel, dim3(unsigned(std::max<size_t>(blocks, 1))), dim3(kThreads), 0,
                        stream, src, dst, n);
-    HIP_LAUNCH_CHECK();
 }
 
 void sample(int V, int batch, const float *logits, float temperature, uint64_t *rng, uint32_t *tokens,
@@ -4245,7 +4231,6 @@ void sample(int V, int batch, const float *logits, float temperature, uint64_t *
     else
         hipLaunchKernelGGL(sample_kernel, dim3(batch), dim3(kThreads), 0, stream, logits, V, temperature, rng, tokens,
                            tok_stride, len, flags);
-    HIP_LAUNCH_CHECK();
 }
 
 }  // namespace meshgpt::kern

@@ -15,9 +15,17 @@ namespace meshgpt {
 namespace {
 
 void check(hipError_t e, const char *what) {
-    if (e != hipSuccess)
-        throw Error(std::string(what) + ": " + hipGetErrorString(e),
-                    e == hipErrorOutOfMemory ? kOutOfMemory : kDeviceError);
+    if (e == hipSuccess) return;
+    (void)hipGetLastError();  // reported here, not by the next call's sync()
+    throw Error(std::string(what) + ": " + hipGetErrorString(e), e == hipErrorOutOfMemory ? kOutOfMemory : kDeviceError);
+}
+
+// The device of a call, and a clean slate for its launches: a refused one is
+// the thread's last error, which sync() reports; what the caller's own HIP
+// calls left there is not this call's.
+void use_device(int device) {
+    check(hipSetDevice(device), "hipSetDevice");
+    (void)hipGetLastError();
 }
 
 struct DevBuf {
@@ -218,7 +226,8 @@ struct MeshGpt::Impl {
     // After the call's sync: the time between its two marks.
     void close_call() { check(hipEventElapsedTime(&call_ms, call_ev[0], call_ev[1]), "hipEventElapsedTime"); }
 
-    void activate() const { check(hipSetDevice(device), "hipSetDevice"); }
+    // The first thing that a public call does on the device.
+    void activate() const { use_device(device); }
 
     void drop_graph() {
         for (int i = 0; i < 2; ++i) {
@@ -1486,7 +1495,6 @@ struct MeshGpt::Impl {
     // The first len tokens of b sequences; with `checked`, finish() on the way.
     void read_tokens(uint32_t *out, size_t b, size_t len, bool checked = false) {
         if (b > batch || len > length) throw Error("requested tokens exceed the generated sequences");
-        activate();
         dstage.ensure(b * len * 4);
         kern::gather_rows(dtokens.as<uint32_t>(), tcap, int(b), int(len), dstage.as<uint32_t>(), stream);
         const bool ask = checked && known_flags < 0;
@@ -1810,7 +1818,10 @@ size_t MeshGpt::sequence_length() const { return impl_->length; }
 
 float MeshGpt::last_call_ms() const { return impl_->call_ms; }
 
-void MeshGpt::read_tokens(uint32_t *out, size_t batch, size_t length) { impl_->read_tokens(out, batch, length); }
+void MeshGpt::read_tokens(uint32_t *out, size_t batch, size_t length) {
+    impl_->activate();
+    impl_->read_tokens(out, batch, length);
+}
 
 std::vector<float> MeshGpt::last_logits() {
     std::vector<float> out(impl_->batch * impl_->cfg.vocab_size);
@@ -1837,7 +1848,7 @@ bool sample_logits(int device, const float *logits, size_t rows, size_t vocab, f
     int count = 0;
     check(hipGetDeviceCount(&count), "hipGetDeviceCount");
     if (device < 0 || device >= count) throw Error("invalid device ordinal", kDeviceError);
-    check(hipSetDevice(device), "hipSetDevice");
+    use_device(device);
     DevBuf dl, drng, dtok, dlen, dflags;
     dl.ensure(rows * vocab * 4);
     drng.ensure(rows * 8);
@@ -1877,7 +1888,7 @@ void sample_logits_noalloc(int device, const float *logits, size_t rows, size_t 
         int device;
         ~Restore() { (void)hipSetDevice(device); }
     } restore{caller};
-    check(hipSetDevice(device), "hipSetDevice");
+    use_device(device);
     int *counters = nullptr;
     check(kern::noalloc_scratch(device, &counters), "hipGetSymbolAddress(scratch)");
     kern::fill_int(nonfinite, 0, 1, stream);
@@ -1894,7 +1905,7 @@ void device_expf(int device, const float *x, size_t n, float *out) {
     int count = 0;
     check(hipGetDeviceCount(&count), "hipGetDeviceCount");
     if (device < 0 || device >= count) throw Error("invalid device ordinal", kDeviceError);
-    check(hipSetDevice(device), "hipSetDevice");
+    use_device(device);
     DevBuf dx, dy;
     dx.ensure(n * 4);
     dy.ensure(n * 4);
@@ -1909,7 +1920,7 @@ double copy_bandwidth(int device, size_t bytes, int iters) {
     int count = 0;
     check(hipGetDeviceCount(&count), "hipGetDeviceCount");
     if (device < 0 || device >= count) throw Error("invalid device ordinal", kDeviceError);
-    check(hipSetDevice(device), "hipSetDevice");
+    use_device(device);
     const size_t n = bytes / 16;
     DevBuf src, dst;
     src.ensure(n * 16);

@@ -428,13 +428,11 @@ void rows_block(const BlockArgs &a, hipStream_t stream) {
     case 512: launch_rows_block<512>(a, stream); break;
     default: launch_rows_block<1024>(a, stream); break;
     }
-    (void)hipGetLastError();
 }
 
 void last_rows(const float *q, const float *x, int nseq, int n, int W, float *q_out, float *x_out, int *len,
                hipStream_t stream) {
     hipLaunchKernelGGL(last_rows_kernel, dim3(nseq), dim3(256), 0, stream, q, x, n, W, q_out, x_out, len);
-    (void)hipGetLastError();
 }
 
 void last_merge(const Shape &s, const float *part, int nsplit, KvView kv, int nseq, int n, int xsa, float *y,
@@ -442,7 +440,6 @@ void last_merge(const Shape &s, const float *part, int nsplit, KvView kv, int ns
     const int pairs = nseq * s.H;
     hipLaunchKernelGGL(last_merge_kernel, dim3((pairs + 3) / 4), dim3(256), 0, stream, s, part, nsplit, kv, n, pairs,
                        xsa, y);
-    (void)hipGetLastError();
 }
 
 }  // namespace meshgpt::kern

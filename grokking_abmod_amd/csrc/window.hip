@@ -464,9 +464,10 @@ void launch_window(const WindowArgs &a, int batch, hipStream_t stream) {
     const size_t lds = (3 * 4 * NW * (W + 4) + 16 + W + 256 + kRing) * 4 + 32 * 8;
     const size_t staged = (size_t(a.L) * 2 * W * (4 * a.A + a.F) + size_t(a.V) * W) * 4;
     auto launch = [&](auto kernel, size_t bytes) {
-        if (bytes > 65536)
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes));
+        // A refusal is the thread's last error, which the model's next wait reports.
+        if (bytes > 65536 && hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)) != hipSuccess)
+            return;
         hipLaunchKernelGGL(kernel, dim3(batch), dim3(64 * NW), bytes, stream, a);
     };
     if constexpr (NW == 8) {
@@ -521,7 +522,6 @@ void window_generate(const Shape &s, WindowArgs a, int batch, hipStream_t stream
         a.context <= kWindowRows / 2 ? launch_window<C, D, 8>(a, batch, stream)
                                      : launch_window<C, D, 16>(a, batch, stream);
     });
-    (void)hipGetLastError();
 }
 
 }  // namespace meshgpt::kern

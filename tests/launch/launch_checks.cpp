@@ -1,0 +1,156 @@
+// What the host launches, checked on a machine without a GPU: the library's
+// objects against fake_hip.cpp.  `launch_checks NAME` runs one check.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "fake_hip.hpp"
+#include "kernels.hpp"
+#include "model.hpp"
+#include "train.hpp"
+
+using namespace meshgpt;
+
+namespace {
+
+void expect(bool ok, const std::string &what) {
+    if (ok) return;
+    std::fprintf(stderr, "check failed: %s\n", what.c_str());
+    std::exit(1);
+}
+
+// The status of the Error that f throws, 0 when it returns.
+template <class F>
+int status_of(F &&f) {
+    try {
+        f();
+    } catch (const Error &e) {
+        return e.status;
+    }
+    return 0;
+}
+
+GptConfig shape(size_t W, size_t H, size_t C, size_t L = 2, size_t A = 4, size_t F = 6) {
+    GptConfig c;
+    c.vocab_size = 64;
+    c.context = C;
+    c.width = W;
+    c.heads = H;
+    c.layers = L;
+    c.attention_mesh_depth = A;
+    c.ffn_mesh_depth = F;
+    return c;
+}
+
+void generate(MeshGpt &m, size_t batch, size_t prompt, size_t count, float temperature = 0.0f) {
+    const std::vector<uint32_t> prompts(batch * prompt, 1);
+    std::vector<uint32_t> out(batch * (prompt + count));
+    m.generate_tokens(prompts.data(), batch, prompt, count, temperature, 7, out.data());
+}
+
+// Programs that between them take each route.
+std::vector<std::pair<const char *, std::function<void()>>> programs() {
+    return {
+        {"window", [] {
+             MeshGpt m(0, shape(32, 4, 32), 7, 2);
+             generate(m, 2, 5, 60);
+         }},
+        {"long prefill", [] {
+             MeshGpt m(0, shape(128, 2, 330), 7, 8);
+             const std::vector<uint32_t> prompts(8 * 300, 1);
+             m.prefill(prompts.data(), 8, 300, 0.0f, 7, 320);
+             m.decode(2);
+             std::vector<uint32_t> out(8 * 300);
+             m.read_tokens(out.data(), 8, 300);
+         }},
+        {"decode", [] {
+             setenv("MG_DISABLE_PERSISTENT", "1", 1);
+             MeshGpt m(0, shape(128, 4, 256), 7, 64);
+             generate(m, 64, 16, 20);
+             unsetenv("MG_DISABLE_PERSISTENT");
+         }},
+        {"logits", [] {
+             MeshGpt m(0, shape(64, 4, 64), 7);
+             const std::vector<uint32_t> tokens(1024, 1);
+             std::vector<float> out(1024 * 64);
+             for (size_t sequence : {4, 32, 64}) m.logits(tokens.data(), 1024, sequence, false, out.data(), out.size());
+             m.hidden_states(tokens.data(), 1024, 64, out.data(), out.size());
+         }},
+        {"training", [] {
+             for (size_t W : {32, 256}) {
+                 MeshGpt m(0, shape(W, 4, 64), 7);
+                 const std::vector<uint32_t> tokens(256, 1);
+                 for (size_t sequence : {4, 32, 64}) m.train_batch(tokens.data(), tokens.data(), 256, sequence, {});
+             }
+         }},
+        {"sampler", [] {
+             for (size_t V : {64, 1000, 50000}) {
+                 const std::vector<float> logits(2 * V, 0.0f);
+                 uint64_t rng[2] = {1, 2};
+                 uint32_t tokens[2];
+                 sample_logits(0, logits.data(), 2, V, 0.5f, rng, tokens);
+             }
+         }},
+    };
+}
+
+// A launch that the runtime refuses is reported by the call that made it, for
+// every kernel that the programs launch.
+void refused_launches() {
+    for (const auto &program : programs()) {
+        std::set<std::string> kernels;
+        fake::on_launch = [&](const fake::Launch &l) { kernels.insert(l.kernel); };
+        program.second();
+        fake::on_launch = nullptr;
+        expect(!kernels.empty(), std::string(program.first) + " launches kernels");
+        for (const std::string &k : kernels) {
+            fake::refuse = k;
+            expect(status_of(program.second) == kDeviceError, std::string(program.first) + " reports a refused " + k);
+            fake::refuse.clear();
+        }
+        expect(status_of(program.second) == 0, std::string(program.first) + " runs after refusals");
+    }
+    // Windows that need more LDS than a launch has unasked.
+    MeshGpt m(0, shape(128, 4, 32, 2), 7, 1);
+    fake::refuse_attributes = true;
+    expect(status_of([&] { generate(m, 1, 30, 40); }) == kDeviceError, "a refused LDS size is reported");
+    fake::refuse_attributes = false;
+    expect(status_of([&] { generate(m, 1, 30, 40); }) == 0, "and the model goes on");
+}
+
+// An error that a program's own HIP calls left on the thread, or an allocation
+// that failed and was reported, is no launch error of the next call.
+void foreign_errors() {
+    for (const auto &program : programs()) {
+        void *p = nullptr;
+        (void)hipMalloc(&p, size_t(1) << 50);
+        expect(status_of(program.second) == 0, std::string(program.first) + " after a foreign error");
+    }
+    MeshGpt m(0, shape(32, 4, 32), 7, 1);
+    fake::memory = 0;
+    expect(status_of([&] { generate(m, 100000, 5, 8); }) == kOutOfMemory, "no memory for a batch");
+    fake::memory = size_t(1) << 33;
+    expect(status_of([&] { generate(m, 1, 5, 8); }) == 0, "a smaller batch after it");
+}
+
+const std::map<std::string, void (*)()> kChecks = {
+    {"refused_launches", refused_launches},
+    {"foreign_errors", foreign_errors},
+};
+
+}  // namespace
+
+int main(int argc, char **argv) {
+    const auto check = kChecks.find(argc > 1 ? argv[1] : "");
+    if (check == kChecks.end()) {
+        for (const auto &c : kChecks) std::puts(c.first.c_str());
+        return 2;
+    }
+    check->second();
+    std::puts("ok");
+}
