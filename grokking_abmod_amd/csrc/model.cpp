@@ -1434,15 +1434,17 @@ struct MeshGpt::Impl {
     // Whether tokens can be generated from whole windows in one launch.
     bool window_usable() const { return use_window && kern::window_supported(shape, cfg.context); }
 
-    // `steps` generated tokens, each from its whole window (kern::window_generate).
+    // `steps` generated tokens, each from its whole window (kern::window_generate),
+    // in launches of kern::window_steps() tokens (MG_WINDOW_STEPS overrides it).
     // Where the last of them still fits the context, the cache is left as a
     // decode to that length leaves it.
     void window(size_t steps) {
         if (length + steps > tcap) throw Error("generation exceeds the reserved token capacity");
         known_flags = -1;
-        constexpr size_t kLaunchSteps = 4096;  // bounds a launch to some tens of milliseconds
+        const int forced = env_int("MG_WINDOW_STEPS", 0);
+        const size_t most = forced > 0 ? size_t(forced) : kern::window_steps(shape, cfg.context, cfg.layers, batch);
         for (size_t done = 0; done < steps;) {
-            const size_t n = std::min(steps - done, kLaunchSteps), before = length + n - 1;
+            const size_t n = std::min(steps - done, most), before = length + n - 1;
             const bool keep = done + n == steps && before <= cfg.context;
             kern::WindowArgs a{};
             a.E = E.as<float>();

@@ -138,7 +138,30 @@ void foreign_errors() {
     expect(status_of([&] { generate(m, 1, 5, 8); }) == 0, "a smaller batch after it");
 }
 
+// No launch of whole windows holds the GPU for long: 50 ms at 1 us for a layer
+// of a stack, or five for its block's attention, and a round of 256 sequences
+// (the most that a window of 64 rows of 128 channels takes).
+void window_launches() {
+    for (size_t layers : {1, 2, 12, 40})
+        for (size_t depth : {1, 6, 14})
+            for (size_t batch : {1, 300, 1024}) {
+                MeshGpt m(0, shape(128, 4, 64, layers, depth, depth), 7, 1);
+                size_t steps = 0;
+                fake::on_launch = [&](const fake::Launch &l) {
+                    if (l.kernel.find("window_kernel") == std::string::npos) return;
+                    const auto *a = static_cast<const kern::WindowArgs *>(l.args[0]);
+                    const double us = double(a->steps) * double((batch + 255) / 256) * double(layers) * double(5 * depth + 5);
+                    expect(a->steps == 1 || us <= 50000.0, "a launch of " + std::to_string(us) + " us");
+                    steps += size_t(a->steps);
+                };
+                generate(m, batch, 64, 5000);
+                fake::on_launch = nullptr;
+                expect(steps == 4999 || steps == 5000, "every token past the context from a window");
+            }
+}
+
 const std::map<std::string, void (*)()> kChecks = {
+    {"window_launches", window_launches},
     {"refused_launches", refused_launches},
     {"foreign_errors", foreign_errors},
 };

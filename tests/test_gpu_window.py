@@ -73,6 +73,28 @@ def test_decode_continues_a_window_generation(monkeypatch):
         assert np.array_equal(model.generate_tokens(prompts, 20, 0.7, 7), whole)
 
 
+@pytest.mark.parametrize("temperature", [0.0, 0.7])
+@pytest.mark.parametrize("count", [20, 60])
+@pytest.mark.parametrize("cfg", [dict(width=32, heads=4, context=32), dict(width=128, heads=2, context=40)],
+                         ids=["W32", "W128"])
+def test_a_generation_in_several_launches(cfg, count, temperature, monkeypatch):
+    """Launches of 7 tokens give one launch's tokens, logits and state, inside the
+    context (from which decode goes on) and past it."""
+    prompts = G.random_prompts(40, 3, 5, 7)
+    got = []
+    for steps in ("0", "7"):
+        monkeypatch.setenv("MG_WINDOW_STEPS", steps)
+        monkeypatch.setenv("MG_DISABLE_PERSISTENT", "1")
+        with G.MeshGpt(0, G.GptConfig(vocab_size=40, layers=2, **cfg), 7, max_batch=3) as model:
+            model.prefill(prompts, temperature, 7, reserve=70)
+            tokens = model.generate_tokens(prompts, count, temperature, 7)
+            last = model.last_logits(3)
+            if count == 20:
+                model.decode(6)
+            got.append((tokens, last, model.read_tokens(3), model.last_logits(3)))
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
 def test_window_generation_reports_nonfinite_logits():
     cfg = dict(vocab_size=28, context=16, width=32, heads=4, layers=1)
     o = O.config(**cfg)
