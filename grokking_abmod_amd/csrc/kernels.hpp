@@ -273,8 +273,8 @@ struct WindowArgs {
     float scale_log2;     // set by window_generate
 };
 bool window_supported(const Shape &s, size_t context);
-// Tokens of one launch: as many as take some 20 ms, at least one.
-size_t window_steps(const Shape &s, size_t context, size_t layers, size_t batch);
+// The time of a token of a batch, estimated from its size (us).
+double window_us(const Shape &s, size_t context, size_t layers, size_t batch, size_t vocab);
 void window_generate(const Shape &s, WindowArgs a, int batch, hipStream_t stream);
 // Greedy / temperature sampling from logits rows; appends the token and bumps len.
 void sample(int V, int batch, const float *logits, float temperature, uint64_t *rng, uint32_t *tokens,

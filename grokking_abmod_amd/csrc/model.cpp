@@ -1434,15 +1434,43 @@ struct MeshGpt::Impl {
     // Whether tokens can be generated from whole windows in one launch.
     bool window_usable() const { return use_window && kern::window_supported(shape, cfg.context); }
 
+    // Whether they are, against the cached decode inside the context and a
+    // prefill a token past it.  What the three take is estimated (us a token):
+    // the decode by its launches (two a block) for up to some 300 sequences and
+    // by its rows from there on, the prefill by its launches, mesh layers and
+    // rows.  Measured (window; other): W32, context 64, two blocks of 22 layers,
+    // 128 sequences 11; 85.  W128, context 64, the same: 16 sequences 37; 37, 128
+    // 38; 80, 512 75; 84, 1024 148; 123, 4096 589; 414.  Twelve blocks: 16 259; 142,
+    // 128 260; 212.  W64, six blocks of 45 layers: 128 88; 140, 512 176; 150, 1024
+    // 352; 260.  Past the context the windows lose only where a prefill runs on
+    // the matrix cores and the stacks are deep (W128, twelve blocks of 45 layers:
+    // 16 572; 507, 256 582; 776, 1024 2289; 2223; six: 4096 4464; 4132).
+    double window_us() const { return kern::window_us(shape, cfg.context, cfg.layers, batch, cfg.vocab_size); }
+    double decode_us() const {
+        const double row = 0.00026 * shape.W + 0.004 * (shape.H - 4) + 0.0005 * (4 * shape.A + shape.F);
+        return batch < 64 ? 20.0 + 11.0 * double(cfg.layers)
+                          : 30.0 + double(cfg.layers) * std::max(18.0, std::max(0.041, row) * double(batch));
+    }
+    double prefill_us() const {
+        const double stack_layers = double(4 * shape.A + shape.F);
+        return double(cfg.layers) * (20.0 + 0.5 * stack_layers + double(batch) * (0.095 + 0.00125 * stack_layers));
+    }
+    bool window_inside(size_t tokens) const {
+        return double(tokens) * window_us() <= prefill_us() + double(tokens - 1) * decode_us();
+    }
+    bool window_past() const {
+        return !kern::attn_prefill_mfma_supported(shape, int(cfg.context)) || 1.04 * window_us() <= prefill_us();
+    }
+
     // `steps` generated tokens, each from its whole window (kern::window_generate),
-    // in launches of kern::window_steps() tokens (MG_WINDOW_STEPS overrides it).
+    // in launches of some 10 ms (MG_WINDOW_STEPS: of that many tokens).
     // Where the last of them still fits the context, the cache is left as a
     // decode to that length leaves it.
     void window(size_t steps) {
         if (length + steps > tcap) throw Error("generation exceeds the reserved token capacity");
         known_flags = -1;
         const int forced = env_int("MG_WINDOW_STEPS", 0);
-        const size_t most = forced > 0 ? size_t(forced) : kern::window_steps(shape, cfg.context, cfg.layers, batch);
+        const size_t most = forced > 0 ? size_t(forced) : size_t(std::max(1.0, 10000.0 / window_us()));
         for (size_t done = 0; done < steps;) {
             const size_t n = std::min(steps - done, most), before = length + n - 1;
             const bool keep = done + n == steps && before <= cfg.context;
@@ -1698,19 +1726,25 @@ void MeshGpt::generate_tokens(const uint32_t *prompts, size_t batch, size_t prom
     // (window.hip).  A shape that the persistent decode takes as well uses it
     // up to the context: its token is one row's work against a window's (W128,
     // two blocks, context 32: 7.6 us a token against 16).
-    const bool window = m.window_usable();
-    if (count > 0 && !(window && !m.persistent_usable())) {
+    // Tokens past the context, and inside it where that is estimated to be
+    // faster, come from windows.
+    const bool window = m.window_usable(), persistent = m.persistent_usable(), past = window && m.window_past();
+    const size_t room = m.length <= m.cfg.context ? m.cfg.context + 1 - m.length : 0;
+    const size_t inside = window ? std::min(count, room) : count;
+    if (count > 0 && !(window && !persistent && (inside > 0 ? m.window_inside(inside) : past))) {
         m.step();  // the prompt's prefill and the first token
         ++done;
     }
-    const size_t room = m.length <= m.cfg.context ? m.cfg.context + 1 - m.length : 0;
-    const size_t inside = window ? std::min(count - done, room) : count - done;
-    if (done > 0 && inside > 0 && m.decodable(inside) && m.persistent_usable() && m.persistent_preferred(inside) &&
-        m.persistent(inside))
-        done += inside;
-    if (window && done < count) {
-        m.window(count - done);
-        done = count;
+    if (const size_t rest = done > 0 && inside > done ? inside - done : 0) {
+        if (persistent && m.decodable(rest) && m.persistent_preferred(rest) && m.persistent(rest))
+            done += rest;
+        else if (window && !m.window_inside(rest))
+            for (; done < inside; ++done) m.step();
+    }
+    if (window && done < count && (past || done < inside)) {
+        const size_t n = (past ? count : inside) - done;
+        m.window(n);
+        done += n;
     }
     for (; done < count; ++done) m.step();
     m.read_tokens(out, batch, prompt_len + count, true);

@@ -23,7 +23,6 @@
 // 21.7 and 3.9; W128, context 64: 17.3 and 9.5.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -459,11 +458,16 @@ __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
     }
 }
 
+// Bytes of LDS of a workgroup of `waves` waves, and of the weights and token
+// vectors that it may hold beside them.
+size_t window_lds(int W, int waves) { return (3 * 4 * size_t(waves) * (W + 4) + 16 + W + 256 + kRing) * 4 + 32 * 8; }
+size_t window_weights(const Shape &s, size_t layers, size_t vocab) {
+    return (layers * 2 * s.W * (4 * s.A + s.F) + vocab * s.W) * 4;
+}
+
 template <int CPL, int HD, int NW>
-void launch_window(const WindowArgs &a, int batch, hipStream_t stream) {
-    constexpr size_t W = 16 * CPL;
-    const size_t lds = (3 * 4 * NW * (W + 4) + 16 + W + 256 + kRing) * 4 + 32 * 8;
-    const size_t staged = (size_t(a.L) * 2 * W * (4 * a.A + a.F) + size_t(a.V) * W) * 4;
+void launch_window(const Shape &s, const WindowArgs &a, int batch, hipStream_t stream) {
+    const size_t lds = window_lds(16 * CPL, NW), staged = window_weights(s, size_t(a.L), size_t(a.V));
     auto launch = [&](auto kernel, size_t bytes) {
         // A refusal is the thread's last error, which the model's next wait reports.
         if (bytes > 65536 && hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -516,24 +520,23 @@ bool window_supported(const Shape &s, size_t context) {
     return context <= size_t(kWindowRows) && s.V <= 256 && s.hd == s.hdp && by_window_shape(s, [](auto, auto) {});
 }
 
-// An upper estimate of a token's time: rounds of one workgroup a CU (256), and
-// for each layer of each stack, with eight more a block for the attention, 0.15
-// us and 0.1 for each 1024 values of the window.  Measured, without the eight, a
-// layer: 0.18 us for 32 rows of 32 channels, 0.27 for 64 of 32, 0.38 for 64 of
-// 64 and 32 of 128, 0.9 for 64 of 128 (four and six layers a stack, one to 256
-// sequences).
-size_t window_steps(const Shape &s, size_t context, size_t layers, size_t batch) {
-    const double rounds = double((batch + 255) / 256), stack_layers = double(layers) * double(4 * s.A + s.F + 8);
-    const double us = rounds * stack_layers * (0.15 + 0.1 * double(context) * s.W / 1024.0);
-    return size_t(std::max(1.0, 20000.0 / us));
+// Workgroups run 256 at a time, a CU's LDS or wave slots each (windows of up to
+// 32 narrow rows overlap somewhat), and a layer of a stack takes the time below;
+// the last block works for one row past its keys.  Measured between one and
+// twelve blocks, stacks of 4 to 9 layers and 16 to 4096 sequences: within 15 %
+// wherever another route comes near.
+double window_us(const Shape &s, size_t context, size_t layers, size_t batch, size_t vocab) {
+    const bool wide = context > kWindowRows / 2, staged = !wide && window_lds(s.W, 8) + window_weights(s, layers, vocab) <= kWindowLds;
+    const double layer = s.W == 32 ? (wide ? 0.22 : 0.15) : s.W == 64 ? (wide ? 0.335 : 0.22) : wide ? 1.03 : staged ? 0.33 : 0.53;
+    return double((batch + 255) / 256) * (double(layers) - 0.33) * double(4 * s.A + s.F) * layer;
 }
 
 void window_generate(const Shape &s, WindowArgs a, int batch, hipStream_t stream) {
     a.scale_log2 = float(1.4426950408889634 / std::sqrt(double(s.hd)));
     by_window_shape(s, [&](auto cpl, auto hd) {
         constexpr int C = decltype(cpl)::value, D = decltype(hd)::value;
-        a.context <= kWindowRows / 2 ? launch_window<C, D, 8>(a, batch, stream)
-                                     : launch_window<C, D, 16>(a, batch, stream);
+        a.context <= kWindowRows / 2 ? launch_window<C, D, 8>(s, a, batch, stream)
+                                     : launch_window<C, D, 16>(s, a, batch, stream);
     });
 }
 

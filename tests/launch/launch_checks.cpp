@@ -145,7 +145,7 @@ void window_launches() {
     for (size_t layers : {1, 2, 12, 40})
         for (size_t depth : {1, 6, 14})
             for (size_t batch : {1, 300, 1024}) {
-                MeshGpt m(0, shape(128, 4, 64, layers, depth, depth), 7, 1);
+                MeshGpt m(0, shape(128, 8, 64, layers, depth, depth), 7, 1);
                 size_t steps = 0;
                 fake::on_launch = [&](const fake::Launch &l) {
                     if (l.kernel.find("window_kernel") == std::string::npos) return;
@@ -160,7 +160,48 @@ void window_launches() {
             }
 }
 
+// The route of tokens inside and past the context, by what each was measured to
+// take where the persistent decode does not run: 'w' a window, 'c' the cached
+// decode, 'p' a prefill a token.
+void window_routes() {
+    struct Case {
+        size_t W, H, C, L, A, F, batch;
+        char inside, past;
+    };
+    const Case cases[] = {
+        {32, 4, 64, 2, 4, 6, 4096, 'w', 'w'},  {32, 4, 32, 12, 9, 9, 16, 'w', 'w'},   {64, 4, 64, 2, 4, 6, 1024, 'w', 'w'},
+        {64, 4, 64, 6, 9, 9, 128, 'w', 'w'},   {64, 4, 64, 6, 9, 9, 1024, 'c', 'w'},  {64, 4, 64, 12, 9, 9, 16, 'c', 'w'},
+        {128, 4, 32, 2, 4, 6, 1024, 'w', 'w'}, {128, 4, 32, 12, 9, 9, 16, 'c', 'w'},  {128, 4, 32, 12, 9, 9, 512, 'c', 'w'},
+        {128, 4, 64, 2, 4, 6, 128, 'w', 'w'},  {128, 4, 64, 2, 4, 6, 512, 'w', 'w'},  {128, 4, 64, 2, 4, 6, 4096, 'c', 'w'},
+        {128, 4, 64, 12, 4, 6, 16, 'c', 'w'},  {128, 4, 64, 12, 4, 6, 256, 'c', 'w'}, {128, 4, 64, 12, 9, 9, 16, 'c', 'p'},
+        {128, 8, 64, 12, 9, 9, 16, 'c', 'w'},  {128, 4, 48, 12, 9, 9, 16, 'c', 'w'},  {128, 4, 64, 12, 9, 9, 256, 'c', 'w'},
+    };
+    setenv("MG_DISABLE_PERSISTENT", "1", 1);
+    for (const Case &c : cases) {
+        MeshGpt m(0, shape(c.W, c.H, c.C, c.L, c.A, c.F), 7, c.batch);
+        size_t windows = 0;
+        fake::on_launch = [&](const fake::Launch &l) {
+            if (l.kernel.find("window_kernel") != std::string::npos)
+                windows += size_t(static_cast<const kern::WindowArgs *>(l.args[0])->steps);
+        };
+        const std::string what = "W" + std::to_string(c.W) + " context " + std::to_string(c.C) + " batch " +
+                                 std::to_string(c.batch) + " blocks " + std::to_string(c.L) + " stacks of " +
+                                 std::to_string(c.A);
+        generate(m, c.batch, 4, c.C - 4);
+        expect(windows == (c.inside == 'w' ? c.C - 4 : 0), what + ": inside the context");
+        windows = 0;
+        generate(m, c.batch, c.C + 1, 3);
+        expect(windows == (c.past == 'w' ? 3 : 0), what + ": past the context");
+        windows = 0;
+        generate(m, c.batch, c.C - 3, 9);  // four tokens inside the context
+        expect(windows >= (c.past == 'w' ? 5u : 0u) && windows <= (c.past == 'w' ? 9u : 4u), what + ": across it");
+        fake::on_launch = nullptr;
+    }
+    unsetenv("MG_DISABLE_PERSISTENT");
+}
+
 const std::map<std::string, void (*)()> kChecks = {
+    {"window_routes", window_routes},
     {"window_launches", window_launches},
     {"refused_launches", refused_launches},
     {"foreign_errors", foreign_errors},

@@ -95,6 +95,22 @@ def test_a_generation_in_several_launches(cfg, count, temperature, monkeypatch):
     assert all(np.array_equal(a, b) for a, b in zip(*got))
 
 
+@pytest.mark.parametrize("cfg,count", [(dict(width=32, heads=4, context=32), 40),
+                                       (dict(width=128, heads=4, context=64, attention_mesh_depth=9), 75)],
+                         ids=["windows", "decode-then-windows"])
+def test_more_sequences_than_workgroups_run_at_once(cfg, count):
+    """A sequence's tokens are its own in a batch that takes three rounds, from
+    windows alone and from the cached decode up to the context."""
+    kw = dict(vocab_size=40, layers=2, **cfg)
+    g, o = G.GptConfig(**kw), O.config(**kw)
+    params = O.initialize(o, 7)
+    prompts = G.random_prompts(40, 600, 5, 7)
+    with G.MeshGpt(0, g, 7, max_batch=600) as model:
+        got = model.generate_tokens(prompts, count, 0.7, 7)
+        for b in (0, 255, 256, 599):
+            check_trajectory(o, params, prompts[b], got[b], 0.7, 7 + b, _last(model), cached=False)
+
+
 def test_window_generation_reports_nonfinite_logits():
     cfg = dict(vocab_size=28, context=16, width=32, heads=4, layers=1)
     o = O.config(**cfg)
