@@ -1081,6 +1081,11 @@ struct MeshGpt::Impl {
                 c.ma = ma;
                 c.mf = mf;
                 c.dx = dx;
+                c.table = table;
+                c.sequence = seq;
+                c.H = H;
+                c.norm = cfg.qk_norm;
+                c.rotate = cfg.rope;
                 if (b == L) {
                     c.dn = dn;
                     c.x_last = X(L);
@@ -1102,11 +1107,6 @@ struct MeshGpt::Impl {
                     c.n1 = at(k.n1);
                     c.x_below = X(b);
                     c.inv1 = at(k.inv1);
-                    c.table = table;
-                    c.sequence = seq;
-                    c.H = H;
-                    c.norm = cfg.qk_norm;
-                    c.rotate = cfg.rope;
                 }
                 if (b > 0) {
                     const TrainBlock &k = p.blocks[b - 1];

@@ -200,7 +200,24 @@ void window_routes() {
     unsetenv("MG_DISABLE_PERSISTENT");
 }
 
+// Every launch of the training chain has the shape that its kernel divides by.
+void chain_shapes() {
+    MeshGpt m(0, shape(128, 4, 32, 3), 7);
+    size_t launches = 0;
+    fake::on_launch = [&](const fake::Launch &l) {
+        if (l.kernel.find("backward_chain_kernel") == std::string::npos) return;
+        const auto *a = static_cast<const kern::train::BackwardChain *>(l.args[0]);
+        expect(a->H == 4 && a->sequence == 32 && a->rows == 64 && a->ma.W == 128, "a launch's shape");
+        ++launches;
+    };
+    const std::vector<uint32_t> tokens(64, 1);
+    m.train_batch(tokens.data(), tokens.data(), 64, 32, {});
+    fake::on_launch = nullptr;
+    expect(launches == 4, "one launch before, between and after three blocks");
+}
+
 const std::map<std::string, void (*)()> kChecks = {
+    {"chain_shapes", chain_shapes},
     {"window_routes", window_routes},
     {"window_launches", window_launches},
     {"refused_launches", refused_launches},
