@@ -48,6 +48,16 @@ struct DevBuf {
         bytes = std::max<size_t>(n, 256);
         return true;
     }
+    // The same where the caller can do without; false when there is no memory.
+    bool try_ensure(size_t n) {
+        try {
+            ensure(n);
+        } catch (const Error &e) {
+            if (e.status != kOutOfMemory) throw;
+            return false;
+        }
+        return true;
+    }
     template <class T>
     T *as() const {
         return static_cast<T *>(p);
@@ -593,9 +603,9 @@ struct MeshGpt::Impl {
                                   kern::attn_prefill_mfma_supported(shape, rows.rows_per_seq);
         // Long sequences: split FP16 operands for the (sequence, head) pairs
         // whose values allow it (MG_DISABLE_SPLIT_PREFILL=1 keeps FP32).
-        const bool split_prefill =
-            mfma_prefill && use_split_prefill && kern::attn_split_supported(shape, rows.rows_per_seq);
-        if (split_prefill) wsplit.ensure(kern::attn_split_bytes(shape, nseq, rows.rows_per_seq));
+        const bool split_prefill = mfma_prefill && use_split_prefill &&
+                                   kern::attn_split_supported(shape, rows.rows_per_seq) &&
+                                   wsplit.try_ensure(kern::attn_split_bytes(shape, nseq, rows.rows_per_seq));
         // Short sequences: one thread per (row, head) (MG_DISABLE_SHORT_PREFILL=1
         // keeps the VALU flash kernel).
         const bool short_prefill = !decode && use_short_prefill &&
@@ -609,13 +619,14 @@ struct MeshGpt::Impl {
         // gather and the merge) against that block's attention and half of its
         // meshes for every other row.
         const int n = rows.rows_per_seq;
-        const bool compact = last && !decode && rows_prefill && mfma_prefill && last_row_pays(rows.rows);
-        const int last_split = compact ? splits_for(size_t(nseq)) : 0;
+        const size_t row = size_t(nseq) * cfg.width;
+        const int last_split = last ? splits_for(size_t(nseq)) : 0;
+        const bool compact =
+            last && !decode && rows_prefill && mfma_prefill && last_row_pays(rows.rows) &&
+            wlast.try_ensure((3 * row + size_t(nseq) * (cfg.heads * size_t(last_split) * (shape.hdp + 2) + 1)) * 4);
         float *last_q = nullptr, *last_x = nullptr, *last_y = nullptr, *last_part = nullptr;
         int *last_len = nullptr;
         if (compact) {
-            const size_t row = size_t(nseq) * cfg.width;
-            wlast.ensure((3 * row + size_t(nseq) * (cfg.heads * size_t(last_split) * (shape.hdp + 2) + 1)) * 4);
             last_q = wlast.as<float>();
             last_x = last_q + row;
             last_y = last_x + row;

@@ -1,5 +1,6 @@
 #include "fake_hip.hpp"
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -8,7 +9,7 @@ namespace fake {
 std::function<void(const Launch &)> on_launch;
 std::string refuse;
 bool refuse_attributes = false;
-size_t memory = size_t(1) << 33;
+size_t memory = size_t(1) << 33, peak = 0;
 }  // namespace fake
 
 namespace {
@@ -103,6 +104,7 @@ hipError_t hipMalloc(void **p, size_t n) {
     *p = std::calloc(n, 1);
     blocks()[*p] = n;
     used += n;
+    fake::peak = std::max(fake::peak, used);
     return hipSuccess;
 }
 hipError_t hipFree(void *p) {

@@ -23,7 +23,7 @@ extern std::function<void(const Launch &)> on_launch;
 extern std::string refuse;
 // hipFuncSetAttribute fails.
 extern bool refuse_attributes;
-// Device bytes there are; hipMalloc fails past them.
-extern size_t memory;
+// Device bytes there are (hipMalloc fails past them) and the most in use so far.
+extern size_t memory, peak;
 
 }  // namespace fake

@@ -216,7 +216,41 @@ void chain_shapes() {
     expect(launches == 4, "one launch before, between and after three blocks");
 }
 
+// A prefill that fits without the split attention's planes, or without the last
+// rows' buffers, runs without them where there is no memory for them.
+void scratch_limits() {
+    const std::vector<uint32_t> prompts(8 * 600, 1);
+    std::set<std::string> kernels;
+    auto prefill = [&] {
+        MeshGpt m(0, shape(256, 4, 640), 7, 8);
+        kernels.clear();
+        fake::on_launch = [&](const fake::Launch &l) { kernels.insert(l.kernel); };
+        m.prefill(prompts.data(), 8, 600, 0.0f, 7, 620);
+        m.decode(2);
+        fake::on_launch = nullptr;
+    };
+    auto launched = [&](const char *name) {
+        for (const std::string &k : kernels)
+            if (k.find(name) != std::string::npos) return true;
+        return false;
+    };
+    prefill();
+    expect(launched("attn_split_kernel") && launched("last_merge_kernel"), "both where there is memory");
+    setenv("MG_DISABLE_SPLIT_PREFILL", "1", 1);
+    fake::peak = 0;
+    prefill();
+    unsetenv("MG_DISABLE_SPLIT_PREFILL");
+    fake::memory = fake::peak;
+    expect(status_of(prefill) == 0, "a prefill in the memory that it took without planes");
+    expect(!launched("attn_split_kernel") && launched("attn_prefill_mfma_kernel"), "on the FP32 kernel");
+    fake::memory -= 3 * 8 * 256 * 4;  // less than the last rows' buffers take
+    expect(status_of(prefill) == 0, "a prefill without the last rows' buffers");
+    expect(!launched("last_merge_kernel"), "with every row in the last block");
+    fake::memory = size_t(1) << 33;
+}
+
 const std::map<std::string, void (*)()> kChecks = {
+    {"scratch_limits", scratch_limits},
     {"chain_shapes", chain_shapes},
     {"window_routes", window_routes},
     {"window_launches", window_launches},
