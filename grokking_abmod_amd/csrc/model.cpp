@@ -178,7 +178,7 @@ struct MeshGpt::Impl {
     bool use_split_prefill = true;
     bool use_short_prefill = true;
     bool use_window = true;
-    bool use_chain = true;
+    bool use_chain = true, force_chain = false;
 
     // Training (gpu.rs:1915-2003): the activations of the last forward, the
     // gradient, AdamW's moments and the running powers of its betas (reset
@@ -349,6 +349,7 @@ struct MeshGpt::Impl {
         use_rows_prefill = env_int("MG_DISABLE_ROWS_PREFILL", 0) == 0;
         use_window = env_int("MG_DISABLE_WINDOW", 0) == 0;
         use_chain = env_int("MG_DISABLE_TRAIN_CHAIN", 0) == 0;
+        force_chain = env_int("MG_FORCE_TRAIN_CHAIN", 0) != 0;
         use_short_prefill = env_int("MG_DISABLE_SHORT_PREFILL", 0) == 0;
 
         const size_t C = cfg.context;
@@ -979,7 +980,7 @@ struct MeshGpt::Impl {
         }
         auto X = [&](int b) { return at(p.x) + size_t(b) * RW; };
         auto last = [&](size_t o, int depth) { return at(o) + size_t(depth - 1) * RW; };
-        const bool chain = use_chain && T::chain_fits(ma, mf, H);
+        const bool chain = use_chain && T::chain_fits(ma, mf, H) && (force_chain || T::chain_pays(ma, mf, R));
         auto attend = [&](int b) {
             const TrainBlock &k = p.blocks[b];
             T::attention_forward(at(k.qr), at(k.kr), last(k.vs, A), at(k.y), at(k.z), at(k.lse), R, seq, W, H,

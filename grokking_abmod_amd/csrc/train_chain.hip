@@ -426,6 +426,22 @@ bool chain_fits(const Mesh &ma, const Mesh &mf, int H) {
     return hd >= 2 && hd <= 64 && (hd & (hd - 1)) == 0 && by_chain_shape(ma, mf, [](auto, auto, auto) {});
 }
 
+// Against the separate launches, an AdamW update (us, chain and separate).  Few
+// rows and shallow stacks gain the launches: W64, four layers and six, 256 rows
+// 130 and 138, 4096 220 and 237.  A wave takes its rows one after another, so
+// the gain is gone where every SIMD has several: W128, 4096 rows 307 and 321,
+// 8192 507 and 504, 16384 844 and 820; W32 neighbour 8192 310 and 317, butterfly
+// 16384 513 and 497.  Butterfly strides cost the shuffles of W128 more than the
+// launches of few rows (256 rows 181 and 175, 1024 204 and 209), and the stacks
+// of up to eight layers, whose sums fill the registers, gain in between only (W64,
+// seven layers: 512 159 and 155, 2048 197 and 205, 6144 336 and 334; butterfly 2048
+// 210 and 208).
+bool chain_pays(const Mesh &ma, const Mesh &mf, int rows) {
+    if (ma.depth > 4) return !ma.butterfly && rows >= 1536 && rows <= 4096;
+    if (ma.W > 64) return rows <= 4096 && !(ma.butterfly && rows < 512);
+    return rows <= 8192;
+}
+
 void forward_chain(const ForwardChain &a, hipStream_t stream) {
     by_chain_shape(a.ma, a.mf, [&](auto C, auto A, auto F) {
         hipLaunchKernelGGL((forward_chain_kernel<decltype(C)::value, decltype(A)::value, decltype(F)::value>),

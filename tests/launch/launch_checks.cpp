@@ -249,7 +249,32 @@ void scratch_limits() {
     fake::memory = size_t(1) << 33;
 }
 
+// The training chain is taken for the row counts at which it was measured faster.
+void chain_routes() {
+    struct Case {
+        size_t W, A, F, rows;
+        bool butterfly, chain;
+    };
+    const Case cases[] = {{32, 4, 6, 256, false, true},     {64, 4, 6, 8192, true, true},    {32, 4, 6, 16384, true, false},
+                          {128, 4, 6, 64, false, true},     {128, 4, 6, 2048, true, true},   {128, 4, 6, 256, true, false},
+                          {128, 4, 6, 16384, false, false}, {64, 7, 7, 256, false, false},   {64, 7, 7, 2048, false, true},
+                          {64, 7, 7, 2048, true, false},    {64, 7, 7, 16384, false, false}, {128, 5, 5, 2048, false, false}};
+    for (const Case &c : cases) {
+        GptConfig g = shape(c.W, 4, 32, 1, c.A, c.F);
+        g.connectivity = c.butterfly ? MeshConnectivity::Butterfly : MeshConnectivity::Neighbor;
+        MeshGpt m(0, g, 7);
+        bool chain = false;
+        fake::on_launch = [&](const fake::Launch &l) { chain |= l.kernel.find("chain_kernel") != std::string::npos; };
+        const std::vector<uint32_t> tokens(c.rows, 1);
+        m.train_batch(tokens.data(), tokens.data(), c.rows, 4, {});
+        fake::on_launch = nullptr;
+        expect(chain == c.chain, "W" + std::to_string(c.W) + ", " + std::to_string(c.A) + " layers, " +
+                                     std::to_string(c.rows) + " rows" + (c.butterfly ? ", butterfly" : ""));
+    }
+}
+
 const std::map<std::string, void (*)()> kChecks = {
+    {"chain_routes", chain_routes},
     {"scratch_limits", scratch_limits},
     {"chain_shapes", chain_shapes},
     {"window_routes", window_routes},

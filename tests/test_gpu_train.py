@@ -191,6 +191,7 @@ def test_chained_launches_give_the_separate_launches_bits(cfg, b, s, monkeypatch
     got = {}
     for off in ("0", "1"):
         monkeypatch.setenv("MG_DISABLE_TRAIN_CHAIN", off)
+        monkeypatch.setenv("MG_FORCE_TRAIN_CHAIN", "1")  # also where the separate launches are faster
         with G.MeshGpt(0, g, 7) as model:
             model.set_parameters(np.random.default_rng(3).uniform(
                 -1.0, 1.0, G.parameter_count(g)).astype(np.float32))
