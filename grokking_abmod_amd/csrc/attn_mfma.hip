@@ -4,8 +4,8 @@
 //
 // One workgroup takes 64 to 256 queries of one (sequence, head)
 // (attn_prefill_mfma chooses); each wave owns 16 or 32 of them (one or two
-// 16-query blocks).  Sequences of 288 rows or more run here only where
-// attn_split.hip cannot take them.  At 8192 rows eight waves share each K/V tile
+// 16-query blocks).  Long sequences run here only where attn_split.hip cannot
+// take them.  At 8192 rows eight waves share each K/V tile
 // among 256 queries and put four waves on every SIMD (two workgroups per CU, by
 // LDS): 23.69 ms a prefill against 23.95 with four waves (and 24.8 with 32-key
 // tiles, which let four workgroups share a CU).  Keys stream through LDS in

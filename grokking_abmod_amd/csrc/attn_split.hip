@@ -74,12 +74,6 @@ typedef __attribute__((address_space(3))) float lds_f32;
 constexpr float kXsaNormFloor = float(double(1e-12f) * double(1e-12f));
 
 constexpr int kBK = kSplitKeys;
-// Sequences of this many rows take the split kernels: writing the planes and the
-// launch that looks for pairs left to FP32 cost more than the faster products
-// gain below it (W512, 6 blocks, one prefill against the FP32 kernel: 8 x 256
-// rows 0.51 and 0.47 ms, 16 x 449 0.99 and 1.16; W1024, 12 blocks: 16 x 300
-// 2.21 and 2.32).
-constexpr int kSplitRows = 288;
 constexpr float kLowScale = 2048.0f;  // of v's second half
 constexpr float kQScale = 16384.0f, kKScale = 4096.0f, kScoreUnit = 1.0f / (16384.0f * 4096.0f);
 
@@ -411,8 +405,23 @@ attn_split_kernel(Shape s, const float *__restrict__ q, KvView kv, const _Float1
 
 }  // namespace
 
-bool attn_split_supported(const Shape &s, int rows_per_seq) {
-    return s.hd == s.hdp && (s.hd == 32 || s.hd == 64) && s.W % 4 == 0 && s.qk_norm && rows_per_seq >= kSplitRows;
+bool attn_split_supported(const Shape &s) {
+    return s.hd == s.hdp && (s.hd == 32 || s.hd == 64) && s.W % 4 == 0 && s.qk_norm;
+}
+
+// Writing the planes and the launch that looks for pairs left to FP32 cost some
+// 5 us a block, which the faster products gain back where there are enough of
+// them.  A forward against the FP32 kernel alone (us, W512, 6 blocks, head width
+// 64): 288 rows and 8 pairs 383 and 356, 96 498 and 471, 128 569 and 579; 350 rows
+// and 64 pairs 483 and 489, 96 574 and 619; 449 rows and 32 pairs 460 and 446, 64
+// 510 and 586; 576 rows and 8 pairs 453 and 464, 32 505 and 542.  Head width 32:
+// 384 rows and 64 pairs 388 and 375, 128 451 and 476; 449 rows and 16 pairs 364 and
+// 381.  8 x 256 rows 0.51 and 0.47 ms.
+bool attn_split_pays(const Shape &s, int nseq, int rows_per_seq) {
+    const int pairs = nseq * s.H;
+    if (rows_per_seq >= 576) return true;
+    if (rows_per_seq >= 448) return s.hd == 32 || pairs >= 64;
+    return pairs >= 128 ? rows_per_seq >= 288 : pairs >= 80 && rows_per_seq > 320;
 }
 
 size_t attn_split_bytes(const Shape &s, int nseq, int rows_per_seq) {

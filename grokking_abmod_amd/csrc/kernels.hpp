@@ -239,7 +239,9 @@ void attn_prefill_mfma(const Shape &s, const float *q, KvView kv, int nseq, int 
 // into two halves, at FP32 accuracy (attn_split.hip), in attn_split_bytes() of
 // scratch.  Pairs whose values span too wide a range for it are left to
 // attn_prefill_mfma, which takes the returned ranges.
-bool attn_split_supported(const Shape &s, int rows_per_seq);
+bool attn_split_supported(const Shape &s);
+// Whether it is faster for this many sequences of this many rows.
+bool attn_split_pays(const Shape &s, int nseq, int rows_per_seq);
 size_t attn_split_bytes(const Shape &s, int nseq, int rows_per_seq);
 const int2 *attn_split(const Shape &s, const float *q, KvView kv, int nseq, int rows_per_seq, float *y, int xsa,
                        void *scratch, hipStream_t stream);

@@ -175,7 +175,7 @@ struct MeshGpt::Impl {
     bool persistent_ok = false;
     bool use_mfma_prefill = true;
     bool use_rows_prefill = true;
-    bool use_split_prefill = true;
+    bool use_split_prefill = true, force_split = false;
     bool use_short_prefill = true;
     bool use_window = true;
     bool use_chain = true, force_chain = false;
@@ -346,6 +346,7 @@ struct MeshGpt::Impl {
         persistent_ok = row_decode && env_int("MG_DISABLE_PERSISTENT", 0) == 0;
         use_mfma_prefill = env_int("MG_DISABLE_MFMA_PREFILL", 0) == 0;
         use_split_prefill = env_int("MG_DISABLE_SPLIT_PREFILL", 0) == 0;
+        force_split = env_int("MG_FORCE_SPLIT_PREFILL", 0) != 0;
         use_rows_prefill = env_int("MG_DISABLE_ROWS_PREFILL", 0) == 0;
         use_window = env_int("MG_DISABLE_WINDOW", 0) == 0;
         use_chain = env_int("MG_DISABLE_TRAIN_CHAIN", 0) == 0;
@@ -605,7 +606,8 @@ struct MeshGpt::Impl {
         // Long sequences: split FP16 operands for the (sequence, head) pairs
         // whose values allow it (MG_DISABLE_SPLIT_PREFILL=1 keeps FP32).
         const bool split_prefill = mfma_prefill && use_split_prefill &&
-                                   kern::attn_split_supported(shape, rows.rows_per_seq) &&
+                                   kern::attn_split_supported(shape) &&
+                                   (force_split || kern::attn_split_pays(shape, nseq, rows.rows_per_seq)) &&
                                    wsplit.try_ensure(kern::attn_split_bytes(shape, nseq, rows.rows_per_seq));
         // Short sequences: one thread per (row, head) (MG_DISABLE_SHORT_PREFILL=1
         // keeps the VALU flash kernel).

@@ -61,12 +61,12 @@ std::vector<std::pair<const char *, std::function<void()>>> programs() {
              generate(m, 2, 5, 60);
          }},
         {"long prefill", [] {
-             MeshGpt m(0, shape(128, 2, 330), 7, 8);
-             const std::vector<uint32_t> prompts(8 * 300, 1);
-             m.prefill(prompts.data(), 8, 300, 0.0f, 7, 320);
+             MeshGpt m(0, shape(128, 2, 630), 7, 8);
+             const std::vector<uint32_t> prompts(8 * 600, 1);
+             m.prefill(prompts.data(), 8, 600, 0.0f, 7, 620);
              m.decode(2);
-             std::vector<uint32_t> out(8 * 300);
-             m.read_tokens(out.data(), 8, 300);
+             std::vector<uint32_t> out(8 * 600);
+             m.read_tokens(out.data(), 8, 600);
          }},
         {"decode", [] {
              setenv("MG_DISABLE_PERSISTENT", "1", 1);
@@ -273,7 +273,29 @@ void chain_routes() {
     }
 }
 
+// Split attention is taken for the sizes at which it was measured faster.
+void split_routes() {
+    struct Case {
+        size_t H, n, batch;
+        bool split;
+    };
+    const Case cases[] = {{2, 288, 8, false},  {2, 288, 64, true},   {2, 320, 48, false}, {2, 330, 48, true}, {2, 384, 16, false},
+                          {2, 449, 16, false}, {2, 449, 32, true},   {4, 449, 1, true},   {4, 447, 1, false}, {2, 576, 1, true},
+                          {2, 287, 64, false}, {4, 2048, 1, true}};
+    for (const Case &c : cases) {
+        MeshGpt m(0, shape(128, c.H, 2048, 1), 7);
+        bool split = false;
+        fake::on_launch = [&](const fake::Launch &l) { split |= l.kernel.find("attn_split_kernel") != std::string::npos; };
+        const std::vector<uint32_t> tokens(c.n * c.batch, 1);
+        std::vector<float> out(c.n * c.batch * 64);
+        m.logits(tokens.data(), tokens.size(), c.n, false, out.data(), out.size());
+        fake::on_launch = nullptr;
+        expect(split == c.split, std::to_string(c.batch * c.H) + " pairs of " + std::to_string(c.n) + " rows");
+    }
+}
+
 const std::map<std::string, void (*)()> kChecks = {
+    {"split_routes", split_routes},
     {"chain_routes", chain_routes},
     {"scratch_limits", scratch_limits},
     {"chain_shapes", chain_shapes},

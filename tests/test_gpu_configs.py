@@ -573,8 +573,8 @@ def _prefill_error(got, ref):
 
 
 # The matrix-core prefill around its dispatch lines: FP32 workgroups of 64 (head
-# width 64), 128 (head width 32) and, from 2048 rows, 256 queries; split FP16
-# from 288 rows, its 128- and 256-query workgroups; whole and ragged key tiles.
+# width 64), 128 (head width 32) and, from 2048 rows, 256 queries; split FP16 in
+# its 128- and 256-query workgroups; whole and ragged key tiles.
 @pytest.mark.parametrize("heads", [2, 4])
 @pytest.mark.parametrize("n", [64, 129, 287, 288, 320, 449, 2047, 2048, 2113])
 def test_long_prefill_matches_the_oracle(n, heads):
@@ -592,6 +592,7 @@ def test_long_prefill_matches_the_oracle(n, heads):
     for off in ("0", "1"):
         with pytest.MonkeyPatch.context() as mp:
             mp.setenv("MG_DISABLE_SPLIT_PREFILL", off)
+            mp.setenv("MG_FORCE_SPLIT_PREFILL", "1")  # also where FP32 is faster
             with G.MeshGpt(0, g, 7) as model:
                 model.set_parameters(params)
                 error[off] = _prefill_error(model.logits(tokens, n), ref)
@@ -605,6 +606,7 @@ def _split_and_fp32(kw, params, tokens, n):
     for off in ("0", "1"):
         with pytest.MonkeyPatch.context() as mp:
             mp.setenv("MG_DISABLE_SPLIT_PREFILL", off)
+            mp.setenv("MG_FORCE_SPLIT_PREFILL", "1")  # also where FP32 is faster
             with G.MeshGpt(0, G.GptConfig(**kw), 7) as model:
                 model.set_parameters(params)
                 got.append(model.logits(tokens, n))
