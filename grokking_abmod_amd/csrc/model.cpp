@@ -500,9 +500,11 @@ struct MeshGpt::Impl {
     // The same for n floats that must be finite (validate_finite's error).
     template <class Ready>
     void download_finite(float *out, const float *src, size_t n, const char *name, Ready ready) {
-        // Few values are looked through here (12288: 4 us), more where they lie
-        // (two launches and a word's copy, 15 us).
-        constexpr size_t kHostCheck = 32768;
+        // Few values are looked through here, more where they lie (two launches
+        // and a word's copy).  A call beside its kernels takes 26 us and 0.53 ns a
+        // value with the check here, 52 us and 0.25 ns with it there: 33040 values
+        // 43 and 61 us, 112000 85 and 96, 252000 160 and 114.
+        constexpr size_t kHostCheck = 98304;
         static_assert(kHostCheck * 4 <= kChunk, "in one chunk");
         if (n <= kHostCheck) {
             download(out, src, n * 4, "download", [&] {

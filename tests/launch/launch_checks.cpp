@@ -294,7 +294,23 @@ void split_routes() {
     }
 }
 
+// A result is looked through on the host up to the size at which the device's
+// launches cost less.
+void finite_checks() {
+    MeshGpt m(0, shape(32, 4, 32), 7);
+    for (size_t rows : {8, 728, 1536, 1544, 8000}) {
+        bool device = false;
+        fake::on_launch = [&](const fake::Launch &l) { device |= l.kernel.find("nonfinite_kernel") != std::string::npos; };
+        const std::vector<uint32_t> tokens(rows, 1);
+        std::vector<float> out(rows * 64);
+        m.logits(tokens.data(), rows, 8, false, out.data(), out.size());
+        fake::on_launch = nullptr;
+        expect(device == (rows * 64 > 98304), std::to_string(rows * 64) + " values");
+    }
+}
+
 const std::map<std::string, void (*)()> kChecks = {
+    {"finite_checks", finite_checks},
     {"split_routes", split_routes},
     {"chain_routes", chain_routes},
     {"scratch_limits", scratch_limits},

@@ -1,7 +1,7 @@
 """Results and prompts of every size through the pinned staging of a model.
 
 Downloads travel in chunks of 1 MiB, two in flight, and are checked for
-non-finite values on the host (up to 32768 values) or on the device; uploads up
+non-finite values on the host (up to 98304 values) or on the device; uploads up
 to 1 MiB are staged.  The sizes around those lines against the same rows asked
 for in small calls, and the error path of both checks.
 """
@@ -18,9 +18,9 @@ pytestmark = pytest.mark.gpu
 SHAPE = dict(vocab_size=256, context=4, width=64, heads=4, layers=1, attention_mesh_depth=2, ffn_mesh_depth=2)
 
 
-# rows of 256 logits: 32768 values and one row more, one chunk, a row either
+# rows of 256 logits: 98304 values and four rows more, one chunk, a row either
 # side of it, two chunks and more than two, whole and ragged
-@pytest.mark.parametrize("rows", [4, 128, 132, 1020, 1024, 1028, 2048, 2052, 5000])
+@pytest.mark.parametrize("rows", [4, 128, 132, 384, 388, 1020, 1024, 1028, 2048, 2052, 5000])
 def test_downloads_of_every_size(rows):
     tokens = np.random.default_rng(rows).integers(0, 256, rows).astype(np.uint32)
     with G.MeshGpt(0, G.GptConfig(**SHAPE), 7) as model:
