@@ -986,15 +986,16 @@ void by_lanes(int hd, F &&f) {
 
 // Whether a shape takes the matrix-core attention kernels, which work on 16 x 16
 // blocks of (query, key) and 64 rows a workgroup, or the wave-per-row kernels,
-// whose time grows with the keys a row attends over.  One gradient of 2048
-// rows, two blocks, wave against matrix kernels: head width 32 at 12 rows a
-// sequence 300 and 300 us, at 16 326 and 288, at 64 531 and 272; head width 64
-// at 12 728 and 828, at 16 786 and 782, at 32 878 and 734; head width 128 at
-// 16 1250 and 1337, at 32 1346 and 1242.  The line lies above the reference's
-// default context of 32 and not at 16: a thousand AdamW steps there carry every
-// rounding difference on, and that run keeps its published trajectory bit for
-// bit on the wave kernels.  Wider heads always take the wave kernels.
-bool matrix_attention(int sequence, int hd) { return hd <= 128 && sequence > 32; }
+// whose time grows with the keys a row attends over.  One AdamW update of 2048
+// rows, two blocks, matrix and wave kernels (us): head width 8 (W128) at 24 rows a
+// sequence 277 and 257, at 28 266 and 257, at 32 260 and 274; 16 (W256) at 20 464
+// and 448, at 24 453 and 464; 32 (W256) at 20 455 and 445, at 24 440 and 461; 64
+// (W512) at 16 723 and 716, at 24 702 and 734; 128 (W256) at 24 453 and 451, at 28 452 and
+// 454, at 32 436 and 478.  With 256 rows the matrix kernels win from 16 on, by less.
+// Wider heads always take the wave kernels.
+bool matrix_attention(int sequence, int hd) {
+    return hd <= 128 && sequence > (hd <= 8 ? 28 : hd <= 64 ? 20 : 24);
+}
 
 // Sequences up to this length run the attention backward as one launch, whose
 // key waves redo the later queries' XSA backward (a few rows each).

@@ -111,16 +111,20 @@ def test_loss_and_gradients_match_the_oracle(cfg, cases):
                 assert abs(model.cross_entropy(x, targets, s) - loss) <= 1e-6 * (1 + abs(loss))
 
 
-# Sequences past the wave attention kernels' 32 rows, on the matrix-core
-# attention: the first length there, one row into a second workgroup of 64,
-# ragged and whole tiles, every padded head width (8 and 12 dims padded to 16,
-# 24 to 32, 40 to 64, 72 to 128) and head widths that are no multiple of four;
-# the wave kernels at their last length.
+# Sequences past the wave attention kernels' rows (28 for heads of up to 8 dims,
+# 20 up to 64, 24 up to 128), on the matrix-core attention: the first length
+# there, one row into a second workgroup of 64, ragged and whole tiles, every
+# padded head width (8 and 12 dims padded to 16, 24 to 32, 40 to 64, 72 to 128)
+# and head widths that are no multiple of four; the wave kernels at their last
+# length.
 LONG = [(dict(width=32, heads=4), 65), (dict(width=24, heads=2), 100), (dict(width=48, heads=2), 127),
         (dict(width=128, heads=2), 64), (dict(width=128, heads=2), 129), (dict(width=32, heads=1), 192),
         (dict(width=40, heads=1, xsa=0), 97), (dict(width=72, heads=1), 70), (dict(width=128, heads=1), 130),
         (dict(width=30, heads=3, rope=0, qk_norm=0), 66), (dict(width=12, heads=2), 161),
-        (dict(width=128, heads=2), 32), (dict(width=32, heads=4), 33), (dict(width=256, heads=2), 33)]
+        (dict(width=128, heads=2), 32), (dict(width=32, heads=4), 33), (dict(width=256, heads=2), 33),
+        (dict(width=32, heads=4), 28), (dict(width=32, heads=4), 29), (dict(width=64, heads=4), 20),
+        (dict(width=64, heads=4), 21), (dict(width=128, heads=2), 21), (dict(width=256, heads=2), 24),
+        (dict(width=256, heads=2), 25), (dict(width=72, heads=1), 25)]
 
 
 @pytest.mark.parametrize("cfg,s", LONG, ids=[f"W{c['width']}-H{c['heads']}-S{s}" for c, s in LONG])
