@@ -17,16 +17,17 @@
 // scratch; head reductions (QK-Norm, XSA) and the RoPE pair exchange stay
 // inside a wave (a head is hd <= 64 consecutive channels = consecutive lanes).
 //
-// What bounds it is instruction issue: five VALU instructions a value and layer
-// (product, multiply-add, exponential, multiply-add, maximum; values are carried
-// times log2(e), or it is six) and an LDS write and read of the value, behind a
-// barrier each layer that only other workgroups' waves on the SIMD can fill.
-// Widths 512 and 1024 keep to 128 registers for four waves a SIMD; 128 and 256,
-// with 16 rows a thread, would spill and keep three.  A prefill of 256 x 128 rows
-// (W1024, 12 blocks, 13 launches of this kernel, 527 us each before and 446 now): 8.84 ms,
-// 7.94 with the scaled values alone, 7.63 with four waves as well.
-// Not kept: strides of 256 and 512 from the thread's own registers (7.73 ms), weights
-// loaded two layers ahead (7.74).
+// What bounds it is instruction issue: six VALU instructions a value and layer
+// (product, multiply-add, ELU's product, exponential, sum and maximum) and an LDS
+// write and read of the value, behind a barrier each layer that only other
+// workgroups' waves on the SIMD can fill.  Widths 512 and 1024 keep to 128
+// registers for four waves a SIMD; 128 and 256, with 16 rows a thread, would
+// spill and keep three.  A prefill of 256 x 128 rows (W1024, 12 blocks, 13 launches
+// of this kernel): 7.8 ms, 456 us a launch (8.84 and 527 with three waves).
+// Values carried times log2(e) save the ELU's product and take 7.68 ms (446), but a
+// finite value above 2.36e38 is infinite in those units.  Not kept either, timed
+// with them: strides of 256 and 512 from the thread's own registers (7.73 ms against
+// 7.63), weights loaded two layers ahead (7.74).
 #include <hip/hip_runtime.h>
 
 #include "dpp.hpp"
@@ -39,14 +40,11 @@ constexpr float kEps = 1e-5f;  // src/gpt/mod.rs:38
 // (f64(1e-12f))^2 rounded to f32: the XSA norm floor of reference.rs:591.
 constexpr float kXsaNormFloor = float(double(1e-12f) * double(1e-12f));
 
-constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
-
-// The ELU of a value t carried times log2(e): max(t, log2(e) (clamp(2^t, 0, 1)
-// - 1)) with the NaN-propagating maximum, which keeps a NaN t NaN
-// (kernels.hip's elu).
-__device__ __forceinline__ float elu_log2(float t) {
-    const float e = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(t), 0.0f, 1.0f);
-    return __builtin_elementwise_maximum(t, __builtin_fmaf(e, kLog2e, -kLog2e));
+__device__ __forceinline__ float elu_f(float z) {
+    // max(z, clamp(exp(z), 0, 1) - 1) with the NaN-propagating maximum, which
+    // keeps a NaN z NaN (kernels.hip's elu)
+    const float e = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(z * 1.4426950408889634f), 0.0f, 1.0f);
+    return __builtin_elementwise_maximum(z, e - 1.0f);
 }
 
 template <int W>
@@ -117,8 +115,8 @@ struct Tile {
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
             for (int i = 0; i < RG; ++i) {
-                const float t = v[k][i] * w[k].x + p[k][i] * w[k].y;
-                v[k][i] = LAST ? t : elu_log2(t);
+                const float z = v[k][i] * w[k].x + p[k][i] * w[k].y;
+                v[k][i] = LAST ? z : elu_f(z);
             }
     }
     template <bool LAST>
@@ -134,8 +132,6 @@ struct Tile {
     // A mesh stack on v in place: layer l maps v[c] to v[c] w0 + v[c + st] w1
     // with ELU on every layer but the last (reference.rs:422-453).
     // Butterfly strides double from 1 and wrap at W (W is a power of two).
-    // Values are carried times log2(e), which the ELU's exponential would
-    // otherwise multiply in.
     __device__ void mesh(float (&v)[CPT][RG], const float2 *__restrict__ w, int depth, const Shape &s) {
         float2 wc[CPT];
 #pragma unroll
@@ -260,27 +256,23 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
                 }
             }
         }
-#pragma unroll
-        for (int k = 0; k < CPT; ++k)
-#pragma unroll
-            for (int i = 0; i < RG; ++i) y[k][i] *= kLog2e;
         t.mesh(y, reinterpret_cast<const float2 *>(a.wproj), s.A, s);
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) x[k][i] = __builtin_fmaf(y[k][i], kLn2, x[k][i]);
+            for (int i = 0; i < RG; ++i) x[k][i] += y[k][i];
         float inv[RG];
         t.row_inv_rms(x, inv);
         float n[CPT][RG];
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * (inv[i] * kLog2e);
+            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * inv[i];
         t.mesh(n, reinterpret_cast<const float2 *>(a.wffn), s.F, s);
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) x[k][i] = __builtin_fmaf(n[k][i], kLn2, x[k][i]);
+            for (int i = 0; i < RG; ++i) x[k][i] += n[k][i];
     }
     if (post || a.embed) {
 #pragma unroll
@@ -292,8 +284,7 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
     }
     if (!a.xn && !pre) return;
 
-    // The next RMSNorm: the final one for the head, or the block's pre-norm,
-    // whose rows enter the meshes times log2(e).
+    // The next RMSNorm: the final one for the head, or the block's pre-norm.
     float n[CPT][RG];
     {
         float inv[RG];
@@ -310,7 +301,7 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * (inv[i] * kLog2e);
+            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * inv[i];
     }
 
     // Q, K and V meshes, one after another, each from the normalised rows.
@@ -340,7 +331,7 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
 #pragma unroll
                 for (int i = 0; i < RG; ++i) {
                     float q = v[k][i];
-                    q *= s.qk_norm ? rsqrtf(head_sum<HD>(q * q, s.hd) * (1.0f / float(s.hd)) + kEps * kLog2e * kLog2e) : kLn2;
+                    if (s.qk_norm) q *= rsqrtf(head_sum<HD>(q * q, s.hd) * (1.0f / float(s.hd)) + kEps);
                     if (s.rope) {
                         const float p = __shfl_xor(q, s.half, 64);
                         const float2 cs = a.rope[size_t(posof(i)) * s.half + (d < s.half ? d : d - s.half)];
@@ -348,9 +339,6 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
                     }
                     v[k][i] = q;
                 }
-            } else {
-#pragma unroll
-                for (int i = 0; i < RG; ++i) v[k][i] *= kLn2;
             }
 #pragma unroll
             for (int i = 0; i < RG; ++i) {

@@ -5,8 +5,8 @@
 // What bounds it is the chain of dependent steps of one token, not work: the
 // default model's window (32 rows of 32 channels, two blocks) is 0.2 MFLOP.  As
 // one launch per operator a token took seven launches of 3-9 us (48 us); in one
-// launch it takes 7.2 us, about half of it the mesh layers (a wave issues some
-// 40 dependent instructions for a layer of q, k and v).  A workgroup keeps a
+// launch it takes 7.3 us, about half of it the mesh layers (a wave issues some
+// 45 dependent instructions for a layer of q, k and v).  A workgroup keeps a
 // sequence's window to itself from token to token:
 //  - a row lies in 16 lanes, channel CPL l + j in register j of lane l (CPL =
 //    W / 16), four rows a wave: a mesh layer's partner is another register, or
@@ -38,16 +38,16 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr float kRmsEps = 1e-5f;  // src/gpt/mod.rs:38
 // (f64(1e-12f))^2 rounded to f32: the XSA norm floor of reference.rs:591
 constexpr float kXsaFloor = float(double(1e-12f) * double(1e-12f));
-constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
+constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kRing = 2 * kWindowRows;  // tokens kept in LDS
 constexpr size_t kWindowLds = 160 * 1024;  // a CU's
 
-// The ELU of a value t carried times log2(e): t, or log2(e) (2^t - 1) where t is
-// not positive, NaN included.  A select on t, which does not wait for the
-// exponential, keeps the dependent chain one step shorter than a maximum.
-__device__ __forceinline__ float elu_log2(float t) {
-    const float e = __builtin_fmaf(__builtin_amdgcn_exp2f(t), kLog2e, -kLog2e);
-    return t > 0.0f ? t : e;
+// The ELU: z, or e^z - 1 where z is not positive, NaN included.  A select on z,
+// which does not wait for the exponential, keeps the dependent chain one step
+// shorter than a maximum.
+__device__ __forceinline__ float elu(float z) {
+    const float e = __builtin_amdgcn_exp2f(z * kLog2e) - 1.0f;
+    return z > 0.0f ? z : e;
 }
 
 // v of the lane 16 (32) away combined with the lane's own: register swaps
@@ -96,8 +96,8 @@ __device__ __forceinline__ void partner(const float (&x)[CPL], float (&p)[CPL]) 
     }
 }
 
-// N mesh stacks of one depth (reference.rs:422-453) on x, in place, values
-// carried times log2(e); stack i's weights at w[i].  Strides are 1, or
+// N mesh stacks of one depth (reference.rs:422-453) on x, in place; stack i's
+// weights at w[i].  Strides are 1, or
 // 2^(layer mod log2 W) (W = 16 CPL).  Two layers' weights are in registers or
 // on their way while a third is computed.
 template <bool BF, int N, int CPL>
@@ -142,7 +142,7 @@ struct Stacks {
 #pragma unroll
             for (int j = 0; j < CPL; ++j) {
                 const float z = x[i][j] * buf[B][i][j].x + p[i][j] * buf[B][i][j].y;
-                x[i][j] = last ? z : elu_log2(z);
+                x[i][j] = last ? z : elu(z);
             }
         if (!last) load(l + 2, B);
         return last;
@@ -167,26 +167,25 @@ __device__ __forceinline__ void stacks(float (&x)[N][CPL], const float *const (&
     s.all(x);
 }
 
-// n = RMSNorm(x) times log2(e) (reference.rs:392-409).
+// n = RMSNorm(x) (reference.rs:392-409).
 template <int CPL>
-__device__ __forceinline__ void norm_log2(const float (&x)[CPL], float (&n)[CPL]) {
+__device__ __forceinline__ void norm(const float (&x)[CPL], float (&n)[CPL]) {
     float sq = 0.0f;
 #pragma unroll
     for (int j = 0; j < CPL; ++j) sq = fmaf(x[j], x[j], sq);
-    const float inv = rsqrtf(group_sum<16>(sq) * (1.0f / float(16 * CPL)) + kRmsEps) * kLog2e;
+    const float inv = rsqrtf(group_sum<16>(sq) * (1.0f / float(16 * CPL)) + kRmsEps);
 #pragma unroll
     for (int j = 0; j < CPL; ++j) n[j] = x[j] * inv;
 }
 
 template <int CPL>
-__device__ __forceinline__ void put_row(float *row, const float (&x)[CPL], float scale) {
+__device__ __forceinline__ void put_row(float *row, const float (&x)[CPL]) {
     if constexpr (CPL == 2) {
-        *reinterpret_cast<float2 *>(row) = make_float2(x[0] * scale, x[1] * scale);
+        *reinterpret_cast<float2 *>(row) = make_float2(x[0], x[1]);
     } else {
 #pragma unroll
         for (int j = 0; j < CPL; j += 4)
-            *reinterpret_cast<float4 *>(row + j) =
-                make_float4(x[j] * scale, x[j + 1] * scale, x[j + 2] * scale, x[j + 3] * scale);
+            *reinterpret_cast<float4 *>(row + j) = make_float4(x[j], x[j + 1], x[j + 2], x[j + 3]);
     }
 }
 
@@ -310,7 +309,6 @@ __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
         if (d < half) turn[j].y = -turn[j].y;
     }
     const size_t gA = size_t(2) * W * a.A, gF = size_t(2) * W * a.F;
-    const float qk_eps = kRmsEps * kLog2e * kLog2e;  // QK-Norm of rows carried times log2(e)
     const float *weights = a.w, *E = a.E;
     if constexpr (STAGED) {
         const int nw = a.L * int(4 * gA + gF);
@@ -335,7 +333,7 @@ __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
             const bool tail = l + 1 == a.L;  // only the last row goes on, past its keys and values
             const bool goes_on = !tail || wave == last_wave;
             float qkv[3][CPL];
-            norm_log2(x, qkv[0]);
+            norm(x, qkv[0]);
 #pragma unroll
             for (int j = 0; j < CPL; ++j) qkv[1][j] = qkv[2][j] = qkv[0][j];
             if constexpr (GROUP == 3) {
@@ -353,15 +351,14 @@ __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
             // QK-Norm, then slice RoPE (reference.rs:174-193), each when on.
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                float inv = kLn2;
                 if (a.qk_norm) {
                     float sq = 0.0f;
 #pragma unroll
                     for (int j = 0; j < CPL; ++j) sq = fmaf(qkv[i][j], qkv[i][j], sq);
-                    inv = rsqrtf(group_sum<LPH>(sq) * (1.0f / float(HD)) + qk_eps);
-                }
+                    const float inv = rsqrtf(group_sum<LPH>(sq) * (1.0f / float(HD)) + kRmsEps);
 #pragma unroll
-                for (int j = 0; j < CPL; ++j) qkv[i][j] *= inv;
+                    for (int j = 0; j < CPL; ++j) qkv[i][j] *= inv;
+                }
                 if (a.rotate) {
                     float o[CPL];
 #pragma unroll
@@ -377,9 +374,9 @@ __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
                 }
             }
             float *at = Q + row * STRIDE + CPL * l16;
-            put_row(at, qkv[0], 1.0f);
-            put_row(at + ROWS * STRIDE, qkv[1], 1.0f);
-            put_row(at + 2 * ROWS * STRIDE, qkv[2], kLn2);
+            put_row(at, qkv[0]);
+            put_row(at + ROWS * STRIDE, qkv[1]);
+            put_row(at + 2 * ROWS * STRIDE, qkv[2]);
             if (a.kc && s + 1 == a.steps && row <= last) {
                 // The cache as the decode of this length leaves it: every row of the window.
                 const int c0 = CPL * l16;
@@ -389,7 +386,7 @@ __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
                     const size_t to = size_t(l) * a.layer_elems +
                                       (size_t(b * H + c / HD) * a.cap + row) * HD + c % HD;
                     a.kc[to] = qkv[1][j];
-                    a.vc[to] = qkv[2][j] * kLn2;
+                    a.vc[to] = qkv[2][j];
                 }
             }
             __syncthreads();
@@ -402,22 +399,20 @@ __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
             if (goes_on) {
                 float z[1][CPL];
                 take(Q + row * STRIDE + CPL * l16, z[0]);
-#pragma unroll
-                for (int j = 0; j < CPL; ++j) z[0][j] *= kLog2e;
                 const float *const wp[1] = {w + 3 * gA}, *const wf[1] = {w + 4 * gA};
                 stacks<BF>(z, wp, a.A, l16);
 #pragma unroll
-                for (int j = 0; j < CPL; ++j) x[j] = fmaf(z[0][j], kLn2, x[j]);
-                norm_log2(x, z[0]);
+                for (int j = 0; j < CPL; ++j) x[j] += z[0][j];
+                norm(x, z[0]);
                 stacks<BF>(z, wf, a.F, l16);
 #pragma unroll
-                for (int j = 0; j < CPL; ++j) x[j] = fmaf(z[0][j], kLn2, x[j]);
+                for (int j = 0; j < CPL; ++j) x[j] += z[0][j];
             }
         }
         if (row == last) {
             float n[CPL];
-            norm_log2(x, n);
-            put_row(xn + CPL * l16, n, kLn2);
+            norm(x, n);
+            put_row(xn + CPL * l16, n);
         }
         __syncthreads();
         // The tied head: 16 lanes a token.

@@ -25,7 +25,7 @@ import pytest
 import grokking_abmod_amd as G
 import oracle_lib as O
 from conftest import ROOT, TOL, assert_close
-from trajectory import check_trajectory
+from trajectory import check_trajectory, largest_values
 
 pytestmark = pytest.mark.gpu
 
@@ -739,3 +739,21 @@ def test_row_tiles_match_the_oracle(W, H, n, A, F, butterfly, switch):
         got = model.logits(tokens, n)
     # the 2-norm allowance of _prefill_error's other uses: forty f32 roundings, four times
     assert _prefill_error(got, O.logits(o, params, tokens, n)) <= 1e-5
+
+
+# Widths of each register-tile kernel, and the general block kernel's.
+@pytest.mark.parametrize("W,H", [(64, 4), (128, 4), (256, 4), (512, 8), (1024, 16)])
+def test_a_mesh_may_reach_the_largest_values(W, H):
+    """A V mesh whose first layer reaches 3.3e38 and whose second brings it back:
+    finite values are used as they are, in whatever units a kernel works."""
+    kw = dict(vocab_size=16, context=24, width=W, heads=H, layers=1, attention_mesh_depth=2, ffn_mesh_depth=2,
+              embedding=1)
+    o = O.config(**kw)
+    params = O.initialize(o, 7)
+    largest_values(params, W, O.group_offsets(o)[3])
+    tokens = G.random_prompts(16, 3, 24, 11).reshape(-1)
+    with G.MeshGpt(0, G.GptConfig(**kw), 7) as model:
+        model.set_parameters(params)
+        got = model.logits(tokens, 24)
+    # the 2-norm allowance of _prefill_error's other uses: forty f32 roundings, four times
+    assert _prefill_error(got, O.logits(o, params, tokens, 24)) <= 1e-5

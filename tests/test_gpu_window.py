@@ -12,7 +12,7 @@ import pytest
 import grokking_abmod_amd as G
 import oracle_lib as O
 from conftest import assert_close
-from trajectory import check_trajectory
+from trajectory import check_trajectory, largest_values
 
 pytestmark = pytest.mark.gpu
 
@@ -109,6 +109,23 @@ def test_more_sequences_than_workgroups_run_at_once(cfg, count):
         got = model.generate_tokens(prompts, count, 0.7, 7)
         for b in (0, 255, 256, 599):
             check_trajectory(o, params, prompts[b], got[b], 0.7, 7 + b, _last(model), cached=False)
+
+
+@pytest.mark.parametrize("W,H", [(32, 4), (64, 4), (128, 4)])
+def test_a_mesh_may_reach_the_largest_values(W, H):
+    """As the register-tile kernels' test of the same name: windows past the context."""
+    kw = dict(vocab_size=16, context=20, width=W, heads=H, layers=1, attention_mesh_depth=2, ffn_mesh_depth=2,
+              embedding=1)
+    o = O.config(**kw)
+    params = O.initialize(o, 7)
+    largest_values(params, W, O.group_offsets(o)[3])
+    prompts = G.random_prompts(16, 2, 21, 7)
+    with G.MeshGpt(0, G.GptConfig(**kw), 7, max_batch=2) as model:
+        model.set_parameters(params)
+        got = model.generate_tokens(prompts, 6, 0.0, 7)
+        last = model.last_logits(2)
+    ref = [O.logits(o, params, got[b, -21:-1], 20)[-1] for b in range(2)]
+    assert_close(last, ref, what="last logits")
 
 
 def test_window_generation_reports_nonfinite_logits():

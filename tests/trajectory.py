@@ -82,3 +82,15 @@ def check_trajectory(o, params, prompt, got, temperature, seed, device_logits, c
         assert divergences <= max_divergences, f"more than {max_divergences} divergences, last at {where}"
         rest = O.generate(o, params, got[:k + 1], len(got) - k - 1, temperature, next_seed, cached=cached)
         expected = rest
+
+
+def largest_values(params, W, v):
+    """Table rows of entries 0.8 to 1.2 in size, and a V mesh of two layers (at
+    params[v]) that takes the positive ones to between 2.1e38 and 3.3e38 and back."""
+    rng = np.random.default_rng(3)
+    table = params[:16 * W].reshape(16, W)
+    table[:] = rng.choice([-1.0, 1.0], (16, W)) * rng.uniform(0.8, 1.2, (16, W))
+    mesh = params[v:v + 4 * W].reshape(2, W, 2)
+    mesh[:, :, 1] = 0.0
+    mesh[0, :, 0] = 2.7e38
+    mesh[1, :, 0] = 1e-38
