@@ -305,7 +305,6 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
     }
 
     // Q, K and V meshes, one after another, each from the normalised rows.
-    const size_t meshw = size_t(s.A) * W;
     const bool no_q = a.q_last && (r0 + C::R) / rps == r0 / rps && r0 + C::R < a.ro.rows;  // no sequence ends here
     for (int m = no_q ? 1 : 0; m < 3; ++m) {
         const float *wm = m == 0 ? a.wq : (m == 1 ? a.wk : a.wv);
@@ -315,7 +314,6 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
 #pragma unroll
             for (int i = 0; i < RG; ++i) v[k][i] = n[k][i];
         t.mesh(v, reinterpret_cast<const float2 *>(wm), s.A, s);
-        (void)meshw;
         // Addresses and RoPE factors are formed here for each mesh: hoisted out of
         // the loop they would hold up to 60 registers through every layer.  (With
         // 16 rows a thread, widths 128 and 256, forming them spills.)

@@ -964,24 +964,23 @@ __global__ void __launch_bounds__(kThreads) attention_output_grad_wave(const flo
 // f(registers a lane, lanes) of a (row, head)'s group.
 template <class F>
 void by_lanes(int hd, F &&f) {
-    auto call = [&](auto e, auto g) { f(e, g); };
     using std::integral_constant;
     if (hd <= 8)
-        call(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+        f(integral_constant<int, 1>{}, integral_constant<int, 8>{});
     else if (hd <= 16)
-        call(integral_constant<int, 1>{}, integral_constant<int, 16>{});
+        f(integral_constant<int, 1>{}, integral_constant<int, 16>{});
     else if (hd <= 32)
-        call(integral_constant<int, 1>{}, integral_constant<int, 32>{});
+        f(integral_constant<int, 1>{}, integral_constant<int, 32>{});
     else if (hd <= 64)
-        call(integral_constant<int, 1>{}, integral_constant<int, 64>{});
+        f(integral_constant<int, 1>{}, integral_constant<int, 64>{});
     else if (hd <= 128)
-        call(integral_constant<int, 2>{}, integral_constant<int, 64>{});
+        f(integral_constant<int, 2>{}, integral_constant<int, 64>{});
     else if (hd <= 256)
-        call(integral_constant<int, 4>{}, integral_constant<int, 64>{});
+        f(integral_constant<int, 4>{}, integral_constant<int, 64>{});
     else if (hd <= 512)
-        call(integral_constant<int, 8>{}, integral_constant<int, 64>{});
+        f(integral_constant<int, 8>{}, integral_constant<int, 64>{});
     else
-        call(integral_constant<int, 16>{}, integral_constant<int, 64>{});
+        f(integral_constant<int, 16>{}, integral_constant<int, 64>{});
 }
 
 // Whether a shape takes the matrix-core attention kernels, which work on 16 x 16

@@ -66,15 +66,13 @@ __device__ __forceinline__ float sum_groups(float v) {
 // v of lane l ^ M inside 16 lanes.
 template <int M>
 __device__ __forceinline__ float lane_xor(float v, int l16) {
+    static_assert(M == 1 || M == 2 || M == 4, "half the lanes of a head: two, four or eight heads in 16");
     if constexpr (M == 1)
         return dpp_move<0xB1>(v, v);  // quad_perm [1,0,3,2]
     else if constexpr (M == 2)
         return dpp_move<0x4E>(v, v);  // quad_perm [2,3,0,1]
-    else if constexpr (M == 4) {
-        const float down = dpp_move<0x124>(v, v), up = dpp_move<0x12C>(v, v);  // row_ror:4, :12
-        return (l16 & 4) ? down : up;
-    } else
-        return dpp_move<0x128>(v, v);  // row_ror:8
+    const float down = dpp_move<0x124>(v, v), up = dpp_move<0x12C>(v, v);  // row_ror:4, :12
+    return (l16 & 4) ? down : up;
 }
 
 // Lane l of each 16 gets v of lane (l + K) mod 16.
@@ -286,7 +284,7 @@ template <int CPL, int HD, int NW, bool STAGED, bool BF>
 __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
     constexpr int W = 16 * CPL, H = W / HD, LPH = 16 / H, ROWS = 4 * NW, KB = ROWS / 16, STRIDE = W + 4;
     constexpr int GROUP = CPL * NW <= 32 ? 3 : 1;  // stacks side by side, as registers allow
-    static_assert(H <= 16 && 16 % H == 0, "a head is whole lanes");
+    static_assert(H == 2 || H == 4 || H == 8, "a head is two, four or eight whole lanes");
     extern __shared__ __align__(16) float lds[];
     // The matrix products read whole 16-dim blocks, past a narrow last head.
     float *Q = lds, *K = Q + ROWS * STRIDE, *V = K + ROWS * STRIDE, *xn = V + ROWS * STRIDE + 16, *logits = xn + W;
@@ -362,13 +360,7 @@ __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
                 if (a.rotate) {
                     float o[CPL];
 #pragma unroll
-                    for (int j = 0; j < CPL; ++j)
-                        {
-                        if constexpr (LPH > 1)
-                            o[j] = lane_xor<LPH / 2>(qkv[i][j], l16);
-                        else
-                            o[j] = qkv[i][(j + CPL / 2) % CPL];
-                    }
+                    for (int j = 0; j < CPL; ++j) o[j] = lane_xor<LPH / 2>(qkv[i][j], l16);
 #pragma unroll
                     for (int j = 0; j < CPL; ++j) qkv[i][j] = qkv[i][j] * turn[j].x + o[j] * turn[j].y;
                 }
