@@ -1877,7 +1877,7 @@ void MeshGpt::read_tokens(uint32_t *out, size_t batch, size_t length) {
 
 std::vector<float> MeshGpt::last_logits() {
     std::vector<float> out(impl_->batch * impl_->cfg.vocab_size);
-    last_logits(out.data(), out.size());
+    if (!out.empty()) last_logits(out.data(), out.size());
     return out;
 }
 

@@ -309,7 +309,14 @@ void finite_checks() {
     }
 }
 
+// Before a batch there are no logits, which is no error.
+void no_batch() {
+    MeshGpt m(0, shape(32, 4, 32), 7);
+    expect(status_of([&] { expect(m.last_logits().empty(), "no logits"); }) == 0, "last_logits before a batch");
+}
+
 const std::map<std::string, void (*)()> kChecks = {
+    {"no_batch", no_batch},
     {"finite_checks", finite_checks},
     {"split_routes", split_routes},
     {"chain_routes", chain_routes},
