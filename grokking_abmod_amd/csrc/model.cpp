@@ -1906,7 +1906,7 @@ bool sample_logits(int device, const float *logits, size_t rows, size_t vocab, f
     drng.ensure(rows * 8);
     dtok.ensure(rows * 4);
     dlen.ensure(rows * 4);
-    dflags.ensure(8);  // non-finite logits of the decode, of a downloaded result
+    dflags.ensure(4);
     check(hipMemcpy(dl.p, logits, rows * vocab * 4, hipMemcpyHostToDevice), "upload logits");
     check(hipMemcpy(drng.p, rng_states, rows * 8, hipMemcpyHostToDevice), "upload rng");
     check(hipMemset(dlen.p, 0, rows * 4), "clear lengths");
