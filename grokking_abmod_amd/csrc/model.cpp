@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 
 #include "kernels.hpp"
 
@@ -151,6 +152,7 @@ struct MeshGpt::Impl {
     static constexpr size_t kUpload = size_t(1) << 20, kChunk = size_t(1) << 20, kChunks = 2, kWords = 256;
     PinnedBuf hio;  // the upload, then the download chunks, then single words
     DevBuf dstage;
+    std::mutex reading;  // of the chunks, dstage and the download's flag: threads may read a model's results at once
     hipEvent_t chunk_ev[kChunks] = {};
     bool upload_busy = false;    // hio's upload may still be read by the stream
     int known_flags = -1;        // dflags' value when the host has it
@@ -506,6 +508,7 @@ struct MeshGpt::Impl {
         // 43 and 61 us, 112000 85 and 96, 252000 160 and 114.
         constexpr size_t kHostCheck = 98304;
         static_assert(kHostCheck * 4 <= kChunk, "in one chunk");
+        const std::lock_guard<std::mutex> guard(reading);
         if (n <= kHostCheck) {
             download(out, src, n * 4, "download", [&] {
                 ready();
@@ -1541,6 +1544,7 @@ struct MeshGpt::Impl {
     // The first len tokens of b sequences; with `checked`, finish() on the way.
     void read_tokens(uint32_t *out, size_t b, size_t len, bool checked = false) {
         if (b > batch || len > length) throw Error("requested tokens exceed the generated sequences");
+        const std::lock_guard<std::mutex> guard(reading);
         dstage.ensure(b * len * 4);
         kern::gather_rows(dtokens.as<uint32_t>(), tcap, int(b), int(len), dstage.as<uint32_t>(), stream);
         const bool ask = checked && known_flags < 0;
@@ -1886,6 +1890,7 @@ void MeshGpt::last_logits(float *out, size_t capacity) {
     const size_t n = m.batch * m.cfg.vocab_size;
     Impl::check_capacity(out, capacity, n);
     m.activate();
+    const std::lock_guard<std::mutex> guard(m.reading);
     if (n) m.download(out, m.dlogits.p, n * 4, "download logits", [] {});
 }
 

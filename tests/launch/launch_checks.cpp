@@ -1,5 +1,6 @@
 // What the host launches, checked on a machine without a GPU: the library's
 // objects against fake_hip.cpp.  `launch_checks NAME` runs one check.
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -7,6 +8,7 @@
 #include <map>
 #include <set>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "fake_hip.hpp"
@@ -315,7 +317,33 @@ void no_batch() {
     expect(status_of([&] { expect(m.last_logits().empty(), "no logits"); }) == 0, "last_logits before a batch");
 }
 
+// Threads that read a model's results at once each get theirs.
+void threads_reading() {
+    MeshGpt m(0, shape(1024, 16, 64, 8, 10, 10), 7, 64);
+    const std::vector<uint32_t> prompts(64 * 40, 1);
+    m.prefill(prompts.data(), 64, 40, 0.0f, 7, 50);
+    const std::vector<float> weights = m.parameters();  // four chunks
+    std::vector<std::thread> readers;
+    std::atomic<int> wrong{0};
+    for (int t = 0; t < 4; ++t)
+        readers.emplace_back([&, t] {
+            std::vector<uint32_t> tokens(64 * 40);
+            for (int i = 0; i < 40; ++i) {
+                if (t < 2) {
+                    wrong += m.parameters() != weights;
+                } else {
+                    m.read_tokens(tokens.data(), 64, 40);
+                    wrong += tokens != prompts && tokens != std::vector<uint32_t>(64 * 40, 0);  // no kernel gathers here
+                    for (float v : m.last_logits()) wrong += v != 0.0f;
+                }
+            }
+        });
+    for (std::thread &r : readers) r.join();
+    expect(wrong == 0, std::to_string(wrong) + " reads held another's data");
+}
+
 const std::map<std::string, void (*)()> kChecks = {
+    {"threads_reading", threads_reading},
     {"no_batch", no_batch},
     {"finite_checks", finite_checks},
     {"split_routes", split_routes},

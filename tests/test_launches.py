@@ -27,7 +27,7 @@ def checks(tmp_path_factory):
     objects = [os.path.join(OBJECTS, f) for f in sorted(os.listdir(OBJECTS))
                if f.endswith(".o") and f not in ("capi.o", "mesh_gpt_cli.o", "mesh_gpt_bench.o")]
     exe = str(tmp_path_factory.mktemp("launch") / "launch_checks")
-    built = subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROCM, "include"),
+    built = subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-pthread", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROCM, "include"),
                             "-I", CSRC, os.path.join(HERE, "launch_checks.cpp"), os.path.join(HERE, "fake_hip.cpp"),
                             *objects, "-o", exe], capture_output=True, text=True)
     assert built.returncode == 0, built.stderr
@@ -36,7 +36,7 @@ def checks(tmp_path_factory):
 
 @pytest.mark.parametrize("name", ["refused_launches", "foreign_errors", "window_launches", "window_routes", "chain_shapes",
                                   "scratch_limits", "chain_routes", "split_routes", "finite_checks",
-                                  "no_batch"])
+                                  "no_batch", "threads_reading"])
 def test_launches(checks, name):
     run = subprocess.run([checks, name], capture_output=True, text=True, timeout=300)
     assert run.returncode == 0 and run.stdout == "ok\n", run.stdout + run.stderr
