@@ -702,8 +702,19 @@ def test_split_prefill_reports_values_that_overflow():
                                          (1024, 16, 64, 4), (1024, 16, 259, 1), (512, 8, 511, 1), (512, 8, 513, 1)])
 def test_last_rows_alone_match_all_rows(W, H, n, batch):
     """The last rows' logits: 1e-5 of their 2-norm, four times forty f32 roundings."""
+    _check_last_rows(W, H, n, batch)
+
+
+@pytest.mark.parametrize("switch", [dict(xsa=0), dict(qk_norm=0), dict(rope=0), dict(qk_norm=0, rope=0, xsa=0)],
+                         ids=["no-xsa", "no-qk", "no-rope", "none"])
+@pytest.mark.parametrize("W,H,n,batch", [(128, 4, 64, 32), (256, 4, 1025, 1), (512, 8, 70, 8), (1024, 16, 259, 1)])
+def test_last_rows_alone_without_operators(W, H, n, batch, switch):
+    _check_last_rows(W, H, n, batch, **switch)
+
+
+def _check_last_rows(W, H, n, batch, **switch):
     kw = dict(vocab_size=64, context=n + 1, width=W, heads=H, layers=2, attention_mesh_depth=5, ffn_mesh_depth=4,
-              connectivity=1)
+              connectivity=1, **switch)
     g = G.GptConfig(**kw)
     tokens = G.random_prompts(64, batch, n, 11)
     with G.MeshGpt(0, g, 7, max_batch=batch) as model:
