@@ -301,7 +301,11 @@ matrix_forward_kernel(AttnShape s, const float *__restrict__ q, const float *__r
 // From dy = d loss / d y, D = dy . y per row and the forward's lse:
 //   blockIdx.y = 0: dq_i = scale sum_j P_ij (dy_i . v_j - D_i) k_j
 //   blockIdx.y = 1: dk_j = scale sum_i P_ij (dy_i . v_j - D_i) q_i,  dv_j += sum_i P_ij dy_i
-// (the same fixed order of sums in every run).
+// (the same fixed order of sums in every run).  A masked pair has weight 0 and the
+// products still read its rows.  The forward keeps a later row that is not finite
+// from the losses of earlier ones; here it needs no such care: with or without a
+// target, the final norm's backward of that row multiplies by values that are not
+// finite, and every weight's gradient adds all rows.
 template <int HDP>
 __global__ void __launch_bounds__(64 * kWaves)
 matrix_backward_kernel(AttnShape s, const float *__restrict__ q, const float *__restrict__ k,
