@@ -987,13 +987,18 @@ struct MeshGpt::Impl {
         }
         auto X = [&](int b) { return at(p.x) + size_t(b) * RW; };
         auto last = [&](size_t o, int depth) { return at(o) + size_t(depth - 1) * RW; };
-        const bool chain = use_chain && T::chain_fits(ma, mf, H) && (force_chain || T::chain_pays(ma, mf, R));
+        // The two passes of the chain read and store what the separate launches do,
+        // so that each is taken where it is faster.
+        const bool chain_up = use_chain && T::chain_fits(ma, mf, H) &&
+                              (force_chain || T::forward_chain_pays(ma, R, backward));
+        const bool chain_down =
+            use_chain && T::backward_chain_fits(ma, mf, H) && (force_chain || T::backward_chain_pays(ma, L, R));
         auto attend = [&](int b) {
             const TrainBlock &k = p.blocks[b];
             T::attention_forward(at(k.qr), at(k.kr), last(k.vs, A), at(k.y), at(k.z), at(k.lse), R, seq, W, H,
                                  cfg.xsa, stream);
         };
-        if (chain) {
+        if (chain_up) {
             // A launch before, between and after the attentions.
             for (int b = 0; b <= L; ++b) {
                 T::ForwardChain c{};
@@ -1092,7 +1097,7 @@ struct MeshGpt::Impl {
             T::attention_backward(at(k.qr), at(k.kr), last(k.vs, A), at(k.y), at(k.lse), dt, dy, dq, dk, dv,
                                   at(p.dsum), R, seq, W, H, cfg.xsa, stream);
         };
-        if (chain) {
+        if (chain_down) {
             for (int b = L; b >= 0; --b) {
                 T::BackwardChain c{};
                 float *out[5] = {};

@@ -97,8 +97,10 @@ void mesh_backward_set(const Mesh &m, int count, const float *const *in, const f
 // few layers).  Rows are x_b -> xm -> x_{b+1} of block b; null pointers leave a
 // part out.
 bool chain_fits(const Mesh &ma, const Mesh &mf, int H);
-// Whether it is faster than the separate launches for this many rows.
-bool chain_pays(const Mesh &ma, const Mesh &mf, int rows);
+bool backward_chain_fits(const Mesh &ma, const Mesh &mf, int H);
+// Whether each is faster than the separate launches for this many rows.
+bool forward_chain_pays(const Mesh &ma, int rows, bool backward);
+bool backward_chain_pays(const Mesh &ma, int layers, int rows);
 struct ForwardChain {
     int rows;
     Mesh ma, mf;

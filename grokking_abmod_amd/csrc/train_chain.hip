@@ -15,13 +15,13 @@
 // kernel in train.hip on the same operands in the same order, and every stored
 // activation and partial sum is the one that kernel stores, so the results are
 // the same bits.  The backward keeps the sums of five stacks' weight gradients
-// in registers, which limits the depths (kChainSums).
+// in registers, which limits its depths (kChainSums).
 //
 // One AdamW update, separate launches against these: 256 rows of width 32 (the
-// demo corpus) 212 us and 198, 2048 rows of width 128 (512 equations) 284 and
-// 251.  A middle launch now takes 10 us forward and 19 us backward at width 32,
-// 19 and 31 at width 128.  Without the loads at the front (each stack's behind
-// the one before) the updates took 219 and 275.
+// demo corpus, attention by waves) 212 us and 198, 2048 rows of width 128 (512
+// equations) 284 and 251.  A middle launch takes 10 us forward and 19 us backward
+// at width 32, 19 and 31 at width 128.  Without the loads at the front (each
+// stack's behind the one before) the updates took 219 and 275.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -32,7 +32,7 @@ namespace meshgpt::kern::train {
 namespace {
 
 // Registers for weight-gradient sums: two a layer and channel of a lane.
-constexpr int kChainSums = 112;
+constexpr int kChainSums = 96;
 
 // Loads above stay above: a chain's operands are all on their way before its
 // first product, so that it waits for memory once and not once a stack.
@@ -426,20 +426,28 @@ bool chain_fits(const Mesh &ma, const Mesh &mf, int H) {
     return hd >= 2 && hd <= 64 && (hd & (hd - 1)) == 0 && by_chain_shape(ma, mf, [](auto, auto, auto) {});
 }
 
-// Against the separate launches, an AdamW update (us, chain and separate).  Few
-// rows and shallow stacks gain the launches: W64, four layers and six, 256 rows
-// 130 and 138, 4096 220 and 237.  A wave takes its rows one after another, so
-// the gain is gone where every SIMD has several: W128, 4096 rows 307 and 321,
-// 8192 507 and 504, 16384 844 and 820; W32 neighbour 8192 310 and 317, butterfly
-// 16384 513 and 497.  Butterfly strides cost the shuffles of W128 more than the
-// launches of few rows (256 rows 181 and 175, 1024 204 and 209), and the stacks
-// of up to eight layers, whose sums fill the registers, gain in between only (W64,
-// seven layers: 512 159 and 155, 2048 197 and 205, 6144 336 and 334; butterfly 2048
-// 210 and 208).
-bool chain_pays(const Mesh &ma, const Mesh &mf, int rows) {
-    if (ma.depth > 4) return !ma.butterfly && rows >= 1536 && rows <= 4096;
-    if (ma.W > 64) return rows <= 4096 && !(ma.butterfly && rows < 512);
-    return rows <= 8192;
+// The backward keeps the sums of five stacks in registers.
+bool backward_chain_fits(const Mesh &ma, const Mesh &mf, int H) { return ma.depth <= 4 && chain_fits(ma, mf, H); }
+
+// An AdamW update (a captured step) or, without a backward, cross_entropy against
+// the separate launches: the chain stores what they store and reads what one of
+// them reads, so it is ahead at most sizes (1024 to 131072 rows 0.91 to 0.99 of an
+// update and 0.79 to 0.96 of a cross_entropy).  Behind it is by the shuffles of
+// butterfly strides where few rows wait for them: W64, seven layers, 256 rows 1.03
+// of an update; W128, four, 1.01 to 1.04.
+bool forward_chain_pays(const Mesh &ma, int rows, bool backward) {
+    return !backward || !ma.butterfly || rows >= 1024 || (ma.depth <= 4 && ma.W <= 64);
+}
+
+// A wave takes its rows one after another and one workgroup's registers fill a
+// SIMD, so the launches saved are lost again where every SIMD has several rows.
+// An update with the forward chain, with this one as well (of the separate
+// launches' time): W32 256 rows 0.975 and 0.982, 2048 0.968 and 0.928, 4096 0.937 and
+// 0.952; W128 256 rows 0.996 and 1.033 (six blocks 0.978 and 0.941), 1024 0.973 and 0.947, 4096 0.950 and 0.939,
+// 8192 0.947 and 0.991.  Stacks of up to eight layers had a form too and gained
+// nothing at any size.
+bool backward_chain_pays(const Mesh &ma, int layers, int rows) {
+    return ma.W > 64 ? (rows >= 512 || layers >= 4) && rows <= 4096 : rows <= 3072;
 }
 
 void forward_chain(const ForwardChain &a, hipStream_t stream) {
@@ -453,7 +461,7 @@ void backward_chain(const BackwardChain &a, std::vector<GradReduce> *reductions,
                     hipStream_t stream) {
     const int groups = mesh_wave_groups(a.rows);
     by_chain_shape(a.ma, a.mf, [&](auto C, auto A, auto F) {
-        constexpr int CC = decltype(C)::value, AA = decltype(A)::value, FF = decltype(F)::value;
+        constexpr int CC = decltype(C)::value, AA = std::min(decltype(A)::value, 4), FF = decltype(F)::value;
         static_assert(2 * CC * (4 * AA + FF) <= kChainSums, "weight-gradient sums stay in registers");
         const size_t lds = size_t(kThreads / 64) * std::max(a.ma.depth, a.mf.depth) * a.ma.W * 2 * sizeof(float);
         hipLaunchKernelGGL((backward_chain_kernel<CC, AA, FF>), dim3(unsigned(groups)), dim3(kThreads), lds, stream, a);

@@ -204,7 +204,9 @@ void window_routes() {
 
 // Every launch of the training chain has the shape that its kernel divides by.
 void chain_shapes() {
+    setenv("MG_FORCE_TRAIN_CHAIN", "1", 1);
     MeshGpt m(0, shape(128, 4, 32, 3), 7);
+    unsetenv("MG_FORCE_TRAIN_CHAIN");
     size_t launches = 0;
     fake::on_launch = [&](const fake::Launch &l) {
         if (l.kernel.find("backward_chain_kernel") == std::string::npos) return;
@@ -251,27 +253,36 @@ void scratch_limits() {
     fake::memory = size_t(1) << 33;
 }
 
-// The training chain is taken for the row counts at which it was measured faster.
+// The training chains are taken for the row counts at which they were measured
+// faster, the forward one in every cross_entropy.
 void chain_routes() {
     struct Case {
         size_t W, A, F, rows;
-        bool butterfly, chain;
+        bool butterfly, forward, backward;
     };
-    const Case cases[] = {{32, 4, 6, 256, false, true},     {64, 4, 6, 8192, true, true},    {32, 4, 6, 16384, true, false},
-                          {128, 4, 6, 64, false, true},     {128, 4, 6, 2048, true, true},   {128, 4, 6, 256, true, false},
-                          {128, 4, 6, 16384, false, false}, {64, 7, 7, 256, false, false},   {64, 7, 7, 2048, false, true},
-                          {64, 7, 7, 2048, true, false},    {64, 7, 7, 16384, false, false}, {128, 5, 5, 2048, false, false}};
+    const Case cases[] = {
+        {32, 4, 6, 256, false, true, true},    {64, 4, 6, 256, true, true, true},     {32, 4, 6, 4096, true, true, false},
+        {128, 4, 6, 64, false, true, false},   {128, 4, 6, 2048, true, true, true},   {128, 4, 6, 256, true, false, false},
+        {128, 4, 6, 8192, false, true, false}, {64, 7, 7, 256, false, true, false},   {64, 7, 7, 2048, false, true, false},
+        {64, 7, 7, 256, true, false, false},   {64, 7, 7, 2048, true, true, false},   {128, 5, 5, 2048, false, false, false}};
     for (const Case &c : cases) {
         GptConfig g = shape(c.W, 4, 32, 1, c.A, c.F);
         g.connectivity = c.butterfly ? MeshConnectivity::Butterfly : MeshConnectivity::Neighbor;
         MeshGpt m(0, g, 7);
-        bool chain = false;
-        fake::on_launch = [&](const fake::Launch &l) { chain |= l.kernel.find("chain_kernel") != std::string::npos; };
+        bool forward = false, backward = false;
+        fake::on_launch = [&](const fake::Launch &l) {
+            forward |= l.kernel.find("forward_chain_kernel") != std::string::npos;
+            backward |= l.kernel.find("backward_chain_kernel") != std::string::npos;
+        };
+        const std::string what = "W" + std::to_string(c.W) + ", " + std::to_string(c.A) + " layers, " +
+                                 std::to_string(c.rows) + " rows" + (c.butterfly ? ", butterfly" : "");
         const std::vector<uint32_t> tokens(c.rows, 1);
         m.train_batch(tokens.data(), tokens.data(), c.rows, 4, {});
+        expect(forward == c.forward && backward == c.backward, what);
+        forward = false;
+        m.cross_entropy(tokens.data(), tokens.data(), c.rows, 4);
+        expect(forward == (c.A <= 4 || c.W <= 64), what + ", the loss alone");
         fake::on_launch = nullptr;
-        expect(chain == c.chain, "W" + std::to_string(c.W) + ", " + std::to_string(c.A) + " layers, " +
-                                     std::to_string(c.rows) + " rows" + (c.butterfly ? ", butterfly" : ""));
     }
 }
 
