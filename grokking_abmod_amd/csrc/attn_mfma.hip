@@ -29,12 +29,12 @@
 
 #include "attn_range.hpp"
 #include "kernels.hpp"
+#include "lds_dma.hpp"
 
 namespace meshgpt::kern {
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) float lds_f32;
 
 // (f64(1e-12f))^2 rounded to f32: the XSA norm floor of reference.rs:591.
 constexpr float kXsaNormFloor = float(double(1e-12f) * double(1e-12f));
@@ -43,33 +43,6 @@ constexpr float kXsaNormFloor = float(double(1e-12f) * double(1e-12f));
 // B[l / 16][l % 16] and holds D[4 (l / 16) + r][l % 16] in element r.
 __device__ __forceinline__ v4f mfma16(float a, float b, v4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// LDS[base + 16 * lane .. +16) = g[0..4) for every lane of the wave; base is
-// wave-uniform.  Earlier LDS reads complete first; m0 is preserved.
-__device__ __forceinline__ void dma16(const float *g, float *base) {
-    const uint32_t m = __builtin_amdgcn_readfirstlane(uint32_t(size_t((lds_f32 *)base)));
-    uint32_t save;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %1\n\t"
-        "s_waitcnt lgkmcnt(0)\n\t"
-        "global_load_lds_dwordx4 %2, off\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(save)
-        : "s"(m), "v"(g)
-        : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// A workgroup barrier that waits for LDS operations only (in-flight global
-// loads, such as the next tile's, keep flying).
-__device__ __forceinline__ void barrier_lds() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 __device__ __forceinline__ float xor_lanes(float v, int mask) {

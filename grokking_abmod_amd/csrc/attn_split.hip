@@ -60,6 +60,7 @@
 
 #include "attn_range.hpp"
 #include "kernels.hpp"
+#include "lds_dma.hpp"
 
 namespace meshgpt::kern {
 namespace {
@@ -68,7 +69,6 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) float lds_f32;
 
 // (f64(1e-12f))^2 rounded to f32: the XSA norm floor of reference.rs:591.
 constexpr float kXsaNormFloor = float(double(1e-12f) * double(1e-12f));
@@ -209,26 +209,6 @@ attn_split_prepare_kernel(KvView kv, int n, int tiles, _Float16 *__restrict__ pl
                                                  : make_int2(-kNoRow, kNoRow);
 }
 
-// LDS[base + 16 * lane .. +16) = g[0..4) for every lane of the wave; base is
-// wave-uniform.  Earlier LDS reads complete first; m0 is preserved.
-__device__ __forceinline__ void dma16(const void *g, void *base) {
-    const uint32_t m = __builtin_amdgcn_readfirstlane(uint32_t(size_t((lds_f32 *)base)));
-    uint32_t save;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %1\n\t"
-        "s_waitcnt lgkmcnt(0)\n\t"
-        "global_load_lds_dwordx4 %2, off\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(save)
-        : "s"(m), "v"(g)
-        : "memory");
-}
-
-// The wave's loads into LDS have landed; its LDS reads are done, and a barrier.
-__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-__device__ __forceinline__ void barrier_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // A workgroup of WAVES waves takes 32 WAVES queries of one (sequence, head),
 // 32 a wave (query lane % 32), and streams its key tiles through LDS, double
 // buffered.  Per tile a wave forms the transposed scores S^T = K Q^T (two
@@ -286,7 +266,7 @@ attn_split_kernel(Shape s, const float *__restrict__ q, KvView kv, const _Float1
         // Probabilities of this tile are in units of 2^-unit; a tile of zeros
         // adds to their sum only.
         const int top = tile_range[t].x, unit = top == -kNoRow ? 14 : 14 + top - E;
-        wait_vm();
+        wait_vm<0>();
         barrier_lds();  // tile t has landed, and every wave is done with tile t - 1
         if (t + 1 < ntile) issue(t + 1);
         const int t0 = t * kBK;

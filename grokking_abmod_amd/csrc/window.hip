@@ -19,8 +19,10 @@
 //  - every wave makes the same draw from the logits in LDS, so the new token
 //    needs no hand-off.
 // Two barriers a block and two for the head remain.  240 tokens from a prompt of
-// 17 (W32, context 32, two blocks): 11.76 ms before, 1.77 now; W128, context 32:
-// 21.7 and 3.9; W128, context 64: 17.3 and 9.5.
+// 17 (W32, context 32, two blocks), one sequence: 11.7 ms before, 1.75 now; W64,
+// context 32: 13.1 and 2.4; W128, context 64: 17.5 and 8.1.  The last family's
+// sixteen waves leave 128 registers a lane, and five of its six forms spill two to
+// five of them (12-24 bytes of scratch a lane).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
