@@ -5,7 +5,7 @@
 // What bounds it is the chain of dependent steps of one token, not work: the
 // default model's window (32 rows of 32 channels, two blocks) is 0.2 MFLOP.  As
 // one launch per operator a token took seven launches of 3-9 us (48 us); in one
-// launch it takes 7.3 us, about half of it the mesh layers (a wave issues some
+// launch it takes 7.1 us, about half of it the mesh layers (a wave issues some
 // 45 dependent instructions for a layer of q, k and v).  A workgroup keeps a
 // sequence's window to itself from token to token:
 //  - a row lies in 16 lanes, channel CPL l + j in register j of lane l (CPL =
