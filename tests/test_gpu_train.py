@@ -184,7 +184,9 @@ CHAIN = [(dict(width=32, heads=4, layers=2), 8, 32), (dict(width=128, heads=4, l
          (dict(width=128, heads=8, layers=2, connectivity=1, rope=0), 9, 9),
          (dict(width=128, heads=4, layers=2, qk_norm=0), 9, 9), (dict(width=64, heads=1, layers=2, xsa=0), 4, 70),
          (dict(width=128, heads=4, layers=2, attention_mesh_depth=5), 9, 9),
-         (dict(width=32, heads=4, layers=2, ffn_mesh_depth=9), 9, 9), (dict(width=32, heads=4, embedding=1), 700, 3)]
+         (dict(width=32, heads=4, layers=2, ffn_mesh_depth=9), 9, 9), (dict(width=32, heads=4, embedding=1), 700, 3),
+         (dict(width=32, heads=4, layers=2), 1100, 4), (dict(width=64, heads=4, layers=3, attention_mesh_depth=7), 300, 8),
+         (dict(width=128, heads=4, layers=2, connectivity=1), 60, 4)]
 
 
 @pytest.mark.parametrize("cfg,b,s", CHAIN, ids=[f"{i}-W{c['width']}-{b}x{s}" for i, (c, b, s) in enumerate(CHAIN)])
@@ -193,17 +195,21 @@ def test_chained_launches_give_the_separate_launches_bits(cfg, b, s, monkeypatch
     rng = np.random.default_rng(b)
     x, y = (rng.integers(0, 11, b * s).astype(np.uint32) for _ in range(2))
     got = {}
-    for off in ("0", "1"):
+    # Both chains also where the separate launches are faster, none, and what the
+    # row counts choose (the last three shapes: one chain of the two, or neither).
+    for off, force in (("0", "1"), ("1", "0"), ("0", "0")):
         monkeypatch.setenv("MG_DISABLE_TRAIN_CHAIN", off)
-        monkeypatch.setenv("MG_FORCE_TRAIN_CHAIN", "1")  # also where the separate launches are faster
+        monkeypatch.setenv("MG_FORCE_TRAIN_CHAIN", force)
         with G.MeshGpt(0, g, 7) as model:
             model.set_parameters(np.random.default_rng(3).uniform(
                 -1.0, 1.0, G.parameter_count(g)).astype(np.float32))
             first = model.loss_and_gradient(x, y, s)
             losses = [model.train_batch(x, y, s) for _ in range(3)]
-            got[off] = (first[0], first[1], losses, model.parameters(), model.cross_entropy(x, y, s))
-    assert got["0"][0] == got["1"][0] and got["0"][2] == got["1"][2] and got["0"][4] == got["1"][4]
-    assert np.array_equal(got["0"][1], got["1"][1]) and np.array_equal(got["0"][3], got["1"][3])
+            got[off + force] = (first[0], first[1], losses, model.parameters(), model.cross_entropy(x, y, s))
+    separate = got.pop("10")
+    for mode, chain in got.items():
+        assert chain[0] == separate[0] and chain[2] == separate[2] and chain[4] == separate[4], mode
+        assert np.array_equal(chain[1], separate[1]) and np.array_equal(chain[3], separate[3]), mode
 
 
 # Stacks deeper than the 16 layers of one kernel launch, in the wave (width
