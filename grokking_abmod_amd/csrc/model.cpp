@@ -533,6 +533,17 @@ struct MeshGpt::Impl {
         if (!grow_b && !grow_t) return;
         sync();
         drop_graph();
+        try {
+            grow_decode(b, t, grow_b);
+        } catch (...) {
+            // Some buffers are gone: the next batch, of any size, allocates them.
+            batch_cap = tcap = batch = length = 0;
+            cached = kNoCache;
+            throw;
+        }
+    }
+
+    void grow_decode(size_t b, size_t t, bool grow_b) {
         if (grow_b) {
             batch_cap = std::max(b, batch_cap);
             const size_t cache = size_t(cfg.layers) * layer_cache_elems() * 4;

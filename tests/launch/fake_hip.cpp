@@ -46,6 +46,12 @@ hipError_t launch(const void *f, dim3 grid, dim3 block, void **args) {
     return hipSuccess;
 }
 
+}  // namespace
+
+size_t fake::size_of(const void *p) { return blocks()[const_cast<void *>(p)]; }
+
+namespace {
+
 template <class T>
 hipError_t handle(T *out) {
     *out = reinterpret_cast<T>(std::malloc(1));

@@ -25,5 +25,7 @@ extern std::string refuse;
 extern bool refuse_attributes;
 // Device bytes there are (hipMalloc fails past them) and the most in use so far.
 extern size_t memory, peak;
+// Bytes of the block that begins at p.
+size_t size_of(const void *p);
 
 }  // namespace fake

@@ -353,7 +353,31 @@ void threads_reading() {
     expect(wrong == 0, std::to_string(wrong) + " reads held another's data");
 }
 
+// A batch that finds no memory leaves a model that smaller batches can use, with
+// all the buffers that their launches name.
+void batch_without_memory() {
+    for (size_t room : {0, 1 << 20, 1 << 22, 1 << 24}) {
+        MeshGpt m(0, shape(32, 4, 32), 7, 2);
+        fake::peak = 0;
+        generate(m, 2, 5, 8);
+        fake::memory = fake::peak + room;
+        expect(status_of([&] { generate(m, 100000, 5, 8); }) == kOutOfMemory, "no memory for a batch");
+        size_t windows = 0;
+        fake::on_launch = [&](const fake::Launch &l) {
+            if (l.kernel.find("window_kernel") == std::string::npos) return;
+            const auto *a = static_cast<const kern::WindowArgs *>(l.args[0]);
+            expect(a->tokens && a->len && a->rng && a->logits && a->flags && a->kc && a->vc, "every buffer is there");
+            expect(a->layer_elems * 2 * 4 <= fake::size_of(a->kc), "the cache holds the layers");
+            ++windows;
+        };
+        expect(status_of([&] { generate(m, 2, 5, 8); }) == 0 && windows == 1, "a smaller batch after it");
+        fake::on_launch = nullptr;
+        fake::memory = size_t(1) << 33;
+    }
+}
+
 const std::map<std::string, void (*)()> kChecks = {
+    {"batch_without_memory", batch_without_memory},
     {"threads_reading", threads_reading},
     {"no_batch", no_batch},
     {"finite_checks", finite_checks},
