@@ -528,13 +528,30 @@ struct MeshGpt::Impl {
         if (out == nullptr || capacity < n) throw Error("output buffer is too small");
     }
 
+    // grow(), and once more without the scratch that earlier prefills could have
+    // done without, where there is no memory.  What grow() did before it threw
+    // stands the second time.
+    template <class F>
+    void with_room(F grow) {
+        try {
+            grow();
+            return;
+        } catch (const Error &e) {
+            if (e.status != kOutOfMemory || !(wsplit.p || wlast.p)) throw;
+        }
+        sync();
+        wsplit.release();
+        wlast.release();
+        grow();
+    }
+
     void ensure_decode(size_t b, size_t t) {
         const bool grow_b = b > batch_cap, grow_t = t > tcap;
         if (!grow_b && !grow_t) return;
         sync();
         drop_graph();
         try {
-            grow_decode(b, t, grow_b);
+            with_room([&] { grow_decode(b, t, grow_b); });
         } catch (...) {
             // Some buffers are gone: the next batch, of any size, allocates them.
             batch_cap = tcap = batch = length = 0;
@@ -583,6 +600,10 @@ struct MeshGpt::Impl {
     }
 
     void ensure_workspace(size_t rows, size_t out_rows, bool kv) {
+        with_room([&] { grow_workspace(rows, out_rows, kv); });
+    }
+
+    void grow_workspace(size_t rows, size_t out_rows, bool kv) {
         const size_t W = cfg.width;
         wx.ensure(rows * W * 4);
         wxn.ensure(rows * W * 4);
@@ -915,17 +936,20 @@ struct MeshGpt::Impl {
     void train_prepare(size_t n) {
         namespace T = kern::train;
         const size_t P = layout.count();
-        bool grown = tact.ensure(train_plan(n).total * 4);
-        grown |= tpart.ensure(train_partial_floats(n) * 4);
-        grown |= tgrad.ensure(P * 4);
         static_assert(sizeof(T::StepScalars) <= kTrainTokensAt, "step scalars precede the tokens");
-        grown |= tin.ensure(kTrainTokensAt + 8 * n);
-        tstage.ensure(kTrainTokensAt + 12 * n);
-        if (tm.ensure(P * 4) | tv.ensure(P * 4)) {
-            grown = true;
-            check(hipMemsetAsync(tm.p, 0, tm.bytes, stream), "clear moments");
-            check(hipMemsetAsync(tv.p, 0, tv.bytes, stream), "clear moments");
-        }
+        bool grown = false;
+        with_room([&] {
+            grown |= tact.ensure(train_plan(n).total * 4);
+            grown |= tpart.ensure(train_partial_floats(n) * 4);
+            grown |= tgrad.ensure(P * 4);
+            grown |= tin.ensure(kTrainTokensAt + 8 * n);
+            tstage.ensure(kTrainTokensAt + 12 * n);
+            if (tm.ensure(P * 4) | tv.ensure(P * 4)) {
+                grown = true;
+                check(hipMemsetAsync(tm.p, 0, tm.bytes, stream), "clear moments");
+                check(hipMemsetAsync(tv.p, 0, tv.bytes, stream), "clear moments");
+            }
+        });
         if (grown) drop_train_graph();
     }
 

@@ -9,7 +9,7 @@ namespace fake {
 std::function<void(const Launch &)> on_launch;
 std::string refuse;
 bool refuse_attributes = false;
-size_t memory = size_t(1) << 33, peak = 0;
+size_t memory = size_t(1) << 33, used = 0, peak = 0;
 }  // namespace fake
 
 namespace {
@@ -22,7 +22,6 @@ std::map<void *, size_t> &blocks() {
     static std::map<void *, size_t> sizes;
     return sizes;
 }
-size_t used = 0;
 hipError_t last = hipSuccess;
 
 // As the runtime does: a failure stays until hipGetLastError reports it.
@@ -106,15 +105,15 @@ hipError_t hipGetLastError(void) {
 const char *hipGetErrorString(hipError_t) { return "refused by the test"; }
 
 hipError_t hipMalloc(void **p, size_t n) {
-    if (used + n > fake::memory) return result(hipErrorOutOfMemory);
+    if (fake::used + n > fake::memory) return result(hipErrorOutOfMemory);
     *p = std::calloc(n, 1);
     blocks()[*p] = n;
-    used += n;
-    fake::peak = std::max(fake::peak, used);
+    fake::used += n;
+    fake::peak = std::max(fake::peak, fake::used);
     return hipSuccess;
 }
 hipError_t hipFree(void *p) {
-    used -= blocks()[p];
+    fake::used -= blocks()[p];
     blocks().erase(p);
     std::free(p);
     return hipSuccess;

@@ -23,8 +23,8 @@ extern std::function<void(const Launch &)> on_launch;
 extern std::string refuse;
 // hipFuncSetAttribute fails.
 extern bool refuse_attributes;
-// Device bytes there are (hipMalloc fails past them) and the most in use so far.
-extern size_t memory, peak;
+// Device bytes there are (hipMalloc fails past them), in use, and the most so far.
+extern size_t memory, used, peak;
 // Bytes of the block that begins at p.
 size_t size_of(const void *p);
 

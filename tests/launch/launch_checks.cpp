@@ -251,6 +251,30 @@ void scratch_limits() {
     expect(status_of(prefill) == 0, "a prefill without the last rows' buffers");
     expect(!launched("last_merge_kernel"), "with every row in the last block");
     fake::memory = size_t(1) << 33;
+
+    // What an earlier prefill left there makes room for a later call of any kind.
+    const std::vector<uint32_t> tokens(12 * 500, 1);
+    std::vector<float> out(12 * 500 * 64);
+    std::vector<uint32_t> generated(40 * 8);
+    const std::function<void(MeshGpt &)> later[] = {
+        [&](MeshGpt &m) { m.logits(tokens.data(), 12 * 500, 500, false, out.data(), out.size()); },
+        [&](MeshGpt &m) { m.generate_tokens(tokens.data(), 40, 4, 4, 0.0f, 7, generated.data()); },
+        [&](MeshGpt &m) { m.train_batch(tokens.data(), tokens.data(), 64, 32, {}); },
+    };
+    for (const auto &call : later) {
+        size_t need = 0;
+        for (const char *off : {"1", "0"}) {
+            setenv("MG_DISABLE_SPLIT_PREFILL", off, 1);
+            MeshGpt m(0, shape(256, 4, 640), 7, 8);
+            fake::peak = 0;
+            m.prefill(prompts.data(), 8, 600, 0.0f, 7, 620);
+            if (need) fake::memory = std::max(need, fake::used);
+            expect(status_of([&] { call(m); }) == 0, "a call in the memory that it took without planes");
+            need = fake::peak;
+            fake::memory = size_t(1) << 33;
+        }
+        unsetenv("MG_DISABLE_SPLIT_PREFILL");
+    }
 }
 
 // The training chains are taken for the row counts at which they were measured
