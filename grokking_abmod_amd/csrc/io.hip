@@ -35,6 +35,19 @@ __global__ void __launch_bounds__(256) nonfinite_kernel(const float *__restrict_
     if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(flag, 1);
 }
 
+__global__ void __launch_bounds__(256) layer_gains_kernel(const float2 *__restrict__ w, int W, float *__restrict__ gain) {
+    __shared__ float waves[4];
+    float top = 0.0f;
+    for (int c = int(threadIdx.x); c < W; c += 256) {
+        const float2 p = w[size_t(blockIdx.x) * W + c];
+        top = fmaxf(top, fabsf(p.x) + fabsf(p.y));
+    }
+    for (int k = 1; k < 64; k <<= 1) top = fmaxf(top, __shfl_xor(top, k, 64));
+    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = top;
+    __syncthreads();
+    if (threadIdx.x == 0) gain[blockIdx.x] = fmaxf(fmaxf(waves[0], waves[1]), fmaxf(waves[2], waves[3]));
+}
+
 }  // namespace
 
 void start_rows(const uint32_t *prompts, int batch, int n, uint32_t *tokens, size_t stride, int *len, uint64_t *rng,
@@ -46,6 +59,11 @@ void start_rows(const uint32_t *prompts, int batch, int n, uint32_t *tokens, siz
 void gather_rows(const uint32_t *tokens, size_t stride, int batch, int n, uint32_t *out, hipStream_t stream) {
     if (batch && n)
         hipLaunchKernelGGL(gather_rows_kernel, dim3(batch), dim3(256), 0, stream, tokens, stride, n, out);
+}
+
+void layer_gains(const float *w, int layers, int W, float *gain, hipStream_t stream) {
+    hipLaunchKernelGGL(layer_gains_kernel, dim3(layers), dim3(256), 0, stream, reinterpret_cast<const float2 *>(w), W,
+                       gain);
 }
 
 void nonfinite(const float *x, size_t n, int *flag, hipStream_t stream) {

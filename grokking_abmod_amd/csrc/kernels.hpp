@@ -28,6 +28,7 @@ struct Shape {
     int rope;      // operator switches (config.rs:33-35): 1 on, 0 off
     int qk_norm;
     int xsa;
+    int wide;      // 1: a mesh value may pass the range of values carried times log2(e)
 };
 
 // Which rows a launch covers.  Row r belongs to sequence r / rows_per_seq and
@@ -294,6 +295,8 @@ void start_rows(const uint32_t *prompts, int batch, int n, uint32_t *tokens, siz
                 uint64_t seed, int *flags, hipStream_t stream);
 // out[b n ..) = the first n tokens of row b.
 void gather_rows(const uint32_t *tokens, size_t stride, int batch, int n, uint32_t *out, hipStream_t stream);
+// gain[l] = the largest |w0| + |w1| of mesh layer l (W weight pairs each).
+void layer_gains(const float *w, int layers, int W, float *gain, hipStream_t stream);
 // *flag = 1 when a value of x[0..n) is not finite, else 0.
 void nonfinite(const float *x, size_t n, int *flag, hipStream_t stream);
 // y[i] = the sampler's f32 exp of x[i] (for verification).

@@ -91,6 +91,25 @@ struct PinnedBuf {
     }
 };
 
+// The bits of the largest |v|, in four chains (half the time of one).
+uint32_t largest_bits(const float *v, size_t n) {
+    auto at = [&](size_t i) {
+        uint32_t b;
+        std::memcpy(&b, v + i, 4);
+        return b & 0x7fffffffu;
+    };
+    uint32_t a = 0, b = 0, c = 0, d = 0;
+    size_t i = 0;
+    for (; i + 4 <= n; i += 4) {
+        a = std::max(a, at(i));
+        b = std::max(b, at(i + 1));
+        c = std::max(c, at(i + 2));
+        d = std::max(d, at(i + 3));
+    }
+    for (; i < n; ++i) a = std::max(a, at(i));
+    return std::max(std::max(a, b), std::max(c, d));
+}
+
 int floor_log2(size_t x) {
     int r = 0;
     while (x >>= 1) ++r;
@@ -194,6 +213,7 @@ struct MeshGpt::Impl {
     kern::train::StepScalars hyper{};  // host copy uploaded before each step (kept alive for the async copy)
     float beta1_power = 1.0f, beta2_power = 1.0f;
     bool derived_stale = false;  // E and the decode tables lag the weights
+    float largest_weight = -1.0f;  // of the parameters as last set, negative after training
     // The captured training step and what it was captured for.
     struct TrainKey {
         size_t n = 0, sequence = 0;
@@ -375,7 +395,7 @@ struct MeshGpt::Impl {
         E.ensure(W * cfg.vocab_size * 4);
         vpad = int((cfg.vocab_size + 3) / 4 * 4);
         Et.ensure(W * size_t(vpad) * 4);
-        params.ensure(layout.count() * 4);
+        params.ensure((layout.count() + stack_layers()) * 4);
         std::vector<float> initial = layout.initialize(cfg, seed);
         set_parameters(initial.data(), initial.size());
         ensure_decode(std::max<size_t>(max_batch, 1), 1);
@@ -383,11 +403,13 @@ struct MeshGpt::Impl {
 
     void set_parameters(const float *values, size_t n) {
         if (n != layout.count()) throw Error("parameter count does not match GPT configuration");
-        validate_finite(values, n, "parameters");
+        const uint32_t top = largest_bits(values, n);  // a value that is not finite has the largest
+        if (top >= 0x7f800000u) validate_finite(values, n, "parameters");
         layout.validate_constraints(cfg, values);
         activate();
         check(hipMemcpyAsync(params.p, values, n * 4, hipMemcpyHostToDevice, stream), "upload parameters");
         reset_optimizer();
+        std::memcpy(&largest_weight, &top, 4);
         refresh_derived();
     }
 
@@ -432,8 +454,54 @@ struct MeshGpt::Impl {
                                         layout.groups[layout.blocks[0].query].offset, q0.as<float>(), stream);
             }
         }
+        // Twice the largest weight bounds every layer's gain, which settles all but
+        // deep or far-flung stacks; the layers' own gains settle those, and weights
+        // that the host does not have.  They lie behind the weights and travel
+        // through the upload's staging (which the stream has read by then).
+        const float coarse = 2.0f * largest_weight;
+        const bool narrow = coarse >= 0.0f && mesh_bound([&](size_t) { return coarse; }) <= 1e38;
+        const size_t gains = stack_layers();
+        const bool known = !narrow && gains * 4 <= kUpload;
+        if (known) {
+            kern::layer_gains(params.as<float>() + layout.groups[layout.blocks[0].query].offset, int(gains), shape.W,
+                              params.as<float>() + n, stream);
+            check(hipMemcpyAsync(hio.p, params.as<float>() + n, gains * 4, hipMemcpyDeviceToHost, stream),
+                  "download gains");
+        }
         sync();
+        shape.wide = env_int("MG_FORCE_WIDE", 0) ||
+                     !(narrow || (known && mesh_bound([&](size_t l) { return hio.as<float>()[l]; }) <= 1e38));
         derived_stale = false;
+    }
+
+    size_t stack_layers() const { return cfg.layers * (4 * cfg.attention_mesh_depth + cfg.ffn_mesh_depth); }
+
+    // A bound on every value inside the blocks' meshes from gain(l), the largest
+    // |w0| + |w1| of layer l of them all.  Prefill and window kernels carry these values
+    // times log2(e), which takes a product off each, unless that could make a
+    // finite one infinite.  RMSNorm's rows are at most sqrt(W) in size, an
+    // attention row mixes value rows, and XSA adds at most their 2-norm.
+    template <class Gain>
+    double mesh_bound(Gain gain) const {
+        const size_t A = cfg.attention_mesh_depth, F = cfg.ffn_mesh_depth;
+        size_t at = 0;
+        double worst = 0.0;
+        auto stack = [&](double top, size_t depth) {
+            for (size_t l = 0; l < depth; ++l) {
+                top = std::max(top, 1.0) * double(gain(at++));
+                worst = std::max(worst, top);
+            }
+            return top;
+        };
+        const double row = std::sqrt(double(cfg.width));
+        for (size_t b = 0; b < cfg.layers; ++b) {
+            stack(row, A);
+            stack(row, A);
+            const double value = stack(row, A);
+            stack(value * (1.0 + std::sqrt(double(cfg.head_width()))), A);
+            stack(row, F);
+        }
+        return worst;
     }
 
     void sync() {
@@ -1306,6 +1374,7 @@ struct MeshGpt::Impl {
             enqueue();
         }
         derived_stale = true;
+        largest_weight = -1.0f;
         const double loss = train_loss(n, supervised);  // throws (weights unchanged) on a non-finite loss
         beta1_power = p1;
         beta2_power = p2;

@@ -17,17 +17,18 @@
 // scratch; head reductions (QK-Norm, XSA) and the RoPE pair exchange stay
 // inside a wave (a head is hd <= 64 consecutive channels = consecutive lanes).
 //
-// What bounds it is instruction issue: six VALU instructions a value and layer
-// (product, multiply-add, ELU's product, exponential, sum and maximum) and an LDS
-// write and read of the value, behind a barrier each layer that only other
-// workgroups' waves on the SIMD can fill.  Widths 512 and 1024 keep to 128
-// registers for four waves a SIMD; 128 and 256, with 16 rows a thread, would
-// spill and keep three.  A prefill of 256 x 128 rows (W1024, 12 blocks, 13 launches
-// of this kernel): 7.8 ms, 456 us a launch (8.84 and 527 with three waves).
-// Values carried times log2(e) save the ELU's product and take 7.68 ms (446), but a
-// finite value above 2.36e38 is infinite in those units.  Not kept either, timed
-// with them: strides of 256 and 512 from the thread's own registers (7.73 ms against
-// 7.63), weights loaded two layers ahead (7.74).
+// What bounds it is instruction issue: five VALU instructions a value and layer
+// (product, multiply-add, exponential, multiply-add, maximum; values are carried
+// times log2(e), or it is six) and an LDS write and read of the value, behind a
+// barrier each layer that only other workgroups' waves on the SIMD can fill.
+// Widths 512 and 1024 keep to 128 registers for four waves a SIMD; 128 and 256,
+// with 16 rows a thread, would spill and keep three.  A prefill of 256 x 128 rows
+// (W1024, 12 blocks, 13 launches of this kernel, 527 us each before and 446 now): 8.84 ms,
+// 7.94 with the scaled values alone, 7.68 with four waves as well.  Values above
+// 2.36e38 are infinite in these units, so models whose weights could reach them
+// (Shape::wide) run in their own: 7.8 ms, 456 us a launch.
+// Not kept: strides of 256 and 512 from the thread's own registers (7.73 ms), weights
+// loaded two layers ahead (7.74).
 #include <hip/hip_runtime.h>
 
 #include "dpp.hpp"
@@ -40,11 +41,22 @@ constexpr float kEps = 1e-5f;  // src/gpt/mod.rs:38
 // (f64(1e-12f))^2 rounded to f32: the XSA norm floor of reference.rs:591.
 constexpr float kXsaNormFloor = float(double(1e-12f) * double(1e-12f));
 
-__device__ __forceinline__ float elu_f(float z) {
-    // max(z, clamp(exp(z), 0, 1) - 1) with the NaN-propagating maximum, which
-    // keeps a NaN z NaN (kernels.hip's elu)
-    const float e = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(z * 1.4426950408889634f), 0.0f, 1.0f);
-    return __builtin_elementwise_maximum(z, e - 1.0f);
+constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
+
+// What a value is multiplied by on its way into the meshes and out of them:
+// SCALED ones are carried times log2(e), which the ELU's exponential would
+// otherwise multiply in (Shape::wide: their own units).
+template <bool SCALED>
+struct Units {
+    static constexpr float in = SCALED ? kLog2e : 1.0f, out = SCALED ? kLn2 : 1.0f;
+};
+
+// The ELU in these units, of t = z or z log2(e): max(z, clamp(exp(z), 0, 1) - 1)
+// with the NaN-propagating maximum, which keeps a NaN NaN (kernels.hip's elu).
+template <bool SCALED>
+__device__ __forceinline__ float elu_units(float t) {
+    const float e = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(SCALED ? t : t * kLog2e), 0.0f, 1.0f);
+    return __builtin_elementwise_maximum(t, SCALED ? __builtin_fmaf(e, kLog2e, -kLog2e) : e - 1.0f);
 }
 
 template <int W>
@@ -70,7 +82,7 @@ __device__ __forceinline__ int chunk_at(int c, int ch) {
     return c * C::R + 4 * ((ch + c / C::ROT) & (C::NCH - 1));
 }
 
-template <int W>
+template <int W, bool SCALED>
 struct Tile {
     using C = RowsCfg<W>;
     static constexpr int CPT = C::CPT, RG = C::RG;
@@ -115,8 +127,8 @@ struct Tile {
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
             for (int i = 0; i < RG; ++i) {
-                const float z = v[k][i] * w[k].x + p[k][i] * w[k].y;
-                v[k][i] = LAST ? z : elu_f(z);
+                const float t = v[k][i] * w[k].x + p[k][i] * w[k].y;
+                v[k][i] = LAST ? t : elu_units<SCALED>(t);
             }
     }
     template <bool LAST>
@@ -132,6 +144,7 @@ struct Tile {
     // A mesh stack on v in place: layer l maps v[c] to v[c] w0 + v[c + st] w1
     // with ELU on every layer but the last (reference.rs:422-453).
     // Butterfly strides double from 1 and wrap at W (W is a power of two).
+    // Values are in the meshes' units.
     __device__ void mesh(float (&v)[CPT][RG], const float2 *__restrict__ w, int depth, const Shape &s) {
         float2 wc[CPT];
 #pragma unroll
@@ -190,14 +203,15 @@ __device__ __forceinline__ float head_sum(float v, int hd) {
 // HD: the head width when it is 32 or 64 (DPP head sums), else 0.  Rows are
 // whole prefill sequences (Rows.len is null: a row's position is its index
 // within its sequence).
-template <int W, int HD>
+template <int W, int HD, bool SCALED>
 __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(BlockArgs a) {
     using C = RowsCfg<W>;
+    using U = Units<SCALED>;
     constexpr int CPT = C::CPT, RG = C::RG;
     __shared__ __align__(16) float lds[2 * C::TILE];
     __shared__ float red[4 * RG];
     const Shape &s = a.s;
-    Tile<W> t;
+    Tile<W, SCALED> t;
     t.lds = lds;
     t.red = red;
     t.parity = 0;
@@ -256,23 +270,29 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
                 }
             }
         }
+        if constexpr (SCALED) {
+#pragma unroll
+            for (int k = 0; k < CPT; ++k)
+#pragma unroll
+                for (int i = 0; i < RG; ++i) y[k][i] *= U::in;
+        }
         t.mesh(y, reinterpret_cast<const float2 *>(a.wproj), s.A, s);
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) x[k][i] += y[k][i];
+            for (int i = 0; i < RG; ++i) x[k][i] = __builtin_fmaf(y[k][i], U::out, x[k][i]);
         float inv[RG];
         t.row_inv_rms(x, inv);
         float n[CPT][RG];
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * inv[i];
+            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * (inv[i] * U::in);
         t.mesh(n, reinterpret_cast<const float2 *>(a.wffn), s.F, s);
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) x[k][i] += n[k][i];
+            for (int i = 0; i < RG; ++i) x[k][i] = __builtin_fmaf(n[k][i], U::out, x[k][i]);
     }
     if (post || a.embed) {
 #pragma unroll
@@ -284,7 +304,8 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
     }
     if (!a.xn && !pre) return;
 
-    // The next RMSNorm: the final one for the head, or the block's pre-norm.
+    // The next RMSNorm: the final one for the head, or the block's pre-norm,
+    // whose rows enter the meshes in their units.
     float n[CPT][RG];
     {
         float inv[RG];
@@ -301,7 +322,7 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
 #pragma unroll
-            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * inv[i];
+            for (int i = 0; i < RG; ++i) n[k][i] = x[k][i] * (inv[i] * U::in);
     }
 
     // Q, K and V meshes, one after another, each from the normalised rows.
@@ -329,7 +350,8 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
 #pragma unroll
                 for (int i = 0; i < RG; ++i) {
                     float q = v[k][i];
-                    if (s.qk_norm) q *= rsqrtf(head_sum<HD>(q * q, s.hd) * (1.0f / float(s.hd)) + kEps);
+                    q *= s.qk_norm ? rsqrtf(head_sum<HD>(q * q, s.hd) * (1.0f / float(s.hd)) + kEps * U::in * U::in)
+                                   : U::out;
                     if (s.rope) {
                         const float p = __shfl_xor(q, s.half, 64);
                         const float2 cs = a.rope[size_t(posof(i)) * s.half + (d < s.half ? d : d - s.half)];
@@ -337,6 +359,9 @@ __global__ void __launch_bounds__(256, RowsCfg<W>::WAVES) rows_block_kernel(Bloc
                     }
                     v[k][i] = q;
                 }
+            } else {
+#pragma unroll
+                for (int i = 0; i < RG; ++i) v[k][i] *= U::out;
             }
 #pragma unroll
             for (int i = 0; i < RG; ++i) {
@@ -396,24 +421,29 @@ bool rows_block_supported(const Shape &s) {
            64 % s.hd == 0;
 }
 
-template <int W>
+template <int W, bool SCALED>
 void launch_rows_block(const BlockArgs &a, hipStream_t stream) {
     const dim3 grid((a.ro.rows + RowsCfg<W>::R - 1) / RowsCfg<W>::R);
     if (a.s.hd == 32)
-        hipLaunchKernelGGL((rows_block_kernel<W, 32>), grid, dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((rows_block_kernel<W, 32, SCALED>), grid, dim3(256), 0, stream, a);
     else if (a.s.hd == 64)
-        hipLaunchKernelGGL((rows_block_kernel<W, 64>), grid, dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((rows_block_kernel<W, 64, SCALED>), grid, dim3(256), 0, stream, a);
     else
-        hipLaunchKernelGGL((rows_block_kernel<W, 0>), grid, dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((rows_block_kernel<W, 0, SCALED>), grid, dim3(256), 0, stream, a);
+}
+
+template <bool SCALED>
+void rows_block_units(const BlockArgs &a, hipStream_t stream) {
+    switch (a.s.W) {
+    case 128: launch_rows_block<128, SCALED>(a, stream); break;
+    case 256: launch_rows_block<256, SCALED>(a, stream); break;
+    case 512: launch_rows_block<512, SCALED>(a, stream); break;
+    default: launch_rows_block<1024, SCALED>(a, stream); break;
+    }
 }
 
 void rows_block(const BlockArgs &a, hipStream_t stream) {
-    switch (a.s.W) {
-    case 128: launch_rows_block<128>(a, stream); break;
-    case 256: launch_rows_block<256>(a, stream); break;
-    case 512: launch_rows_block<512>(a, stream); break;
-    default: launch_rows_block<1024>(a, stream); break;
-    }
+    a.s.wide ? rows_block_units<false>(a, stream) : rows_block_units<true>(a, stream);
 }
 
 void last_rows(const float *q, const float *x, int nseq, int n, int W, float *q_out, float *x_out, int *len,

@@ -6,7 +6,7 @@
 // default model's window (32 rows of 32 channels, two blocks) is 0.2 MFLOP.  As
 // one launch per operator a token took seven launches of 3-9 us (48 us); in one
 // launch it takes 7.1 us, about half of it the mesh layers (a wave issues some
-// 45 dependent instructions for a layer of q, k and v).  A workgroup keeps a
+// 40 dependent instructions for a layer of q, k and v).  A workgroup keeps a
 // sequence's window to itself from token to token:
 //  - a row lies in 16 lanes, channel CPL l + j in register j of lane l (CPL =
 //    W / 16), four rows a wave: a mesh layer's partner is another register, or
@@ -19,10 +19,10 @@
 //  - every wave makes the same draw from the logits in LDS, so the new token
 //    needs no hand-off.
 // Two barriers a block and two for the head remain.  240 tokens from a prompt of
-// 17 (W32, context 32, two blocks), one sequence: 11.7 ms before, 1.75 now; W64,
-// context 32: 13.1 and 2.4; W128, context 64: 17.5 and 8.1.  The last family's
-// sixteen waves leave 128 registers a lane, and five of its six forms spill two to
-// five of them (12-24 bytes of scratch a lane).
+// 17 (W32, context 32, two blocks), one sequence: 11.7 ms before, 1.70 now; W64,
+// context 32: 13.1 and 2.3; W128, context 64: 17.5 and 8.0.  The last family's
+// sixteen waves leave 128 registers a lane, and five of its six forms spill four to
+// eight of them (20-36 bytes of scratch a lane).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -40,16 +40,25 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr float kRmsEps = 1e-5f;  // src/gpt/mod.rs:38
 // (f64(1e-12f))^2 rounded to f32: the XSA norm floor of reference.rs:591
 constexpr float kXsaFloor = float(double(1e-12f) * double(1e-12f));
-constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
 constexpr int kRing = 2 * kWindowRows;  // tokens kept in LDS
 constexpr size_t kWindowLds = 160 * 1024;  // a CU's
 
-// The ELU: z, or e^z - 1 where z is not positive, NaN included.  A select on z,
-// which does not wait for the exponential, keeps the dependent chain one step
-// shorter than a maximum.
-__device__ __forceinline__ float elu(float z) {
-    const float e = __builtin_amdgcn_exp2f(z * kLog2e) - 1.0f;
-    return z > 0.0f ? z : e;
+// What a value is multiplied by on its way into the meshes and out of them:
+// SCALED ones are carried times log2(e), which the ELU's exponential would
+// otherwise multiply in (Shape::wide: their own units).
+template <bool SCALED>
+struct Units {
+    static constexpr float in = SCALED ? kLog2e : 1.0f, out = SCALED ? kLn2 : 1.0f;
+};
+
+// The ELU in these units, of t = z or z log2(e): z, or e^z - 1 where z is not
+// positive, NaN included.  A select on t, which does not wait for the
+// exponential, keeps the dependent chain one step shorter than a maximum.
+template <bool SCALED>
+__device__ __forceinline__ float elu_units(float t) {
+    const float p = __builtin_amdgcn_exp2f(SCALED ? t : t * kLog2e);
+    return t > 0.0f ? t : SCALED ? __builtin_fmaf(p, kLog2e, -kLog2e) : p - 1.0f;
 }
 
 // v of the lane 16 (32) away combined with the lane's own: register swaps
@@ -96,11 +105,11 @@ __device__ __forceinline__ void partner(const float (&x)[CPL], float (&p)[CPL]) 
     }
 }
 
-// N mesh stacks of one depth (reference.rs:422-453) on x, in place; stack i's
-// weights at w[i].  Strides are 1, or
+// N mesh stacks of one depth (reference.rs:422-453) on x, in place, in the
+// meshes' units; stack i's weights at w[i].  Strides are 1, or
 // 2^(layer mod log2 W) (W = 16 CPL).  Two layers' weights are in registers or
 // on their way while a third is computed.
-template <bool BF, int N, int CPL>
+template <bool BF, bool SCALED, int N, int CPL>
 struct Stacks {
     static constexpr int W = 16 * CPL, LEVELS = CPL == 2 ? 5 : (CPL == 4 ? 6 : 7);
     float2 buf[2][N][CPL];
@@ -142,7 +151,7 @@ struct Stacks {
 #pragma unroll
             for (int j = 0; j < CPL; ++j) {
                 const float z = x[i][j] * buf[B][i][j].x + p[i][j] * buf[B][i][j].y;
-                x[i][j] = last ? z : elu(z);
+                x[i][j] = last ? z : elu_units<SCALED>(z);
             }
         if (!last) load(l + 2, B);
         return last;
@@ -161,19 +170,19 @@ struct Stacks {
     }
 };
 
-template <bool BF, int N, int CPL>
+template <bool BF, bool SCALED, int N, int CPL>
 __device__ __forceinline__ void stacks(float (&x)[N][CPL], const float *const (&w)[N], int depth, int l16) {
-    Stacks<BF, N, CPL> s{{}, w, depth, l16};
+    Stacks<BF, SCALED, N, CPL> s{{}, w, depth, l16};
     s.all(x);
 }
 
-// n = RMSNorm(x) (reference.rs:392-409).
+// n = RMSNorm(x) times `unit` (reference.rs:392-409).
 template <int CPL>
-__device__ __forceinline__ void norm(const float (&x)[CPL], float (&n)[CPL]) {
+__device__ __forceinline__ void norm(const float (&x)[CPL], float (&n)[CPL], float unit) {
     float sq = 0.0f;
 #pragma unroll
     for (int j = 0; j < CPL; ++j) sq = fmaf(x[j], x[j], sq);
-    const float inv = rsqrtf(group_sum<16>(sq) * (1.0f / float(16 * CPL)) + kRmsEps);
+    const float inv = rsqrtf(group_sum<16>(sq) * (1.0f / float(16 * CPL)) + kRmsEps) * unit;
 #pragma unroll
     for (int j = 0; j < CPL; ++j) n[j] = x[j] * inv;
 }
@@ -282,9 +291,10 @@ __device__ __forceinline__ void attend(float *Q, const float *K, const float *V,
 
 // A workgroup of NW waves per sequence: windows of up to 4 NW rows.  STAGED: the
 // blocks' weights and the token vectors are copied to LDS first.
-template <int CPL, int HD, int NW, bool STAGED, bool BF>
+template <int CPL, int HD, int NW, bool STAGED, bool BF, bool SCALED>
 __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
     constexpr int W = 16 * CPL, H = W / HD, LPH = 16 / H, ROWS = 4 * NW, KB = ROWS / 16, STRIDE = W + 4;
+    using U = Units<SCALED>;
     constexpr int GROUP = CPL * NW <= 32 ? 3 : 1;  // stacks side by side, as registers allow
     static_assert(H == 2 || H == 4 || H == 8, "a head is two, four or eight whole lanes");
     extern __shared__ __align__(16) float lds[];
@@ -333,32 +343,33 @@ __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
             const bool tail = l + 1 == a.L;  // only the last row goes on, past its keys and values
             const bool goes_on = !tail || wave == last_wave;
             float qkv[3][CPL];
-            norm(x, qkv[0]);
+            norm(x, qkv[0], U::in);
 #pragma unroll
             for (int j = 0; j < CPL; ++j) qkv[1][j] = qkv[2][j] = qkv[0][j];
             if constexpr (GROUP == 3) {
                 const float *const ws[3] = {w, w + gA, w + 2 * gA};
-                stacks<BF>(qkv, ws, a.A, l16);
+                stacks<BF, SCALED>(qkv, ws, a.A, l16);
             } else {
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
                     if (i == 0 && !goes_on) continue;
                     float (&one)[1][CPL] = reinterpret_cast<float(&)[1][CPL]>(qkv[i]);
                     const float *const ws[1] = {w + i * gA};
-                    stacks<BF>(one, ws, a.A, l16);
+                    stacks<BF, SCALED>(one, ws, a.A, l16);
                 }
             }
             // QK-Norm, then slice RoPE (reference.rs:174-193), each when on.
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
+                float inv = U::out;
                 if (a.qk_norm) {
                     float sq = 0.0f;
 #pragma unroll
                     for (int j = 0; j < CPL; ++j) sq = fmaf(qkv[i][j], qkv[i][j], sq);
-                    const float inv = rsqrtf(group_sum<LPH>(sq) * (1.0f / float(HD)) + kRmsEps);
-#pragma unroll
-                    for (int j = 0; j < CPL; ++j) qkv[i][j] *= inv;
+                    inv = rsqrtf(group_sum<LPH>(sq) * (1.0f / float(HD)) + kRmsEps * U::in * U::in);
                 }
+#pragma unroll
+                for (int j = 0; j < CPL; ++j) qkv[i][j] *= inv;
                 if (a.rotate) {
                     float o[CPL];
 #pragma unroll
@@ -368,6 +379,8 @@ __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
                 }
             }
             float *at = Q + row * STRIDE + CPL * l16;
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) qkv[2][j] *= U::out;
             put_row(at, qkv[0]);
             put_row(at + ROWS * STRIDE, qkv[1]);
             put_row(at + 2 * ROWS * STRIDE, qkv[2]);
@@ -393,19 +406,21 @@ __global__ void __launch_bounds__(64 * NW) window_kernel(WindowArgs a) {
             if (goes_on) {
                 float z[1][CPL];
                 take(Q + row * STRIDE + CPL * l16, z[0]);
+#pragma unroll
+                for (int j = 0; j < CPL; ++j) z[0][j] *= U::in;
                 const float *const wp[1] = {w + 3 * gA}, *const wf[1] = {w + 4 * gA};
-                stacks<BF>(z, wp, a.A, l16);
+                stacks<BF, SCALED>(z, wp, a.A, l16);
 #pragma unroll
-                for (int j = 0; j < CPL; ++j) x[j] += z[0][j];
-                norm(x, z[0]);
-                stacks<BF>(z, wf, a.F, l16);
+                for (int j = 0; j < CPL; ++j) x[j] = fmaf(z[0][j], U::out, x[j]);
+                norm(x, z[0], U::in);
+                stacks<BF, SCALED>(z, wf, a.F, l16);
 #pragma unroll
-                for (int j = 0; j < CPL; ++j) x[j] += z[0][j];
+                for (int j = 0; j < CPL; ++j) x[j] = fmaf(z[0][j], U::out, x[j]);
             }
         }
         if (row == last) {
             float n[CPL];
-            norm(x, n);
+            norm(x, n, 1.0f);
             put_row(xn + CPL * l16, n);
         }
         __syncthreads();
@@ -464,15 +479,20 @@ void launch_window(const Shape &s, const WindowArgs &a, int batch, hipStream_t s
             return;
         hipLaunchKernelGGL(kernel, dim3(batch), dim3(64 * NW), bytes, stream, a);
     };
+    if (s.wide) {
+        a.butterfly ? launch(window_kernel<CPL, HD, NW, false, true, false>, lds)
+                    : launch(window_kernel<CPL, HD, NW, false, false, false>, lds);
+        return;
+    }
     if constexpr (NW == 8) {
         if (lds + staged <= kWindowLds) {
-            a.butterfly ? launch(window_kernel<CPL, HD, NW, true, true>, lds + staged)
-                        : launch(window_kernel<CPL, HD, NW, true, false>, lds + staged);
+            a.butterfly ? launch(window_kernel<CPL, HD, NW, true, true, true>, lds + staged)
+                        : launch(window_kernel<CPL, HD, NW, true, false, true>, lds + staged);
             return;
         }
     }
-    a.butterfly ? launch(window_kernel<CPL, HD, NW, false, true>, lds)
-                : launch(window_kernel<CPL, HD, NW, false, false>, lds);
+    a.butterfly ? launch(window_kernel<CPL, HD, NW, false, true, true>, lds)
+                : launch(window_kernel<CPL, HD, NW, false, false, true>, lds);
 }
 
 // f(CPL, HD) for the widths and head widths that have a kernel (2 to 8 heads);

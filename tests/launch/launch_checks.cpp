@@ -1,6 +1,8 @@
 // What the host launches, checked on a machine without a GPU: the library's
 // objects against fake_hip.cpp.  `launch_checks NAME` runs one check.
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -400,7 +402,51 @@ void batch_without_memory() {
     }
 }
 
+// Kernels that carry mesh values times log2(e) run models whose weights keep
+// these below 1e38: a row of at most sqrt(128) through the V mesh's four layers,
+// seven times that at most into the projection's.  Small weights settle it on
+// the host; large or trained ones by the gain of each layer.
+void wide_routes() {
+    for (float gain : {0.0f, 1.0f, 3.0e4f, 4.0e4f, 1.0e30f})
+        for (float largest : {1.0f, 1.0e6f, 0.0f}) {  // 0: after a training step
+            MeshGpt m(0, shape(128, 4, 64), 7, 2);
+            std::vector<float> weights = m.parameters();
+            weights[10 * 128] = largest;
+            size_t asked = 0;
+            std::set<std::string> kernels;
+            fake::on_launch = [&](const fake::Launch &l) {
+                kernels.insert(l.kernel);
+                if (l.kernel.find("layer_gains_kernel") == std::string::npos) return;
+                expect(l.grid.x == 2 * (4 * 4 + 6), "a gain for each layer of the blocks");
+                std::fill_n(*static_cast<float **>(l.args[2]), l.grid.x, gain);
+                ++asked;
+            };
+            m.set_parameters(weights.data(), weights.size());
+            if (largest == 0.0f) {
+                const std::vector<uint32_t> tokens(64, 1);
+                m.train_batch(tokens.data(), tokens.data(), 64, 32, {});
+            }
+            generate(m, 2, 70, 3);
+            fake::on_launch = nullptr;
+            expect(asked == (largest == 1.0f ? 0u : 1u), "the layers' gains are asked for once where they are needed");
+            const char *form = asked && gain > 3.5e4f ? "ELb0EEEv" : "ELb1EEEv";
+            for (const std::string &k : kernels)
+                if (k.find("rows_block_kernel") != std::string::npos || k.find("window_kernel") != std::string::npos)
+                    expect(k.find(form) != std::string::npos, "gain " + std::to_string(gain) + ": " + k);
+        }
+    // The largest weight may be any; one that is not finite is refused as ever.
+    MeshGpt m(0, shape(128, 4, 64), 7, 2);
+    std::vector<float> weights = m.parameters();
+    for (float bad : {INFINITY, -INFINITY, NAN}) {
+        weights[5] = bad;
+        expect(status_of([&] { m.set_parameters(weights.data(), weights.size()); }) == kNonfinite, "a weight refused");
+    }
+    weights[5] = -3.0e38f;
+    expect(status_of([&] { m.set_parameters(weights.data(), weights.size()); }) == 0, "a large weight taken");
+}
+
 const std::map<std::string, void (*)()> kChecks = {
+    {"wide_routes", wide_routes},
     {"batch_without_memory", batch_without_memory},
     {"threads_reading", threads_reading},
     {"no_batch", no_batch},

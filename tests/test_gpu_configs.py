@@ -734,12 +734,14 @@ def _check_last_rows(W, H, n, batch, **switch):
 # The row-tile blocks at each register-tile width: tiles of 4096 / W rows with
 # one row more and one less, both connectivities, stacks of one layer (no ELU),
 # and QK-Norm off (the only factor that takes log2(e) from q and k) or on.
+@pytest.mark.parametrize("wide", ["0", "1"])  # mesh values times log2(e), in their own units
 @pytest.mark.parametrize("switch", [dict(), dict(qk_norm=0), dict(rope=0), dict(qk_norm=0, rope=0, xsa=0)],
                          ids=["all", "no-qk", "no-rope", "none"])
 @pytest.mark.parametrize("W,H,n,A,F,butterfly", [(128, 4, 31, 7, 1, 1), (128, 8, 33, 1, 5, 0), (256, 4, 17, 8, 8, 1),
                                                  (512, 8, 17, 9, 1, 1), (512, 16, 24, 1, 10, 0),
                                                  (1024, 16, 19, 11, 1, 1), (1024, 32, 17, 3, 10, 1)])
-def test_row_tiles_match_the_oracle(W, H, n, A, F, butterfly, switch):
+def test_row_tiles_match_the_oracle(W, H, n, A, F, butterfly, switch, wide, monkeypatch):
+    monkeypatch.setenv("MG_FORCE_WIDE", wide)
     kw = dict(vocab_size=40, context=n, width=W, heads=H, layers=2, attention_mesh_depth=A, ffn_mesh_depth=F,
               connectivity=butterfly, **switch)
     o = O.config(**kw)

@@ -37,9 +37,11 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("wide", ["0", "1"])  # mesh values times log2(e), in their own units
 @pytest.mark.parametrize("temperature", [0.0, 0.7])
 @pytest.mark.parametrize("cfg", CASES, ids=["-".join(f"{k[:3]}{v}" for k, v in c.items()) for c in CASES])
-def test_window_generation_matches_the_oracle(cfg, temperature):
+def test_window_generation_matches_the_oracle(cfg, temperature, wide, monkeypatch):
+    monkeypatch.setenv("MG_FORCE_WIDE", wide)
     kw = dict(dict(vocab_size=40, layers=2), **cfg)
     g, o = G.GptConfig(**kw), O.config(**kw)
     params = O.initialize(o, 7)

@@ -36,7 +36,8 @@ def checks(tmp_path_factory):
 
 @pytest.mark.parametrize("name", ["refused_launches", "foreign_errors", "window_launches", "window_routes", "chain_shapes",
                                   "scratch_limits", "chain_routes", "split_routes", "finite_checks",
-                                  "no_batch", "threads_reading", "batch_without_memory"])
+                                  "no_batch", "threads_reading", "batch_without_memory",
+                                  "wide_routes"])
 def test_launches(checks, name):
     run = subprocess.run([checks, name], capture_output=True, text=True, timeout=300)
     assert run.returncode == 0 and run.stdout == "ok\n", run.stdout + run.stderr
